@@ -23,6 +23,7 @@
 #include "pf_grid.hip"
 #include "pf_p2g.hip"
 #include "pf_project.hip"
+#include "pf_cg.hip"
 #include "pf_g2p.hip"
 #include "pf_lpc.hip"
 #include "pf_mr.hip"
@@ -161,12 +162,13 @@ int pf_create(pf_ctx** out, const pf_grid_desc* d) {
   for (float** p : f32) HIP_TRY(c, dalloc(p, ncell));
   double** f64[] = {&c->b64, &c->x64, &c->r64, &c->cd64, &c->cx64, &c->cy64, &c->cz64};
   for (double** p : f64) HIP_TRY(c, dalloc(p, ncell));
-  HIP_TRY(c, dalloc(&c->sc, 1));
-  HIP_TRY(c, dalloc(&c->partial, (long long)kMaxPartials * 4));
+  HIP_TRY(c, dalloc(&c->sc, 2));
+  HIP_TRY(c, dalloc(&c->partial, (long long)kMaxPartials * kPartialSlots));
   HIP_TRY(c, dalloc(&c->red, 16));
   HIP_TRY(c, hipHostMalloc((void**)&c->red_host, sizeof(double) * 16));
   HIP_TRY(c, hipHostMalloc((void**)&c->done_host, sizeof(int) * 16));
   HIP_TRY(c, hipHostMalloc((void**)&c->sc_host, sizeof(SolveScalars)));
+  HIP_TRY(c, hipHostMalloc((void**)&c->cg_word, sizeof(unsigned long long)));
   HIP_TRY(c, dalloc(&c->u32_dev, 64));
   HIP_TRY(c, hipHostMalloc((void**)&c->u32_host, sizeof(uint32_t) * 64));
   HIP_TRY(c, dalloc(&c->esc_dev, 8));
@@ -222,6 +224,8 @@ int pf_destroy(pf_ctx* c) {
   dfree(c->fbeta); dfree(c->fphi); dfree(c->tiles); dfree(c->tile_flags); dfree(c->snaps);
   hipFree(c->sc); hipFree(c->partial); hipFree(c->red);
   hipHostFree(c->red_host); hipHostFree(c->done_host); hipHostFree(c->sc_host); hipHostFree(c->u32_host);
+  hipHostFree(c->cg_word);
+  dfree(c->cgq);
   hipFree(c->u32_dev); hipFree(c->esc_dev); hipFree(c->vmax_dev);
   for (auto* q : c->g2p_quad) hipFree(q);
   hipFree(c->scan_tiles); hipFree(c->stage_f);

@@ -509,6 +509,122 @@ int mr_mg_apply(pf_ctx* c, const MrOp& op, const VecArgs& va, const float* r, fl
   return PF_OK;
 }
 
+// ---- the Jacobi PCG in one kernel per iteration (pf_cg.hip)
+
+// what the next launch reads: which scalars, sums (nsums partials of each) and vectors
+struct CgState {
+  int cur = 0, sums = 0, nsums = 0, par = 0;
+  unsigned long long seq = 0;  // launches so far
+};
+
+float* cg_r(const pf_ctx* c, int par) { return par ? c->z32 : c->r32; }
+float* cg_q(const pf_ctx* c, int par) { return par ? c->cgq : c->Ap; }
+float* cg_p(const pf_ctx* c, int par) { return par ? c->pB : c->pA; }
+double* cg_sums(const pf_ctx* c, int sums) { return c->partial + sums * CG_SUMS * kMaxPartials; }
+
+CgArgs cg_args(const pf_ctx* c, const CgState& g, const VecArgs& va) {
+  CgArgs a{};
+  a.dc = c->dc; a.list = va.list; a.nlist = va.nlist;
+  a.x = c->x32;
+  a.r = cg_r(c, g.par); a.q = cg_q(c, g.par); a.p = cg_p(c, g.par);
+  a.rn = cg_r(c, g.par ^ 1); a.qn = cg_q(c, g.par ^ 1); a.pn = cg_p(c, g.par ^ 1);
+  a.inv = c->invd32; a.cd = c->cd32; a.cx = c->cx32; a.cy = c->cy32; a.cz = c->cz32;
+  a.sums = cg_sums(c, g.sums);
+  a.sums_out = cg_sums(c, g.sums ^ 1);
+  a.nsums = g.nsums;
+  a.in = c->sc + g.cur;
+  a.out = c->sc + (g.cur ^ 1);
+  a.word = c->cg_word;
+  a.seq = g.seq;
+  return a;
+}
+
+// workgroups: four list blocks to a wave, at most 1024 (every workgroup sums that many
+// partials of five quantities), a multiple of 8 (one share per XCD)
+unsigned cg_grid(long long nlist) {
+  return (unsigned)std::clamp<long long>((((nlist + 15) / 16 + 7) / 8) * 8, 8, 1024);
+}
+
+// the FP64 residual into the buffers that the next launch reads, the direction zero
+// before the first iteration
+int cg_load(pf_ctx* c, CgState& g, VecArgs va, unsigned G, const double* r_src, bool first) {
+  va.part = cg_sums(c, g.sums);
+  g.nsums = (int)std::min(G, 1024u);
+  hipLaunchKernelGGL(k_cg_load, dim3((unsigned)g.nsums), dim3(256), 0, c->stream, va, r_src, c->x32, cg_r(c, g.par),
+                     first ? cg_p(c, g.par) : nullptr, first ? cg_q(c, g.par) : nullptr, c->invd32);
+  LAUNCH_CHECK(c);
+  return PF_OK;
+}
+
+int cg_start(pf_ctx* c, CgState& g, const VecArgs& va, unsigned G, const double* r_src, double delta2,
+             double tol2_abs, int budget, int between) {
+  if (!c->cgq) HIP_TRY(c, dalloc(&c->cgq, c->dc.nblocks * kBlockVol));
+  g.cur = g.par = 0;
+  hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(1), 0, c->stream, c->sc, 1, delta2, tol2_abs, budget, between);
+  return cg_load(c, g, va, G, r_src, true);
+}
+
+// after a residual replacement (g and sc_host hold the paused state)
+int cg_resume(pf_ctx* c, CgState& g, const VecArgs& va, unsigned G) {
+  hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(1), 0, c->stream, c->sc + g.cur, 2, 0.0, 0.0, 0, 0);
+  g.par ^= 1;
+  return cg_load(c, g, va, G, c->r64, false);
+}
+
+// Iterations until the recursion pauses; the state is then in sc_host.  The host follows
+// through one word that each launch stores in pinned memory and stays at most `ahead`
+// launches in front of it, so no iteration waits for the host and a pause costs at most
+// that many launches that return at once.  While residuals are recorded, the stream is
+// drained every `ahead` iterations instead and `look` sees the residual.
+template <typename Look>
+int cg_run(pf_ctx* c, CgState& g, const VecArgs& va, int check, const Look& look) {
+  const int ahead = std::clamp(check, 1, 16);
+  const unsigned grid = cg_grid(va.nlist);
+  volatile unsigned long long* word = c->cg_word;
+  *word = 2 * g.seq;  // (the stream is idle: no launch of an earlier segment is left)
+  auto fetch = [&]() -> int {
+    HIP_TRY(c, hipMemcpyAsync(c->sc_host, c->sc + g.cur, sizeof(SolveScalars), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    // (launches after the pause moved nothing)
+    if (c->sc_host->done) g.par = c->sc_host->par;
+    return PF_OK;
+  };
+  for (int launched = 1;; ++launched) {
+    ++g.seq;
+    const CgArgs a = cg_args(c, g, va);
+    const long long ki = kbegin(c, PF_K_PCG_SPMV);
+    if (grid <= 512)
+      hipLaunchKernelGGL(k_cg_iter<true>, dim3(grid), dim3(256), 0, c->stream, a);
+    else
+      hipLaunchKernelGGL(k_cg_iter<false>, dim3(grid), dim3(256), 0, c->stream, a);
+    kend(c, ki);
+    LAUNCH_CHECK(c);
+    g.cur ^= 1;
+    g.sums ^= 1;
+    g.par ^= 1;
+    g.nsums = (int)grid;
+    if (c->snap_cap > 0) {
+      if (launched % ahead) continue;
+      int st = fetch();
+      if (st) return st;
+      const SolveScalars& S = *c->sc_host;
+      st = look(S.iter, cg_r(c, S.par));
+      if (st || S.done) return st;
+      continue;
+    }
+    unsigned long long w = *word;
+    for (unsigned spin = 0; !(w & 1) && (w >> 1) + ahead < g.seq; w = *word) {
+      // (a launch that failed would never store its word: the stream says so)
+      if ((++spin & 0xffff) == 0) {
+        const hipError_t e = hipStreamQuery(c->stream);
+        if (e != hipSuccess && e != hipErrorNotReady) HIP_TRY(c, e);
+        if (e == hipSuccess && (*word >> 1) < g.seq) return fail(c, PF_ERR_HIP, "solver launches left no state");
+      }
+    }
+    if (w & 1) return fetch();
+  }
+}
+
 // single: the single-phase unit-density projection (ph unused, cdiv ignored);
 // c->mr: the multires finite-volume projection, stopping when
 // |rhs - A x|_inf < max(cfg->tol, mr_rel_tol * |rhs|_inf)
@@ -546,7 +662,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     // assembly's outputs, which k_assemble writes on all 64 cells of every listed
     // block, x64 (k_ir_start writes it there) and r64 (written before it is read).
     int nf = 0;
-    for (float* p : {c->f[F_P], c->x32, c->r32, c->z32, c->pA, c->pB, c->Ap, c->mg_t0})
+    for (float* p : {c->f[F_P], c->x32, c->r32, c->z32, c->pA, c->pB, c->Ap, c->mg_t0, c->cgq})
       if (p) z.f32[nf++] = p;
     z.nf32_all = nf;
     for (float* p : {c->cd32, c->cx32, c->cy32, c->cz32, c->invd32}) z.f32[nf++] = p;
@@ -744,10 +860,10 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   if (lpc_system) c->tiles_valid = true;
   const long long ncell = c->dc.nblocks * kBlockVol;
   // residual snapshot (training data), at most one per `snap_every` iterations
-  auto snapshot = [&](int iter) -> int {
+  auto snapshot = [&](int iter, const float* r32) -> int {
     if (c->snap_cap <= 0 || c->nsnap >= c->snap_cap) return PF_OK;
     if (c->snap_last_iter >= 0 && iter - c->snap_last_iter < c->snap_every) return PF_OK;
-    HIP_TRY(c, hipMemcpyAsync(c->snaps + (long long)c->nsnap * ncell, c->r32, sizeof(float) * (size_t)ncell,
+    HIP_TRY(c, hipMemcpyAsync(c->snaps + (long long)c->nsnap * ncell, r32, sizeof(float) * (size_t)ncell,
                               hipMemcpyDeviceToDevice, c->stream));
     c->nsnap++;
     c->snap_last_iter = iter;
@@ -800,8 +916,13 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     rmax = c->red_host[1];
   }
   if (!refmode && !converged && max_iters > 0 && std::isfinite(rmax)) {
+    // the buffer-addressed kernels take 32-bit byte offsets: arrays below 2 GiB
+    const bool spmv_buffers = c->dc.nblocks * kBlockVol * 4 < (1LL << 31);
+    CgState cg;
+    const bool one_kernel = !mr && spmv_buffers;   // the Jacobi iteration as k_cg_iter
     // (re)start: r32 from r64, x32 = 0, p = 0, z = M(r)
     auto start = [&](int budget) -> int {
+      if (one_kernel && !learned) return cg_start(c, cg, va, G, r_src, delta * delta, tol2_abs, budget, between);
       hipLaunchKernelGGL(k_pcg_load, dim3(G), dim3(256), 0, c->stream, va, r_src, c->x32, c->r32, c->z32, c->pA,
                          c->invd32, learned ? 1 : 0);
       LAUNCH_CHECK(c);
@@ -819,14 +940,12 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     };
     st = start(max_iters);
     if (st) return st;
-    st = snapshot(0);
+    st = snapshot(0, c->r32);
     if (st) return st;
     // the two iteration kernels use at most 1024 workgroups, so the per-iteration
     // scalar kernels sum few partials
     // (the multires SpMV waits on dependent loads per block: it takes more workgroups)
     const unsigned GS = std::min(G, mr ? 4096u : 1024u);
-    // the buffer-addressed SpMV takes 32-bit byte offsets: arrays below 2 GiB
-    const bool spmv_buffers = c->dc.nblocks * kBlockVol * 4 < (1LL << 31);
     VecArgs vs = va;
     // the multires SpMV: blocks of level 0-1 here, level-2 blocks in a second launch
     VecArgs vs01 = va;
@@ -845,7 +964,12 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     int iter_last = 0;
     for (;;) {
       const size_t rec0 = c->krec.size();
-      for (int q = 0; q < q_next; ++q) {
+      const bool fused = one_kernel && !learned;
+      if (fused) {
+        st = cg_run(c, cg, va, check, [&](int iter, const float* r) { return snapshot(iter_base + iter, r); });
+        if (st) return st;
+      }
+      for (int q = 0; q < (fused ? 0 : q_next); ++q) {
         if (mr)
           TIMED(c, PF_K_PCG_SPMV,
                 hipLaunchKernelGGL(k_mr_spmv, dim3(GS), dim3(256), 0, c->stream, vs01, mop, c->z32, c->pA, c->pB,
@@ -880,8 +1004,10 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         }
       }
       LAUNCH_CHECK(c);
-      HIP_TRY(c, hipMemcpyAsync(c->sc_host, c->sc, sizeof(SolveScalars), hipMemcpyDeviceToHost, c->stream));
-      HIP_TRY(c, hipStreamSynchronize(c->stream));
+      if (!fused) {
+        HIP_TRY(c, hipMemcpyAsync(c->sc_host, c->sc, sizeof(SolveScalars), hipMemcpyDeviceToHost, c->stream));
+        HIP_TRY(c, hipStreamSynchronize(c->stream));
+      }
       std::memcpy(c->done_host, &c->sc_host->iter, sizeof(int) * 8);
       // {iter, done, breakdown, stalled, iter_best, max_iter, stall_window, upd}
       // launches after a pause return at once: keep the timings of those that ran
@@ -894,8 +1020,8 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         if (k == PF_K_PCG_UPDATE && kept_u++ >= ran) k = -1;
         if ((k == PF_K_LPC_APPLY || k == PF_K_MG_APPLY) && kept_l++ >= ran) k = -1;
       }
-      if (ran > 0) {
-        st = snapshot(iter_base + c->done_host[0]);
+      if (ran > 0 && !fused) {
+        st = snapshot(iter_base + c->done_host[0], c->r32);
         if (st) return st;
       }
       if (!c->done_host[1]) {
@@ -932,7 +1058,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       converged = met();
       if (trace) {
         double s_rr32 = 0.0;
-        HIP_TRY(c, hipMemcpy(&s_rr32, &c->sc->rr, sizeof(double), hipMemcpyDeviceToHost));
+        s_rr32 = c->sc_host->rr;
         std::fprintf(stderr, "[pf solve] update %d iter %d fp32 rel %.3e true rel %.3e max %.3e%s%s\n", outer, total,
                      std::sqrt(s_rr32 / std::max(bnorm2, 1e-300)), std::sqrt(rr / std::max(bnorm2, 1e-300)), rmax,
                      breakdown ? " breakdown" : "", learned ? " (learned)" : "");
@@ -960,6 +1086,15 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       }
       prev_rr = rr;
       // resume from the true residual; after a breakdown restart the direction too
+      if (fused) {
+        st = breakdown ? start(max_iters - total) : cg_resume(c, cg, va, G);
+        if (st) return st;
+        if (breakdown) {
+          iter_base = total;
+          iter_before = 0;
+        }
+        continue;
+      }
       hipLaunchKernelGGL(k_pcg_load, dim3(G), dim3(256), 0, c->stream, va, c->r64, c->x32, c->r32, c->z32,
                          breakdown ? c->pA : nullptr, c->invd32, learned ? 1 : 0);
       LAUNCH_CHECK(c);

@@ -117,6 +117,7 @@ struct SolveScalars {
   double rr_ref, tol2_abs, rz_pending, rz_cross;  // rz_cross: r_new . z_old at a pause (flexible beta)
   int iter, done, breakdown, stalled;
   int iter_best, max_iter, stall_window, upd;
+  int fresh, par;   // one-kernel iteration: 1 fresh start, 2 resumed; buffers the next launch reads
 };
 
 struct Ctx {
@@ -161,11 +162,13 @@ struct Ctx {
   float *cd32 = nullptr, *cx32 = nullptr, *cy32 = nullptr, *cz32 = nullptr, *invd32 = nullptr;
   double *b64 = nullptr, *x64 = nullptr, *r64 = nullptr;
   double *cd64 = nullptr, *cx64 = nullptr, *cy64 = nullptr, *cz64 = nullptr;
-  SolveScalars* sc = nullptr;       // device
-  double* partial = nullptr;        // per-workgroup partial sums (kMaxPartials * 4)
+  float* cgq = nullptr;             // the one-kernel iteration's second A p (allocated on first use)
+  SolveScalars* sc = nullptr;       // device, two: the one-kernel iteration reads one and writes the other
+  double* partial = nullptr;        // per-workgroup partial sums (kMaxPartials * kPartialSlots)
   double* red = nullptr;            // reduced values (device, 16 doubles)
   double* red_host = nullptr;       // pinned host mirror
   int* done_host = nullptr;         // pinned host mirror of sc->done
+  unsigned long long* cg_word = nullptr;  // pinned: 2 * launch number + done of the last one-kernel iteration
   SolveScalars* sc_host = nullptr;  // pinned host mirror of the whole struct
   uint32_t* u32_dev = nullptr;      // small device scratch (pin detection, counters), 64 words
   uint32_t* u32_host = nullptr;     // pinned mirror, 64 words
@@ -280,6 +283,7 @@ struct Ctx {
 };
 
 constexpr int kMaxPartials = 4096;
+constexpr int kPartialSlots = 12;
 
 // ---- launch helpers shared by the kernel files (implemented in pf_util.hip etc.)
 hipError_t fill_u8(hipStream_t s, uint8_t* p, uint8_t v, long long n);

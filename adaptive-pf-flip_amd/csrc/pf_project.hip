@@ -392,7 +392,7 @@ __global__ void __launch_bounds__(256) k_assemble(ProjArgs a, AsmOut o) {
 struct ZeroArgs {
   const uint32_t* list;
   long long nlist;
-  float* f32[13];
+  float* f32[14];
   int nf32, nf32_all;
   double* f64[7];
   int nf64;

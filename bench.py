@@ -45,6 +45,8 @@ sys.path.insert(0, os.path.join(ROOT, "adaptive-pf-flip_amd"))
 
 HBM_PEAK_GBS = 8000.0
 SPMV_BYTES_PER_CELL = 32  # z, p_old, diag, 3 couplings read; p_new, Ap written (FP32)
+# the Jacobi iteration is one kernel: x, r, p, Ap, 1/diag and the operator read; x, r, p, Ap written
+CG_BYTES_PER_CELL = 52
 # algorithmic bytes per stage (FP32 = 4 B): per particle and per FLUID cell
 P2G_BYTES = (25, 24)        # particle x, y, z, u, v, w, type read; u, v, w, mu, mv, mw written
 STAGE_BYTES = {             # (per particle, per fluid cell, per grid cell)
@@ -446,13 +448,15 @@ def main():
                 roofline["waves_per_simd"] = read_table_value(tf, "resident waves per SIMD")
         nl, ms = live["pcg_spmv"]
         if nl:
-            bytes_per_launch = SPMV_BYTES_PER_CELL * fluid
+            one = args.precond == "jacobi"
+            bytes_per_launch = (CG_BYTES_PER_CELL if one else SPMV_BYTES_PER_CELL) * fluid
             avg = ms / nl
             achieved = bytes_per_launch / (avg * 1e-3) / 1e9
             tf = os.path.join(ROOT, "profiles", "pcg_spmv_rt256_traffic.md")
-            roofline_spmv = {"bound": "hbm", "kernel": "k_pcg_spmv", "achieved": round(achieved, 1),
+            roofline_spmv = {"bound": "hbm", "kernel": "k_cg_iter" if one else "k_pcg_spmv",
+                             "achieved": round(achieved, 1),
                              "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                             "traffic": read_traffic(tf) if (os.path.exists(tf) and n == 256) else None,
+                             "traffic": read_traffic(tf) if (os.path.exists(tf) and n == 256 and not one) else None,
                              "bytes_per_launch": bytes_per_launch, "avg_launch_ms": round(avg, 5)}
     # achievable HBM bandwidth of a plain copy kernel on this box (reported beside
     # the 8 TB/s peak; also the known-size kernel for calibrating HBM counters)
