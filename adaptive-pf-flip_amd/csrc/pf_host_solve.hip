@@ -42,7 +42,6 @@ void mg_free_level(Ctx::MgBuf& b) {
   float** arrs[8] = {&b.cd, &b.cx, &b.cy, &b.cz, &b.inv, &b.x, &b.r, &b.t};
   for (float** a : arrs) dfree(*a);
   for (auto& p : b.h) dfree(p);
-  dfree(b.mx);
   dfree(b.unscale);
 }
 
@@ -52,7 +51,7 @@ int mg_alloc(pf_ctx* c) {
   std::vector<Ctx::MgBuf> levels;
   float* t0 = nullptr;
   uint16_t* h[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-  uint32_t* mx = nullptr;
+  float* mx = nullptr;
   float* unscale = nullptr;
   auto release = [&]() {
     for (auto& b : levels) mg_free_level(b);
@@ -74,7 +73,6 @@ int mg_alloc(pf_ctx* c) {
       if (e == hipSuccess) e = dalloc(a, n);
     for (auto& p : b.h)
       if (e == hipSuccess) e = dalloc(&p, n);
-    if (e == hipSuccess) e = dalloc(&b.mx, 2);
     if (e == hipSuccess) e = dalloc(&b.unscale, 2);
     levels.push_back(b);
   }
@@ -82,7 +80,7 @@ int mg_alloc(pf_ctx* c) {
   if (e == hipSuccess) e = dalloc(&t0, n0);
   for (auto& p : h)
     if (e == hipSuccess) e = dalloc(&p, n0);
-  if (e == hipSuccess) e = dalloc(&mx, 2);
+  if (e == hipSuccess) e = dalloc(&mx, 2 * kMaxPartials);
   if (e == hipSuccess) e = dalloc(&unscale, 2);
   if (e != hipSuccess) {
     release();
@@ -98,6 +96,18 @@ int mg_alloc(pf_ctx* c) {
 
 int mg_coarsen_from(pf_ctx* c, MgLevel F, size_t from);
 
+// workgroups of the kernels that build a level: each reader sums one maximum per workgroup
+unsigned mg_build_grid(long long cells) { return std::min<unsigned>(grid_for(cells, 256), 1024u); }
+
+// a level's FP16 copy, scaled by the maxima of nmx workgroups in c->mg_mx
+void mg_tohalf(pf_ctx* c, const MgLevel& L, uint16_t* const* hb, int nmx, float* unscale) {
+  const long long n = L.d.nblocks * kBlockVol;
+  _Float16* h[5];
+  for (int q = 0; q < 5; ++q) h[q] = reinterpret_cast<_Float16*>(hb[q]);
+  hipLaunchKernelGGL(k_mg_tohalf, dim3(mg_build_grid(n)), dim3(256), 0, c->stream, n, L.cd, L.cx, L.cy, L.cz, L.inv,
+                     h[0], h[1], h[2], h[3], h[4], c->mg_mx, nmx, unscale);
+}
+
 int mg_build(pf_ctx* c) {
   if (!c->mg_t0) {
     int st = mg_alloc(c);
@@ -109,36 +119,17 @@ int mg_build(pf_ctx* c) {
   // the FP16 level-0 operator of the row kernels
   {
     const long long n0 = c->dc.nblocks * kBlockVol;
-    if (!c->mg_mx_valid) {
-      HIP_TRY(c, fill_u32(c->stream, c->mg_mx, 0u, 2));
-      hipLaunchKernelGGL(k_mg_absmax, dim3(std::min<unsigned>(grid_for(n0, 256), 2048u)), dim3(256), 0, c->stream,
-                         n0, c->cd32, c->cx32, c->cy32, c->cz32, c->invd32, c->mg_mx);
-      c->mg_mx_valid = true;
+    int nmx = c->mg_mx_n;  // left by the assembly
+    if (!nmx) {
+      nmx = (int)mg_build_grid(n0);
+      hipLaunchKernelGGL(k_mg_absmax, dim3((unsigned)nmx), dim3(256), 0, c->stream, n0, c->cd32, c->cx32, c->cy32,
+                         c->cz32, c->invd32, c->mg_mx);
     }
-    _Float16* h[5];
-    for (int q = 0; q < 5; ++q) h[q] = reinterpret_cast<_Float16*>(c->mg_h[q]);
-    hipLaunchKernelGGL(k_mg_tohalf, dim3(std::min<unsigned>(grid_for(n0, 256), 4096u)), dim3(256), 0, c->stream, n0,
-                       c->cd32, c->cx32, c->cy32, c->cz32, c->invd32, h[0], h[1], h[2], h[3], h[4], c->mg_mx,
-                       c->mg_unscale);
+    c->mg_mx_n = 0;  // (the levels below use the array next)
+    mg_tohalf(c, mg_level0(c), c->mg_h, nmx, c->mg_unscale);
     LAUNCH_CHECK(c);
   }
   return mg_coarsen_from(c, mg_level0(c), 0);
-}
-
-// a level's inverse diagonal and the FP16 copy its row kernels read (as level 0's)
-int mg_level_finish(pf_ctx* c, Ctx::MgBuf& b) {
-  const long long nl = b.d.nblocks * kBlockVol;
-  const unsigned g = std::min<unsigned>(grid_for(nl, 256), 4096u);
-  hipLaunchKernelGGL(k_mg_inverse, dim3(g), dim3(256), 0, c->stream, mg_level(b), b.inv);
-  HIP_TRY(c, fill_u32(c->stream, b.mx, 0u, 2));
-  hipLaunchKernelGGL(k_mg_absmax, dim3(std::min<unsigned>(grid_for(nl, 256), 2048u)), dim3(256), 0, c->stream, nl,
-                     b.cd, b.cx, b.cy, b.cz, b.inv, b.mx);
-  _Float16* h[5];
-  for (int q = 0; q < 5; ++q) h[q] = reinterpret_cast<_Float16*>(b.h[q]);
-  hipLaunchKernelGGL(k_mg_tohalf, dim3(std::min<unsigned>(grid_for(nl, 256), 4096u)), dim3(256), 0, c->stream, nl,
-                     b.cd, b.cx, b.cy, b.cz, b.inv, h[0], h[1], h[2], h[3], h[4], b.mx, b.unscale);
-  LAUNCH_CHECK(c);
-  return PF_OK;
 }
 
 // levels c->mg[from..] by aggregation from F (the level above c->mg[from])
@@ -146,10 +137,11 @@ int mg_coarsen_from(pf_ctx* c, MgLevel F, size_t from) {
   for (size_t l = from; l < c->mg.size(); ++l) {
     Ctx::MgBuf& b = c->mg[l];
     const MgLevel Cl = mg_level(b);
-    const unsigned g = std::min<unsigned>(grid_for(b.d.nblocks * kBlockVol, 256), 4096u);
-    hipLaunchKernelGGL(k_mg_coarsen, dim3(g), dim3(256), 0, c->stream, F, Cl, b.cd, b.cx, b.cy, b.cz);
-    int st = mg_level_finish(c, b);
-    if (st) return st;
+    const unsigned g = mg_build_grid(b.d.nblocks * kBlockVol);
+    hipLaunchKernelGGL(k_mg_coarsen, dim3(g), dim3(256), 0, c->stream, F, Cl, b.cd, b.cx, b.cy, b.cz, b.inv,
+                       c->mg_mx);
+    mg_tohalf(c, Cl, b.h, (int)g, b.unscale);
+    LAUNCH_CHECK(c);
     F = Cl;
   }
   return PF_OK;
@@ -207,8 +199,10 @@ int mr_mg_build(pf_ctx* c, const MrOp& op) {
   // the level-2 kernels write the cell entry of a block only: the other entries of the
   // cycle's work array stay zero
   HIP_TRY(c, fill_f32(c->stream, c->mg_t0, 0.f, c->dc.nblocks * kBlockVol));
-  int st = mg_level_finish(c, b);
-  if (st) return st;
+  const unsigned g = mg_build_grid(nl);
+  hipLaunchKernelGGL(k_mg_inverse, dim3(g), dim3(256), 0, c->stream, mg_level(b), b.inv, c->mg_mx);
+  mg_tohalf(c, mg_level(b), b.h, (int)g, b.unscale);
+  LAUNCH_CHECK(c);
   return mg_coarsen_from(c, mg_level(b), 2);
 }
 
@@ -640,7 +634,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   const Geom& g = c->geom;
   const long long nb = c->dc.nblocks;
   // 1. the blocks holding FLUID cells (flags; sorted list below)
-  c->mg_mx_valid = false;
+  c->mg_mx_n = 0;
   uint8_t* flag8 = reinterpret_cast<uint8_t*>(c->blk_flag32);
   hipLaunchKernelGGL(k_fluid_flags, dim3(grid_for(nb, 4)), dim3(256), 0, c->stream, c->dc, c->marker, flag8);
   LAUNCH_CHECK(c);
@@ -762,7 +756,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble, dim3(G), dim3(256), 0, c->stream, ma));
     LAUNCH_CHECK(c);
   } else {
-  hipLaunchKernelGGL(k_pin_detect, dim3(list_grid(npb)), dim3(256), 0, c->stream, pa);
+  hipLaunchKernelGGL(k_pin_detect, dim3(std::min(list_grid(npb), 512u)), dim3(256), 0, c->stream, pa);
   LAUNCH_CHECK(c);
   AsmOut ao;
   ao.b64 = c->b64; ao.cd64 = c->cd64; ao.cx64 = c->cx64; ao.cy64 = c->cy64; ao.cz64 = c->cz64;
@@ -781,12 +775,11 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       int s2 = mg_alloc(c);
       if (s2) return s2;
     }
-    HIP_TRY(c, fill_u32(c->stream, c->mg_mx, 0u, 2));
     ao.mx = c->mg_mx;
   }
   TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_assemble, dim3(G), dim3(256), 0, c->stream, pa, ao));
   LAUNCH_CHECK(c);
-  c->mg_mx_valid = want_mx;
+  if (want_mx) c->mg_mx_n = (int)G;
   }
   // red[2] = sum b^2; red[3] = max |b| (sparse assembly only)
   hipLaunchKernelGGL(k_reduce_slots, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, mr ? 1 : 2, 2u,

@@ -253,18 +253,17 @@ struct Ctx {
     float *cd = nullptr, *cx = nullptr, *cy = nullptr, *cz = nullptr, *inv = nullptr;
     float *x = nullptr, *r = nullptr, *t = nullptr;
     // the level's operator as scaled FP16 for the row kernels (cd, cx, cy, cz, inv),
-    // its maxima (float bits) and scales
+    // its scales
     uint16_t* h[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-    uint32_t* mx = nullptr;
     float* unscale = nullptr;
   };
   std::vector<MgBuf> mg;
   float* mg_t0 = nullptr;
-  // FP16 copies of the level-0 cd, cx, cy, cz and diagonal inverse (scaled), their
-  // maxima (float bits) and scales
+  // FP16 copies of the level-0 cd, cx, cy, cz and diagonal inverse (scaled), the maxima of
+  // the level last built (per workgroup, 2 * kMaxPartials) and the scales
   uint16_t *mg_h[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
-  uint32_t* mg_mx = nullptr;
-  bool mg_mx_valid = false;   // mg_mx holds the maxima of the current system (set by the assembly)
+  float* mg_mx = nullptr;
+  int mg_mx_n = 0;            // workgroups of the assembly whose maxima mg_mx holds (0: none)
   float* mg_unscale = nullptr;
   // per-aggregate scaling s = sqrt(w) of level 1's restricted residual and correction
   // (P S B_1 S P^T in place of P B_1 P^T), or null: w = 1.  mg_cs holds the caller's

@@ -184,37 +184,83 @@ __global__ void __launch_bounds__(256) k_mg_prolong(MgWalk w, MgLevel F, MgLevel
 #undef MG_BODY
 }
 
-// the Galerkin coarse operator of level F: sums of the children's cd and of the fine
-// couplings that cross each coarse face
-__global__ void __launch_bounds__(256) k_mg_coarsen(MgLevel F, MgLevel Cl, float* __restrict__ cd,
-                                                    float* __restrict__ cx, float* __restrict__ cy,
-                                                    float* __restrict__ cz) {
-  for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < Cl.d.nblocks * kBlockVol;
-       q += (long long)gridDim.x * 256) {
-    int I, J, K;
-    mg_coords(Cl.d, q, I, J, K);
-    float d = 0.0f, wx = 0.0f, wy = 0.0f, wz = 0.0f;
-    if (I < Cl.nx && J < Cl.ny && K < Cl.nz)
-      for (int e = 0; e < 8; ++e) {
-        const int a = e & 1, b = (e >> 1) & 1, g = e >> 2;
-        const int i = 2 * I + a, j = 2 * J + b, k = 2 * K + g;
-        if (i >= F.nx || j >= F.ny || k >= F.nz) continue;
-        const long long c = bm_index(F.d, i, j, k);
-        d += F.cd[c];
-        // the high-side children's +faces lead into the next aggregate
-        if (a == 1 && i + 1 < F.nx) wx += F.cx[c];
-        if (b == 1 && j + 1 < F.ny) wy += F.cy[c];
-        if (g == 1 && k + 1 < F.nz) wz += F.cz[c];
-      }
-    cd[q] = d;
-    cx[q] = wx;
-    cy[q] = wy;
-    cz[q] = wz;
+// ---- FP16 copies of the level-0 operator for the cycle.  The cycle only has to be
+// an approximate inverse (the solve stops on the FP64 residual), so its level-0
+// passes read the coefficients and the diagonal inverse as FP16, each group scaled
+// by a power of two that brings its maximum to [0.5, 1]: a third fewer bytes per
+// pass.  Zeros stay zero, so the cells outside the system stay out.
+
+__global__ void __launch_bounds__(256) k_mg_absmax(long long n, const float* __restrict__ cd,
+                                                   const float* __restrict__ cx, const float* __restrict__ cy,
+                                                   const float* __restrict__ cz, const float* __restrict__ inv,
+                                                   float* mx) {
+  float ma = 0.0f, mi = 0.0f;
+  for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long long)gridDim.x * 256) {
+    ma = fmaxf(ma, fmaxf(fmaxf(cd[q], cx[q]), fmaxf(cy[q], cz[q])));
+    mi = fmaxf(mi, inv[q]);
   }
+  mg_store_max(ma, mi, mx);
 }
 
-// inv = 1 / A_II (0 outside the system)
-__global__ void __launch_bounds__(256) k_mg_inverse(MgLevel L, float* __restrict__ inv) {
+// the fine couplings that cross the +x, +y or +z face of aggregate (I, J, K), summed over
+// its four children there in a fixed order
+__device__ inline float mg_cross(const MgLevel& F, const float* __restrict__ cw, int ax, int I, int J, int K) {
+  float w = 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int lo = e & 1, hi = e >> 1;
+    const int i = 2 * I + (ax == 0 ? 1 : lo), j = 2 * J + (ax == 1 ? 1 : (ax == 0 ? lo : hi)),
+              k = 2 * K + (ax == 2 ? 1 : hi);
+    if (i >= F.nx || j >= F.ny || k >= F.nz) continue;
+    if ((ax == 0 ? i + 1 < F.nx : (ax == 1 ? j + 1 < F.ny : k + 1 < F.nz))) w += cw[bm_index(F.d, i, j, k)];
+  }
+  return w;
+}
+
+// The Galerkin coarse operator of level F in slab cell q: the sum of the children's cd,
+// the couplings crossing each upper face, and 1 / A_II (0 outside the system), whose
+// lower couplings are the lower aggregates' upper ones, summed again here instead of in
+// a pass of their own.  ma, mi: running maxima.
+__device__ inline void mg_coarsen_cell(const MgLevel& F, const MgLevel& Cl, long long q, float* cd, float* cx,
+                                       float* cy, float* cz, float* inv, float& ma, float& mi) {
+  int I, J, K;
+  mg_coords(Cl.d, q, I, J, K);
+  float d = 0.0f, wx = 0.0f, wy = 0.0f, wz = 0.0f, a = 0.0f;
+  if (I < Cl.nx && J < Cl.ny && K < Cl.nz) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int i = 2 * I + (e & 1), j = 2 * J + ((e >> 1) & 1), k = 2 * K + (e >> 2);
+      if (i < F.nx && j < F.ny && k < F.nz) d += F.cd[bm_index(F.d, i, j, k)];
+    }
+    wx = mg_cross(F, F.cx, 0, I, J, K);
+    wy = mg_cross(F, F.cy, 1, I, J, K);
+    wz = mg_cross(F, F.cz, 2, I, J, K);
+    a = d + wx + wy + wz;
+    if (I > 0) a += mg_cross(F, F.cx, 0, I - 1, J, K);
+    if (J > 0) a += mg_cross(F, F.cy, 1, I, J - 1, K);
+    if (K > 0) a += mg_cross(F, F.cz, 2, I, J, K - 1);
+  }
+  const float v = a > 0.0f ? 1.0f / a : 0.0f;
+  cd[q] = d; cx[q] = wx; cy[q] = wy; cz[q] = wz;
+  inv[q] = v;
+  ma = fmaxf(ma, fmaxf(fmaxf(d, wx), fmaxf(wy, wz)));
+  mi = fmaxf(mi, v);
+}
+
+__global__ void __launch_bounds__(256) k_mg_coarsen(MgLevel F, MgLevel Cl, float* __restrict__ cd,
+                                                    float* __restrict__ cx, float* __restrict__ cy,
+                                                    float* __restrict__ cz, float* __restrict__ inv, float* mx) {
+  float ma = 0.0f, mi = 0.0f;
+  for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < Cl.d.nblocks * kBlockVol;
+       q += (long long)gridDim.x * 256)
+    mg_coarsen_cell(F, Cl, q, cd, cx, cy, cz, inv, ma, mi);
+  mg_store_max(ma, mi, mx);
+}
+
+// inv = 1 / A_II (0 outside the system) and the level's maxima, for a level whose
+// operator another kernel built (the multires block grid)
+__global__ void __launch_bounds__(256) k_mg_inverse(MgLevel L, float* __restrict__ inv, float* mx) {
+  float ma = 0.0f, mi = 0.0f;
   for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < L.d.nblocks * kBlockVol;
        q += (long long)gridDim.x * 256) {
     int i, j, k;
@@ -226,35 +272,12 @@ __global__ void __launch_bounds__(256) k_mg_inverse(MgLevel L, float* __restrict
       if (j > 0) a += L.cy[bm_index(L.d, i, j - 1, k)];
       if (k > 0) a += L.cz[bm_index(L.d, i, j, k - 1)];
     }
-    inv[q] = a > 0.0f ? 1.0f / a : 0.0f;
+    const float v = a > 0.0f ? 1.0f / a : 0.0f;
+    inv[q] = v;
+    ma = fmaxf(ma, fmaxf(fmaxf(L.cd[q], L.cx[q]), fmaxf(L.cy[q], L.cz[q])));
+    mi = fmaxf(mi, v);
   }
-}
-
-// ---- FP16 copies of the level-0 operator for the cycle.  The cycle only has to be
-// an approximate inverse (the solve stops on the FP64 residual), so its level-0
-// passes read the coefficients and the diagonal inverse as FP16, each group scaled
-// by a power of two that brings its maximum to [0.5, 1]: a third fewer bytes per
-// pass.  Zeros stay zero, so the cells outside the system stay out.
-
-// mx[0] = max of cd, cx, cy, cz; mx[1] = max of inv (float bits; all values >= 0)
-__global__ void __launch_bounds__(256) k_mg_absmax(long long n, const float* __restrict__ cd,
-                                                   const float* __restrict__ cx, const float* __restrict__ cy,
-                                                   const float* __restrict__ cz, const float* __restrict__ inv,
-                                                   uint32_t* mx) {
-  float ma = 0.0f, mi = 0.0f;
-  for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long long)gridDim.x * 256) {
-    ma = fmaxf(ma, fmaxf(fmaxf(cd[q], cx[q]), fmaxf(cy[q], cz[q])));
-    mi = fmaxf(mi, inv[q]);
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    ma = fmaxf(ma, __shfl_xor(ma, o, 64));
-    mi = fmaxf(mi, __shfl_xor(mi, o, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMax(&mx[0], __float_as_uint(ma));
-    atomicMax(&mx[1], __float_as_uint(mi));
-  }
+  mg_store_max(ma, mi, mx);
 }
 
 // 2^e with e = the exponent that brings m to [0.5, 1) (1 for m = 0 or not finite)
@@ -270,9 +293,27 @@ __global__ void __launch_bounds__(256) k_mg_tohalf(long long n, const float* __r
                                                    const float* __restrict__ cz, const float* __restrict__ inv,
                                                    _Float16* __restrict__ hcd, _Float16* __restrict__ hcx,
                                                    _Float16* __restrict__ hcy, _Float16* __restrict__ hcz,
-                                                   _Float16* __restrict__ hinv, const uint32_t* mx,
-                                                   float* __restrict__ unscale) {
-  const float ua = mg_pow2_above(__uint_as_float(mx[0])), ui = mg_pow2_above(__uint_as_float(mx[1]));
+                                                   _Float16* __restrict__ hinv, const float* __restrict__ mx,
+                                                   int nmx, float* __restrict__ unscale) {
+  __shared__ float s_mx[4][2];
+  float ma = 0.0f, mi = 0.0f;
+  for (int t = threadIdx.x; t < nmx; t += 256) {
+    ma = fmaxf(ma, mx[t]);
+    mi = fmaxf(mi, mx[kMaxPartials + t]);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    ma = fmaxf(ma, __shfl_xor(ma, o, 64));
+    mi = fmaxf(mi, __shfl_xor(mi, o, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_mx[threadIdx.x >> 6][0] = ma;
+    s_mx[threadIdx.x >> 6][1] = mi;
+  }
+  __syncthreads();
+  ma = fmaxf(fmaxf(s_mx[0][0], s_mx[1][0]), fmaxf(s_mx[2][0], s_mx[3][0]));
+  mi = fmaxf(fmaxf(s_mx[0][1], s_mx[1][1]), fmaxf(s_mx[2][1], s_mx[3][1]));
+  const float ua = mg_pow2_above(ma), ui = mg_pow2_above(mi);
   const float sa = 1.0f / ua, si = 1.0f / ui;  // powers of two: exact
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     unscale[0] = ua;

@@ -243,10 +243,31 @@ __global__ void __launch_bounds__(256) k_pin_detect(ProjArgs a) {
     const uint32_t air = s_air[0] | s_air[1] | s_air[2] | s_air[3];
     const uint32_t mn = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
     const uint32_t cnt = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-    if (air) atomicOr(&a.pin[0], 1u);
-    if (mn != 0xffffffffu) atomicMin(&a.pin[1], mn);
+    // (the flag and the minimum settle early: look before the atomic)
+    if (air && !__hip_atomic_load(&a.pin[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&a.pin[0], 1u);
+    if (mn < __hip_atomic_load(&a.pin[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&a.pin[1], mn);
     if (cnt) atomicAdd(&a.pin[4], cnt);
   }
+}
+
+// A level's maxima of cd, cx, cy, cz (mx[w]) and of inv (mx[kMaxPartials + w]), one per
+// workgroup w; the reader takes the maximum over them.  (One atomicMax per wave on the
+// two words took 23 to 50 us a level, and 300 us of the assembly's 390 at 128^3.)
+__device__ inline void mg_store_max(float ma, float mi, float* mx) {
+  __shared__ float s_mx[4][2];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    ma = fmaxf(ma, __shfl_xor(ma, o, 64));
+    mi = fmaxf(mi, __shfl_xor(mi, o, 64));
+  }
+  if ((threadIdx.x & 63) == 0) {
+    s_mx[threadIdx.x >> 6][0] = ma;
+    s_mx[threadIdx.x >> 6][1] = mi;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2)
+    mx[threadIdx.x * kMaxPartials + blockIdx.x] =
+        fmaxf(fmaxf(s_mx[0][threadIdx.x], s_mx[1][threadIdx.x]), fmaxf(s_mx[2][threadIdx.x], s_mx[3][threadIdx.x]));
 }
 
 struct AsmOut {
@@ -255,8 +276,8 @@ struct AsmOut {
   const float *u, *v, *w, *mu, *mv, *mw;
   double* part;   // slot 0: sum b^2, slot 1: max |b| (the FP64 residual of x = 0)
   float *fbeta, *fphi;  // optional learned-preconditioner features (mean face beta / phi)
-  uint32_t* mx;   // optional: max of the FP32 cd, cx, cy, cz and max of inv (float bits,
-                  // atomicMax; the values are >= 0), what the multigrid build scales by
+  float* mx;      // optional: per workgroup the max of the FP32 cd, cx, cy, cz and (from
+                  // kMaxPartials on) of inv, what the multigrid build scales by
 };
 
 // RHS and assembly, sparse_ops3d_tp.cpp:266-313
@@ -369,18 +390,7 @@ __global__ void __launch_bounds__(256) k_assemble(ProjArgs a, AsmOut o) {
   double v[2] = {bb, bmax};
   const bool mx[2] = {false, true};
   block_reduce_store<2>(v, mx, o.part, kMaxPartials);
-  if (o.mx) {
-    // (fmaxf drops a NaN, as the separate pass over the slab does)
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-      amax = fmaxf(amax, __shfl_xor(amax, s, 64));
-      imax = fmaxf(imax, __shfl_xor(imax, s, 64));
-    }
-    if (lane == 0) {
-      atomicMax(&o.mx[0], __float_as_uint(amax));
-      atomicMax(&o.mx[1], __float_as_uint(imax));
-    }
-  }
+  if (o.mx) mg_store_max(amax, imax, o.mx);  // (fmaxf drops a NaN)
 }
 
 // zero every per-cell array of the listed blocks (blocks that leave the fluid set
