@@ -4,11 +4,10 @@ change to the form that loads after the sums (more than 512 workgroups), and the
 iteration budget at a restart.
 
 Bars: the FP64 oracle's pressure where it is quick (1e-6, the bar of the other projection
-tests), and on larger open tanks the multigrid solve of the same system to the same FP64
-residual.  The two pressures differ by A^-1 of the two residuals, so the velocities'
-difference falls in proportion to the tolerance: at 1e-9 they were 1.1e-5 apart (with a
-density ratio of 1000 the light phase's velocity shows it most), at the 1e-11 used here
-that is 1.1e-7, two orders inside the field bar of 1e-5.
+tests), and on larger open tanks the multigrid solve of the same system to a residual of
+1e-11.  There the velocities' bound is the FP32 storage of the pressure: each of the two
+pressures of a face is off by up to 2^-24 max|p| in either solve, which the face update
+multiplies by (dt / dx) beta, at most (dt / dx) / rho_g.
 """
 import numpy as np
 import pytest
@@ -63,15 +62,16 @@ def test_matches_the_oracle(shape, kind):
 @pytest.mark.parametrize("shape", [(72, 72, 72), (84, 83, 82), (101, 35, 34)])
 def test_matches_multigrid_on_larger_grids(shape):
     print(f"[cg] {shape}", flush=True)
-    _, ctx, _, _, gph = _context(shape, O.SCENE_BUBBLE)
+    dx, ctx, _, _, gph = _context(shape, O.SCENE_BUBBLE)
     faces = []
     for pre in (G.PRECOND_JACOBI, G.PRECOND_MULTIGRID):
         _grid_half(ctx, gph)
         st = ctx.project(gph, 1e-3, G.default_solve_cfg(G.STOP_REL2, 1e-11, 20000, pre))
         assert st.converged == 1 and st.true_rel_residual <= 1e-11 and st.fallback_used == 0
         faces.append([ctx.field(f) for f in range(3)])
+    bound = 4 * (1e-3 / dx) / gph.rho_g * 2.0 ** -24 * np.abs(ctx.field(G.FIELD_P)).max()
     for a, b in zip(*faces):
-        assert rel_err(a, b) < 1e-5
+        assert np.abs(a - b).max() < bound
 
 
 @pytest.mark.parametrize("budget", [1, 2, 60])
