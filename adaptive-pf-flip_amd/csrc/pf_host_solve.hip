@@ -229,6 +229,50 @@ std::vector<float> mg_sweep_weights(const pf_ctx* c) {
   return w;
 }
 
+// Whether the cycle from level l (1..nl) down runs in k_mg_tail: at least two sweeps (the
+// row kernels' FP16 operator), at most a row per thread on level l, and all levels' blocks
+// in its LDS.
+bool mg_in_tail(const pf_ctx* c, int l) {
+  const size_t nl = c->mg.size();
+  long long blocks = 0;
+  for (size_t q = (size_t)l - 1; q < nl; ++q) blocks += c->mg[q].d.nblocks;
+  return c->mg_cfg.sweeps >= 2 && c->mg_cfg.sweeps <= kTailSweeps &&
+         c->mg[(size_t)l - 1].d.nblocks * 16 <= kTailThreads && blocks <= kTailBlocks &&
+         nl - (size_t)l + 1 <= kTailLevels;
+}
+
+float* mg_tail(pf_ctx* c, int l, const int* done, const std::vector<float>& wpre) {
+  MgTailArgs a{};
+  a.done = done;
+  a.n = (int)c->mg.size() - l + 1;
+  int off = 0;
+  for (int q = 0; q < a.n; ++q) {
+    const Ctx::MgBuf& b = c->mg[(size_t)(l - 1 + q)];
+    MgTailLevel& L = a.lv[q];
+    L.d = b.d;
+    L.cd = reinterpret_cast<const _Float16*>(b.h[0]);
+    L.cx = reinterpret_cast<const _Float16*>(b.h[1]);
+    L.cy = reinterpret_cast<const _Float16*>(b.h[2]);
+    L.cz = reinterpret_cast<const _Float16*>(b.h[3]);
+    L.inv = reinterpret_cast<const _Float16*>(b.h[4]);
+    L.unscale = b.unscale;
+    L.rows = (int)b.d.nblocks * 16;
+    L.off = off;
+    off += L.rows * 4;
+  }
+  a.last = mg_level(c->mg.back());
+  Ctx::MgBuf& top = c->mg[(size_t)l - 1];
+  a.r = top.r;
+  a.x = top.x;
+  a.nu = c->mg_cfg.sweeps;
+  for (int q = 0; q < a.nu; ++q) a.w[q] = wpre[(size_t)q];
+  a.coarsest_sweeps = c->mg_cfg.coarsest_sweeps;
+  a.omega = c->mg_cfg.omega;
+  a.omega_c = c->mg_cfg.correction;
+  hipLaunchKernelGGL(k_mg_tail, dim3(1), dim3(kTailThreads), 0, c->stream, a);
+  return top.x;
+}
+
 // coarse levels: level l (1..nl) solves A_l x = r_l from zero (its buffer r holds r_l);
 // returns the buffer that holds x.  (Two corrections per level -- a W-cycle -- cost
 // more launches than they save iterations at 256^3, and twice the 1.8 over-correction
@@ -236,6 +280,7 @@ std::vector<float> mg_sweep_weights(const pf_ctx* c) {
 float* mg_coarse(pf_ctx* c, int l, const int* done, const std::vector<float>& wpre) {
   const int nl = (int)c->mg.size();
   const int nu = c->mg_cfg.sweeps;
+  if (mg_in_tail(c, l)) return mg_tail(c, l, done, wpre);
   MgWalk wd{nullptr, 0, done};
   Ctx::MgBuf& b = c->mg[(size_t)l - 1];
   const MgLevel L = mg_level(b);

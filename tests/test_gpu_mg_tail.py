@@ -4,16 +4,17 @@ keeps the row kernels), ragged and elongated hierarchies, and every sweep count 
 takes (one sweep keeps the separate kernels).
 
 Bar: the projection to a relative FP64 residual of 1e-10 agrees with the Jacobi solve of
-the same open tank to 1e-5 in the velocities (their difference falls in proportion to the
-residuals; at 1e-9 such tanks were 1.1e-5 apart, so 1e-10 leaves a factor of ten), in far
-fewer iterations, without the fallback that a wrong cycle ends in.
+the same open tank in far fewer iterations, without the fallback that a wrong cycle ends
+in.  The velocities' bound: the pressure is stored in FP32, so each of the two pressures of
+a face is off by up to 2^-24 max|p| in either solve, which the face update multiplies by
+(dt / dx) beta, at most (dt / dx) / rho_g: 4 (dt / dx) / rho_g 2^-24 max|p| on a face.
 """
 import numpy as np
 import pytest
 
 import pfflip_amd as G
 import pyoracle as O
-from _helpers import phase, rel_err, scene
+from _helpers import phase, scene
 
 pytestmark = pytest.mark.gpu
 
@@ -34,26 +35,27 @@ def _solve(shape, pre, sweeps=None):
     ctx.apply_gravity(1e-3, -9.81)
     ctx.apply_walls()
     st = ctx.project(gph, 1e-3, G.default_solve_cfg(G.STOP_REL2, 1e-10, 20000, pre))
-    return st, [ctx.field(f) for f in range(3)]
+    p = ctx.field(G.FIELD_P)
+    return st, [ctx.field(f) for f in range(3)], 4 * (1e-3 / dx) / oph.rho_g * 2.0 ** -24 * np.abs(p).max()
 
 
 @pytest.mark.parametrize("shape", [(8, 8, 8), (9, 7, 8), (16, 15, 17), (32, 33, 30), (36, 20, 12), (66, 64, 34),
                                    (96, 24, 20), (70, 66, 36)])
 def test_cycle_with_the_tail(shape):
     print(f"[tail] {shape}", flush=True)
-    mg, f_mg = _solve(shape, G.PRECOND_MULTIGRID)
-    ja, f_ja = _solve(shape, G.PRECOND_JACOBI)
+    mg, f_mg, bound = _solve(shape, G.PRECOND_MULTIGRID)
+    ja, f_ja, _ = _solve(shape, G.PRECOND_JACOBI)
     assert mg.converged == 1 and ja.converged == 1 and mg.fallback_used == 0
     assert mg.iterations < ja.iterations
     for a, b in zip(f_mg, f_ja):
-        assert rel_err(a, b) < 1e-5
+        assert np.abs(a - b).max() < bound
 
 
 @pytest.mark.parametrize("sweeps", [1, 2, 3, 5, 16])
 def test_sweep_counts(sweeps):
     print(f"[tail] sweeps {sweeps}", flush=True)
-    mg, f_mg = _solve((40, 36, 28), G.PRECOND_MULTIGRID, sweeps)
-    ja, f_ja = _solve((40, 36, 28), G.PRECOND_JACOBI)
+    mg, f_mg, bound = _solve((40, 36, 28), G.PRECOND_MULTIGRID, sweeps)
+    ja, f_ja, _ = _solve((40, 36, 28), G.PRECOND_JACOBI)
     assert mg.converged == 1 and mg.fallback_used == 0 and mg.iterations * 2 < ja.iterations
     for a, b in zip(f_mg, f_ja):
-        assert rel_err(a, b) < 1e-5
+        assert np.abs(a - b).max() < bound
