@@ -33,7 +33,7 @@
 #include "pf_render.hip"
 #include "pf_mg.hip"
 #include "pf_mg_tail.hip"
-#include "pf_mr_mg.hip"
+#include "pf_mr_row.hip"
 #include "pf_lpc_cw.hip"
 
 using namespace pf;
@@ -205,7 +205,7 @@ int pf_destroy(pf_ctx* c) {
   for (double* p : f64) hipFree(p);
   dfree(c->mr_lvl); dfree(c->mr_vol64); dfree(c->mr_pfull); dfree(c->mr_bbox); dfree(c->mr_leaves_dev);
   dfree(c->mrf); dfree(c->mrc); dfree(c->mr_pin_dev);
-  dfree(c->mr_f01); dfree(c->mr_f2); dfree(c->mr_list01); dfree(c->mr_list2);
+  dfree(c->mr_info);
   dfree(c->iface); dfree(c->iface_bad);
   dfree(c->pa_alive); dfree(c->pa_key); dfree(c->pa_by_id); dfree(c->pa_new_id);
   dfree(c->pa_cflag); dfree(c->pa_d1); dfree(c->pa_d2); dfree(c->pa_wanted); dfree(c->pa_wscan); dfree(c->pa_cnt);
@@ -220,7 +220,7 @@ int pf_destroy(pf_ctx* c) {
   dfree(c->mg_mx);
   dfree(c->mg_unscale);
   if (c->mr_pin_host) hipHostFree(c->mr_pin_host);
-  for (int a = 0; a < 3; ++a) { dfree(c->mr_valid[a]); dfree(c->mr_cf32[a]); dfree(c->mr_cf64[a]); }
+  for (int a = 0; a < 3; ++a) { dfree(c->mr_valid[a]); dfree(c->mr_cf64[a]); }
   if (c->mr_bbox_host) hipHostFree(c->mr_bbox_host);
   dfree(c->fbeta); dfree(c->fphi); dfree(c->tiles); dfree(c->tile_flags); dfree(c->snaps);
   hipFree(c->sc); hipFree(c->partial); hipFree(c->red);

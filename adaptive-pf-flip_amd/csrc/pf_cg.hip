@@ -231,6 +231,57 @@ __device__ inline void cg_publish(const CgArgs& a, const SolveScalars& S) {
 
 // The list in slots of four blocks (one per 16 lanes of a wave), each XCD a contiguous
 // eighth.
+// The last launch's partial sums: every one that a thread adds is loaded before any is
+// waited for (a load of what other XCDs just wrote takes 1 to 2 us).
+__device__ inline void cg_fetch(const CgArgs& a, double (&w)[4][CG_SUMS]) {
+  const auto bs = buf_rsrc(a.sums, CG_SUMS * kMaxPartials * 8);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int k = 0; k < CG_SUMS; ++k) {
+      const uint32_t t = threadIdx.x + 256 * j;
+      w[j][k] = buf_ld_f64(bs, t < (uint32_t)a.nsums ? (k * kMaxPartials + t) * 8 : kNoLoad);
+    }
+}
+
+// The sums and the recursion's next scalars in S, published by the first workgroup; false
+// when this launch has nothing to do.
+__device__ inline bool cg_advance(const CgArgs& a, const double (&w)[4][CG_SUMS], SolveScalars& S,
+                                  double (&sh)[4][CG_SUMS]) {
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (S.done) {
+    if (lead) cg_publish(a, S);
+    return false;
+  }
+  double v[CG_SUMS];
+#pragma unroll
+  for (int k = 0; k < CG_SUMS; ++k) v[k] = wave_sum((w[0][k] + w[1][k]) + (w[2][k] + w[3][k]));
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < CG_SUMS; ++k) sh[threadIdx.x >> 6][k] = v[k];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < CG_SUMS; ++k) v[k] = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
+  const bool go = cg_scalars(S, v);
+  if (go) S.par ^= 1;
+  if (lead) cg_publish(a, S);
+  return go;
+}
+
+// this launch's partial sums
+__device__ inline void cg_store_sums(const CgArgs& a, double (&v)[CG_SUMS], double (&sh)[4][CG_SUMS]) {
+#pragma unroll
+  for (int k = 0; k < CG_SUMS; ++k) v[k] = wave_sum(v[k]);
+  __syncthreads();  // (every wave has read the sums in sh)
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int k = 0; k < CG_SUMS; ++k) sh[threadIdx.x >> 6][k] = v[k];
+  __syncthreads();
+  if (threadIdx.x < CG_SUMS)
+    a.sums_out[threadIdx.x * kMaxPartials + blockIdx.x] =
+        (sh[0][threadIdx.x] + sh[1][threadIdx.x]) + (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
+}
+
 // one row's inputs
 struct CgLoads {
   CgRow R;
@@ -247,17 +298,8 @@ template <bool PRE>
 __global__ void __launch_bounds__(256) k_cg_iter(CgArgs a) {
   __shared__ double sh[4][CG_SUMS];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // every partial this thread sums is loaded before any is waited for (a load of what
-  // other XCDs just wrote takes 1 to 2 us)
   double w[4][CG_SUMS];
-  const auto bs = buf_rsrc(a.sums, CG_SUMS * kMaxPartials * 8);
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int k = 0; k < CG_SUMS; ++k) {
-      const uint32_t t = threadIdx.x + 256 * j;
-      w[j][k] = buf_ld_f64(bs, t < (uint32_t)a.nsums ? (k * kMaxPartials + t) * 8 : kNoLoad);
-    }
+  cg_fetch(a, w);
   const uint32_t bytes = (uint32_t)(a.dc.nblocks * kBlockVol * 4);
   const uint32_t sy = (uint32_t)a.dc.nbx * kBlockVol * 4, sz = sy * (uint32_t)a.dc.nby;
   const auto br = buf_rsrc(a.r, bytes), bq = buf_rsrc(a.q, bytes), bp = buf_rsrc(a.p, bytes);
@@ -283,32 +325,14 @@ __global__ void __launch_bounds__(256) k_cg_iter(CgArgs a) {
   };
   if (PRE && t0 < e) load();
   SolveScalars S = cg_state(a.in);
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-  if (S.done) {
-    if (lead) cg_publish(a, S);
-    return;
-  }
-  double v[CG_SUMS];
-#pragma unroll
-  for (int k = 0; k < CG_SUMS; ++k) v[k] = wave_sum((w[0][k] + w[1][k]) + (w[2][k] + w[3][k]));
-  if (lane == 0)
-#pragma unroll
-    for (int k = 0; k < CG_SUMS; ++k) sh[wave][k] = v[k];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < CG_SUMS; ++k) v[k] = (sh[0][k] + sh[1][k]) + (sh[2][k] + sh[3][k]);
-  const bool go = cg_scalars(S, v);
-  if (go) S.par ^= 1;
-  if (lead) cg_publish(a, S);
-  if (!go) return;
+  if (!cg_advance(a, w, S, sh)) return;
   const float alpha = (float)S.alpha, beta = (float)S.beta;
   // the new p of any cell from the old r, q, p (the same arithmetic for a block's own
   // cells and for its neighbours')
   auto direction = [&](float r, float q, float p, float inv) {
     return fmaf(beta, p, inv * fmaf(-alpha, q, r));
   };
-#pragma unroll
-  for (int k = 0; k < CG_SUMS; ++k) v[k] = 0.0;
+  double v[CG_SUMS] = {};
   while (t0 < e) {
     if (!PRE) load();
     F4 pn, rn, xn, py, pz;
@@ -338,16 +362,7 @@ __global__ void __launch_bounds__(256) k_cg_iter(CgArgs a) {
     t0 += step;
     if (PRE && t0 < e) load();
   }
-#pragma unroll
-  for (int k = 0; k < CG_SUMS; ++k) v[k] = wave_sum(v[k]);
-  __syncthreads();  // (every wave has read the sums in sh)
-  if (lane == 0)
-#pragma unroll
-    for (int k = 0; k < CG_SUMS; ++k) sh[wave][k] = v[k];
-  __syncthreads();
-  if (threadIdx.x < CG_SUMS)
-    a.sums_out[threadIdx.x * kMaxPartials + blockIdx.x] =
-        (sh[0][threadIdx.x] + sh[1][threadIdx.x]) + (sh[2][threadIdx.x] + sh[3][threadIdx.x]);
+  cg_store_sums(a, v, sh);
 }
 
 }  // namespace pf

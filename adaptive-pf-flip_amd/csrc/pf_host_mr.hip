@@ -169,9 +169,8 @@ int mr_apply_layout(pf_ctx* c, std::vector<Leaf> lv) {
     HIP_TRY(c, dalloc(&c->mr_lvl, ncell));
     for (int a = 0; a < 3; ++a) {
       HIP_TRY(c, dalloc(&c->mr_valid[a], fd[a]->nblocks * kBlockVol));
-      HIP_TRY(c, dalloc(&c->mr_cf32[a], fd[a]->nblocks * kBlockVol));
-      HIP_TRY(c, dalloc(&c->mr_cf64[a], fd[a]->nblocks * kBlockVol));
     }
+    HIP_TRY(c, dalloc(&c->mr_info, c->dc.nblocks));
     HIP_TRY(c, dalloc(&c->mr_vol64, ncell));
     HIP_TRY(c, dalloc(&c->mr_pfull, ncell));
   }
@@ -188,6 +187,8 @@ int mr_apply_layout(pf_ctx* c, std::vector<Leaf> lv) {
   HIP_TRY(c, fill_u8(c->stream, c->mr_lvl, 255, ncell));
   hipLaunchKernelGGL(k_mr_levels, dim3((unsigned)lv.size()), dim3(256), 0, c->stream, c->mr_leaves_dev, (int)lv.size(),
                      c->dc, c->geom, c->mr_lvl);
+  LAUNCH_CHECK(c);
+  hipLaunchKernelGGL(k_mr_info, dim3(grid_for(c->dc.nblocks, 256)), dim3(256), 0, c->stream, mr_grid(c), c->mr_info);
   LAUNCH_CHECK(c);
   c->mr = true;
   for (int a = 0; a < 3; ++a) {

@@ -147,38 +147,9 @@ int mg_coarsen_from(pf_ctx* c, MgLevel F, size_t from) {
   return PF_OK;
 }
 
-// The multires fluid list split by level for the fast solves: blocks of level 0-1 (a
-// wave each) and level-2 blocks (one cell each, four to a wave).  The level-2 kernels
-// write a block's cell entry only, so the PCG's z, p and A p start as zeros.
-int mr_split_lists(pf_ctx* c, const MrGrid& m) {
-  const long long nb = c->dc.nblocks;
-  if (!c->mr_list2) {
-    HIP_TRY(c, dalloc(&c->mr_f01, nb));
-    HIP_TRY(c, dalloc(&c->mr_f2, nb));
-    HIP_TRY(c, dalloc(&c->mr_list01, nb));
-    HIP_TRY(c, dalloc(&c->mr_list2, nb));
-  }
-  HIP_TRY(c, fill_u8(c->stream, c->mr_f01, 0, nb));
-  HIP_TRY(c, fill_u8(c->stream, c->mr_f2, 0, nb));
-  hipLaunchKernelGGL(k_mr_mg_split, dim3(grid_for(c->npblk, 256)), dim3(256), 0, c->stream, c->pblk, c->npblk, m,
-                     c->mr_f01, c->mr_f2);
-  LAUNCH_CHECK(c);
-  HIP_TRY(c, compact_flags_morton(*c, c->dc, c->mr_f01, c->mr_list01, c->u32_dev + 12));
-  HIP_TRY(c, compact_flags_morton(*c, c->dc, c->mr_f2, c->mr_list2, c->u32_dev + 13));
-  HIP_TRY(c, hipMemcpyAsync(c->u32_host + 12, c->u32_dev + 12, 2 * sizeof(uint32_t), hipMemcpyDeviceToHost,
-                            c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  c->mr_n01 = c->u32_host[12];
-  c->mr_n2 = c->u32_host[13];
-  if (c->mr_n01 + c->mr_n2 != c->npblk) return fail(c, PF_ERR_STATE, "multires block split lost blocks");
-  float* arrs[4] = {c->z32, c->pA, c->pB, c->Ap};
-  for (float* q : arrs) HIP_TRY(c, fill_f32(c->stream, q, 0.f, nb * kBlockVol));
-  return PF_OK;
-}
-
 // The multires cycle's levels: the block grid (the uniform hierarchy's second level,
 // c->mg[1]) from R S P, then the uniform levels below it.  Leaves of level 0..2 only.
-int mr_mg_build(pf_ctx* c, const MrOp& op) {
+int mr_mg_build(pf_ctx* c, const MrRowOp& op) {
   for (size_t a = 0; a < c->mr_leaves.size(); a += 4)
     if (c->mr_leaves[a] > 2)
       return fail(c, PF_ERR_ARG, "the multires multigrid takes leaves of level 0 to 2");
@@ -196,9 +167,6 @@ int mr_mg_build(pf_ctx* c, const MrOp& op) {
   hipLaunchKernelGGL(k_mr_mg_coarse, dim3(grid_for(c->dc.nblocks, 4)), dim3(256), 0, c->stream, op, b.d, b.cd, b.cx,
                      b.cy, b.cz);
   LAUNCH_CHECK(c);
-  // the level-2 kernels write the cell entry of a block only: the other entries of the
-  // cycle's work array stay zero
-  HIP_TRY(c, fill_f32(c->stream, c->mg_t0, 0.f, c->dc.nblocks * kBlockVol));
   const unsigned g = mg_build_grid(nl);
   hipLaunchKernelGGL(k_mg_inverse, dim3(g), dim3(256), 0, c->stream, mg_level(b), b.inv, c->mg_mx);
   mg_tohalf(c, mg_level(b), b.h, (int)g, b.unscale);
@@ -497,52 +465,85 @@ int mg_apply(pf_ctx* c, const float* r, float* z, const int* done, double* part)
   return mg_apply_on(c, c->pblk, c->npblk, r, z, done, part, nullptr);
 }
 
+// the assembled multires operator by cell rows (pf_mr_row.hip)
+MrRowOp mr_row_op(const pf_ctx* c) {
+  MrRowOp o;
+  o.dc = c->dc;
+  o.info = c->mr_info;
+  o.cd = c->cd32; o.cx = c->cx32; o.cy = c->cy32; o.cz = c->cz32; o.inv = c->invd32;
+  return o;
+}
+
+// workgroups: four list blocks to a wave, at most 1024 (every workgroup sums that many
+// partials of five quantities), a multiple of 8 (one share per XCD)
+unsigned cg_grid(long long nlist) {
+  return (unsigned)std::clamp<long long>((((nlist + 15) / 16 + 7) / 8) * 8, 8, 1024);
+}
+
+// the same without a sum to keep small
+unsigned mr_grid_wide(long long nlist) {
+  return (unsigned)std::clamp<long long>((((nlist + 15) / 16 + 7) / 8) * 8, 8, 8192);
+}
+
 // z = the multires cycle on r over the listed blocks: nu sweeps on S, the block sums of
 // the residual onto the block grid, the uniform cycle from there, the prolongation and
-// nu sweeps back, the last into z with the partial r.z (mg_grid0n workgroups) in slot 2
-// of part; skipped while *done
-int mr_mg_apply(pf_ctx* c, const MrOp& op, const VecArgs& va, const float* r, float* z, const int* done,
+// nu sweeps back, the last into z with the partial r.z (cg_grid workgroups) in slot 2 of
+// part; skipped while *done
+int mr_mg_apply(pf_ctx* c, const MrRowOp& op, const VecArgs& va, const float* r, float* z, const int* done,
                 double* part) {
   const int nu = std::max(1, c->mg_cfg.sweeps);
   std::vector<float> wpre = mg_sweep_weights(c);
   wpre.resize((size_t)nu, c->mg_cfg.omega);
-  const unsigned g0 = mg_grid0n(va.nlist);
-  double* const rz = part + 2 * kMaxPartials;
-  const float* inv = c->invd32;
-  // the blocks of level 0-1 (a wave each) and of level 2 (four to a wave)
-  VecArgs v01 = va;
-  v01.list = c->mr_list01;
-  v01.nlist = c->mr_n01;
-  const uint32_t* l2 = c->mr_list2;
-  const long long n2 = c->mr_n2;
-  const unsigned gw = list_grid(v01.nlist);
-  const unsigned gw2 = (unsigned)std::clamp<long long>((n2 + 15) / 16, 8, 4096);
-  // 2 nu writes (the prolongation adds in place): the first lands in the work array
+  Ctx::MgBuf& b = c->mg[1];
+  MrCycleArgs a{};
+  a.list = va.list;
+  a.nlist = va.nlist;
+  a.done = done;
+  a.op = op;
+  a.dcc = b.d;
+  a.r = r;
+  a.omega_c = c->mg_cfg.correction;
+  const unsigned g = cg_grid(va.nlist), gw = mr_grid_wide(va.nlist);
+  // the kernels that write an iterate alternate between the work array and z; the first
+  // is chosen so that the last lands in z
+  const int writes = (nu >= 2 ? nu - 1 : 1) + nu;
   float* cur = nullptr;
-  float* nxt = c->mg_t0;
+  float* nxt = (writes & 1) ? z : c->mg_t0;
   auto flip = [&]() {
     cur = nxt;
     nxt = (cur == z) ? c->mg_t0 : z;
   };
-  // one sweep over both lists; the last one leaves the partial r.z in slot 2 (the
-  // level-2 kernel adds its share to the partials the other one wrote)
-  auto sweep = [&](float w, bool last) {
-    hipLaunchKernelGGL(k_mr_mg_sweep, dim3(last ? g0 : gw), dim3(256), 0, c->stream, v01, op, done, inv, r, cur, nxt, w,
-                       last ? rz : nullptr);
-    hipLaunchKernelGGL(k_mr_mg_sweep2, dim3(last ? g0 : gw2), dim3(256), 0, c->stream, l2, n2, op, done, inv, r, cur,
-                       nxt, w, last ? rz : nullptr);
+  a.out = nxt;
+  if (nu >= 2) {
+    a.omega_u = wpre[0];
+    a.omega = wpre[1];
+    hipLaunchKernelGGL(k_mr_cycle<MG_FIRST2>, dim3(gw), dim3(256), 0, c->stream, a);
+  } else {
+    a.omega = wpre[0];
+    hipLaunchKernelGGL(k_mr_cycle_first, dim3(gw), dim3(256), 0, c->stream, a);
+  }
+  flip();
+  for (int q = 2; q < nu; ++q) {
+    a.x = cur; a.out = nxt;
+    a.omega = wpre[(size_t)q];
+    hipLaunchKernelGGL(k_mr_cycle<MG_SWEEP>, dim3(gw), dim3(256), 0, c->stream, a);
     flip();
-  };
-  for (int q = 0; q < nu; ++q) sweep(wpre[(size_t)q], false);
-  Ctx::MgBuf& b = c->mg[1];
-  hipLaunchKernelGGL(k_mr_mg_restrict, dim3(gw), dim3(256), 0, c->stream, v01, op, done, r, cur, b.d, b.r);
-  hipLaunchKernelGGL(k_mr_mg_restrict2, dim3(gw2), dim3(256), 0, c->stream, l2, n2, op, done, r, cur, b.d, b.r);
-  float* const xc = mg_coarse(c, 2, done, wpre);
-  hipLaunchKernelGGL(k_mr_mg_prolong, dim3(gw), dim3(256), 0, c->stream, v01, op, done, b.d, xc, cur,
-                     c->mg_cfg.correction);
-  hipLaunchKernelGGL(k_mr_mg_prolong2, dim3(gw2), dim3(256), 0, c->stream, l2, n2, op, done, b.d, xc, cur,
-                     c->mg_cfg.correction);
-  for (int q = 0; q < nu; ++q) sweep(wpre[(size_t)(nu - 1 - q)], q == nu - 1);
+  }
+  a.x = cur;
+  a.out = b.r;
+  hipLaunchKernelGGL(k_mr_cycle<MG_RESTRICT>, dim3(gw), dim3(256), 0, c->stream, a);
+  a.xc = mg_coarse(c, 2, done, wpre);
+  for (int q = 0; q < nu; ++q) {
+    a.x = cur; a.out = nxt;
+    a.omega = wpre[(size_t)(nu - 1 - q)];
+    a.part = q == nu - 1 ? part + 2 * kMaxPartials : nullptr;
+    const dim3 grid(a.part ? g : gw);
+    if (q == 0)
+      hipLaunchKernelGGL(k_mr_cycle<MG_PSWEEP>, grid, dim3(256), 0, c->stream, a);
+    else
+      hipLaunchKernelGGL(k_mr_cycle<MG_SWEEP>, grid, dim3(256), 0, c->stream, a);
+    flip();
+  }
   LAUNCH_CHECK(c);
   if (cur != z) return fail(c, PF_ERR_STATE, "multires multigrid: cycle did not end in z");
   return PF_OK;
@@ -578,16 +579,17 @@ CgArgs cg_args(const pf_ctx* c, const CgState& g, const VecArgs& va) {
   return a;
 }
 
-// workgroups: four list blocks to a wave, at most 1024 (every workgroup sums that many
-// partials of five quantities), a multiple of 8 (one share per XCD)
-unsigned cg_grid(long long nlist) {
-  return (unsigned)std::clamp<long long>((((nlist + 15) / 16 + 7) / 8) * 8, 8, 1024);
-}
-
 // the FP64 residual into the buffers that the next launch reads, the direction zero
 // before the first iteration
 int cg_load(pf_ctx* c, CgState& g, VecArgs va, unsigned G, const double* r_src, bool first) {
   va.part = cg_sums(c, g.sums);
+  if (c->mr) {
+    g.nsums = (int)cg_grid(va.nlist);
+    hipLaunchKernelGGL(k_mr_load, dim3((unsigned)g.nsums), dim3(256), 0, c->stream, va, mr_row_op(c), r_src, c->x32,
+                       cg_r(c, g.par), first ? cg_p(c, g.par) : nullptr, first ? cg_q(c, g.par) : nullptr, nullptr, 1);
+    LAUNCH_CHECK(c);
+    return PF_OK;
+  }
   g.nsums = (int)std::min(G, 1024u);
   hipLaunchKernelGGL(k_cg_load, dim3((unsigned)g.nsums), dim3(256), 0, c->stream, va, r_src, c->x32, cg_r(c, g.par),
                      first ? cg_p(c, g.par) : nullptr, first ? cg_q(c, g.par) : nullptr, c->invd32);
@@ -632,7 +634,9 @@ int cg_run(pf_ctx* c, CgState& g, const VecArgs& va, int check, const Look& look
     ++g.seq;
     const CgArgs a = cg_args(c, g, va);
     const long long ki = kbegin(c, PF_K_PCG_SPMV);
-    if (grid <= 512)
+    if (c->mr)
+      hipLaunchKernelGGL(k_mr_cg_iter, dim3(grid), dim3(256), 0, c->stream, a, mr_row_op(c));
+    else if (grid <= 512)
       hipLaunchKernelGGL(k_cg_iter<true>, dim3(grid), dim3(256), 0, c->stream, a);
     else
       hipLaunchKernelGGL(k_cg_iter<false>, dim3(grid), dim3(256), 0, c->stream, a);
@@ -772,12 +776,6 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     HIP_TRY(c, fill_u32(c->stream, reinterpret_cast<uint32_t*>(c->mr_pin_dev), 0xffffffffu, 2));
   }
   if (mr) {
-    // multires: couplings are written per fine face, so the arrays start at zero
-    const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
-    for (int a = 0; a < 3; ++a) {
-      HIP_TRY(c, fill_f32(c->stream, c->mr_cf32[a], 0.f, fd[a]->nblocks * kBlockVol));
-      HIP_TRY(c, fill_f64(c->stream, c->mr_cf64[a], 0.0, fd[a]->nblocks * kBlockVol));
-    }
     MrAsm ma{};
     ma.m = mr_grid(c);
     ma.list = c->pblk; ma.nlist = npb;
@@ -785,20 +783,35 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     ma.dt = dt; ma.cdiv = cdiv; ma.pin = c->u32_dev;
     ma.u = c->f[F_U]; ma.v = c->f[F_V]; ma.w = c->f[F_W];
     ma.mu = c->f[F_MU]; ma.mv = c->f[F_MV]; ma.mw = c->f[F_MW];
-    ma.b64 = c->b64; ma.cd64 = c->cd64; ma.vol64 = c->mr_vol64;
-    ma.cd32 = c->cd32; ma.invd32 = c->invd32;
-    for (int a = 0; a < 3; ++a) { ma.cf64[a] = c->mr_cf64[a]; ma.cf32[a] = c->mr_cf32[a]; }
     ma.part = c->partial;
     if (refmode) {
+      // the couplings are written per fine face, so the arrays start at zero
+      const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
+      for (int a = 0; a < 3; ++a) {
+        const long long n = fd[a]->nblocks * kBlockVol;
+        if (!c->mr_cf64[a]) HIP_TRY(c, dalloc(&c->mr_cf64[a], n));
+        HIP_TRY(c, fill_f64(c->stream, c->mr_cf64[a], 0.0, n));
+        ma.cf64[a] = c->mr_cf64[a];
+      }
+      ma.b64 = c->b64; ma.cd64 = c->cd64; ma.vol64 = c->mr_vol64;
       const long long ncell = c->dc.nblocks * kBlockVol;
       ma.rref = c->mrf + 12 * ncell;
       ma.dref = c->mrf + 13 * ncell;
       ma.vtrue = c->mrf + 14 * ncell;
       ma.pin_cell = c->mr_pin_dev;
     }
-    hipLaunchKernelGGL(k_mr_pin, dim3(G), dim3(256), 0, c->stream, ma);
+    HIP_TRY(c, fill_u32(c->stream, c->u32_dev + 5, 0u, 1));
+    hipLaunchKernelGGL(k_mr_pin, dim3(std::min(G, 512u)), dim3(256), 0, c->stream, ma);
     LAUNCH_CHECK(c);
-    TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble, dim3(G), dim3(256), 0, c->stream, ma));
+    if (refmode) {
+      TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble, dim3(G), dim3(256), 0, c->stream, ma));
+    } else {
+      MrCellOut mo;
+      mo.b64 = c->b64; mo.cd64 = c->cd64; mo.cx64 = c->cx64; mo.cy64 = c->cy64; mo.cz64 = c->cz64;
+      mo.vol64 = c->mr_vol64;
+      mo.cd32 = c->cd32; mo.cx32 = c->cx32; mo.cy32 = c->cy32; mo.cz32 = c->cz32; mo.inv32 = c->invd32;
+      TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble_cells, dim3(G), dim3(256), 0, c->stream, ma, mo));
+    }
     LAUNCH_CHECK(c);
   } else {
   hipLaunchKernelGGL(k_pin_detect, dim3(std::min(list_grid(npb), 512u)), dim3(256), 0, c->stream, pa);
@@ -837,18 +850,25 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   va.dc = c->dc; va.list = c->pblk; va.nlist = npb; va.sc = c->sc; va.part = c->partial;
   hipLaunchKernelGGL(k_ir_start, dim3(G), dim3(256), 0, c->stream, va, c->x64, c->invd32, cfg->warm_start);
   LAUNCH_CHECK(c);
-  MrOp mop{};
+  MrRowOp mop{};
+  MrRowOp64 mrow64{};
   MrOp64 mop64{};
   if (mr) {
-    mop.m = mop64.m = mr_grid(c);
-    mop.cd = c->cd32; mop64.cd = c->cd64; mop64.vol = c->mr_vol64;
-    for (int a = 0; a < 3; ++a) { mop.cf[a] = c->mr_cf32[a]; mop64.cf[a] = c->mr_cf64[a]; }
+    mop = mr_row_op(c);
+    mrow64.dc = c->dc; mrow64.info = c->mr_info; mrow64.vol = c->mr_vol64;
+    mrow64.cd = c->cd64; mrow64.cx = c->cx64; mrow64.cy = c->cy64; mrow64.cz = c->cz64;
+    mop64.m = mr_grid(c);
+    mop64.cd = c->cd64; mop64.vol = c->mr_vol64;
+    for (int a = 0; a < 3; ++a) mop64.cf[a] = c->mr_cf64[a];
   }
   const double* r_src = c->r64;  // the FP64 residual the next (re)start loads
   auto residual = [&]() -> int {
-    if (mr)
+    if (mr && refmode)
       TIMED(c, PF_K_RESIDUAL64,
             hipLaunchKernelGGL(k_mr_residual64, dim3(G), dim3(256), 0, c->stream, va, mop64, c->b64, c->x64, c->r64));
+    else if (mr)
+      TIMED(c, PF_K_RESIDUAL64,
+            hipLaunchKernelGGL(k_mr_residual, dim3(G), dim3(256), 0, c->stream, va, mrow64, c->b64, c->x64, c->r64));
     else
     TIMED(c, PF_K_RESIDUAL64,
           hipLaunchKernelGGL(k_residual64, dim3(G), dim3(256), 0, c->stream, va, c->b64, c->x64, c->r64, c->cd64,
@@ -911,10 +931,8 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   // weights (z and partial r.z in slot 2, GT partials)
   bool learned = want_learned || want_mg;
   c->mg_cs_active = c->mg_cs;  // caller-set weights (pf_mg_set_correction_weights) or none
-  if (mr && !refmode) {
-    st = mr_split_lists(c, mop.m);
-    if (st) return st;
-  }
+  if (mr && !refmode && c->u32_host[5])
+    return fail(c, PF_ERR_STATE, "multires leaves above level 2 hold FLUID cells: the fast solves take levels 0 to 2");
   if (learned) {
     st = mr ? mr_mg_build(c, mop) : mg_build(c);
     if (st) return st;
@@ -927,7 +945,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     if (st) return st;
     c->mg_cs_active = c->mg_cs_net;
   }
-  const unsigned GT = learned ? mg_grid0(c) : 1u;
+  const unsigned GT = mr ? cg_grid(npb) : (learned ? mg_grid0(c) : 1u);
   auto papply = [&](const int* done) -> int {
     long long ki = kbegin(c, PF_K_MG_APPLY);
     int s2 = mr ? mr_mg_apply(c, mop, va, c->r32, c->z32, done, c->partial)
@@ -957,17 +975,26 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     // the buffer-addressed kernels take 32-bit byte offsets: arrays below 2 GiB
     const bool spmv_buffers = c->dc.nblocks * kBlockVol * 4 < (1LL << 31);
     CgState cg;
-    const bool one_kernel = !mr && spmv_buffers;   // the Jacobi iteration as k_cg_iter
+    const bool one_kernel = mr || spmv_buffers;   // the Jacobi iteration as k_cg_iter or k_mr_cg_iter
+    const unsigned GL = mr ? cg_grid(npb) : G;    // workgroups of the load, one partial each
+    // r32 from the FP64 residual, x32 = 0 (and p = 0)
+    auto load = [&](const double* src, float* p) {
+      if (mr)
+        hipLaunchKernelGGL(k_mr_load, dim3(GL), dim3(256), 0, c->stream, va, mop, src, c->x32, c->r32, p,
+                           static_cast<float*>(nullptr), static_cast<const float*>(nullptr), 0);
+      else
+        hipLaunchKernelGGL(k_pcg_load, dim3(GL), dim3(256), 0, c->stream, va, src, c->x32, c->r32, c->z32, p,
+                           c->invd32, learned ? 1 : 0);
+    };
     // (re)start: r32 from r64, x32 = 0, p = 0, z = M(r)
     auto start = [&](int budget) -> int {
       if (one_kernel && !learned) return cg_start(c, cg, va, G, r_src, delta * delta, tol2_abs, budget, between);
-      hipLaunchKernelGGL(k_pcg_load, dim3(G), dim3(256), 0, c->stream, va, r_src, c->x32, c->r32, c->z32, c->pA,
-                         c->invd32, learned ? 1 : 0);
+      load(r_src, c->pA);
       LAUNCH_CHECK(c);
       if (learned) {
         int s2 = papply(nullptr);
         if (s2) return s2;
-        hipLaunchKernelGGL(k_pcg_start_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, (int)GT, c->sc,
+        hipLaunchKernelGGL(k_pcg_start_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)GL, (int)GT, c->sc,
                            delta * delta, tol2_abs, budget, between);
       } else {
         hipLaunchKernelGGL(k_pcg_start, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, c->sc, delta * delta,
@@ -982,13 +1009,8 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     if (st) return st;
     // the two iteration kernels use at most 1024 workgroups, so the per-iteration
     // scalar kernels sum few partials
-    // (the multires SpMV waits on dependent loads per block: it takes more workgroups)
-    const unsigned GS = std::min(G, mr ? 4096u : 1024u);
+    const unsigned GS = mr ? cg_grid(npb) : std::min(G, 1024u);
     VecArgs vs = va;
-    // the multires SpMV: blocks of level 0-1 here, level-2 blocks in a second launch
-    VecArgs vs01 = va;
-    vs01.list = c->mr_list01;
-    vs01.nlist = c->mr_n01;
     int iter_before = 0, iter_base = 0;
     double best_rr = rr, prev_rr = rr;
     int no_gain = 0, learned_slow = 0;
@@ -1010,10 +1032,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       for (int q = 0; q < (fused ? 0 : q_next); ++q) {
         if (mr)
           TIMED(c, PF_K_PCG_SPMV,
-                hipLaunchKernelGGL(k_mr_spmv, dim3(GS), dim3(256), 0, c->stream, vs01, mop, c->z32, c->pA, c->pB,
-                                   c->Ap);
-                hipLaunchKernelGGL(k_mr_spmv2, dim3(GS), dim3(256), 0, c->stream, c->mr_list2, c->mr_n2, vs, mop,
-                                   c->z32, c->pA, c->pB, c->Ap));
+                hipLaunchKernelGGL(k_mr_spmv, dim3(GS), dim3(256), 0, c->stream, vs, mop, c->z32, c->pA, c->pB, c->Ap));
         else if (spmv_buffers)
         TIMED(c, PF_K_PCG_SPMV,
               hipLaunchKernelGGL(k_pcg_spmv, dim3(GS), dim3(256), 0, c->stream, vs, c->z32, c->pA, c->pB, c->Ap,
@@ -1024,20 +1043,21 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
                                  c->Ap, c->cd32, c->cx32, c->cy32, c->cz32));
         hipLaunchKernelGGL(k_pcg_alpha, dim3(1), dim3(256), 0, c->stream, c->partial, (int)GS, c->sc);
         if (learned) {
-          TIMED(c, PF_K_PCG_UPDATE,
-                hipLaunchKernelGGL(k_pcg_update_flex, dim3(GS), dim3(256), 0, c->stream, mr ? vs01 : vs, c->x32,
-                                   c->r32, c->z32, c->pA, c->pB, c->Ap);
-                if (mr) hipLaunchKernelGGL(k_mr_update2<true>, dim3(GS), dim3(256), 0, c->stream, c->mr_list2,
-                                           c->mr_n2, vs, c->x32, c->r32, c->z32, c->pA, c->pB, c->Ap, c->invd32));
+          if (mr)
+            TIMED(c, PF_K_PCG_UPDATE,
+                  hipLaunchKernelGGL(k_mr_update, dim3(GS), dim3(256), 0, c->stream, vs, c->mr_info, c->x32, c->r32,
+                                     c->z32, c->pA, c->pB, c->Ap));
+          else
+            TIMED(c, PF_K_PCG_UPDATE,
+                  hipLaunchKernelGGL(k_pcg_update_flex, dim3(GS), dim3(256), 0, c->stream, vs, c->x32, c->r32, c->z32,
+                                     c->pA, c->pB, c->Ap));
           st = papply(done_dev);
           if (st) return st;
           hipLaunchKernelGGL(k_pcg_beta_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)GS, (int)GT, c->sc);
         } else {
           TIMED(c, PF_K_PCG_UPDATE,
-                hipLaunchKernelGGL(k_pcg_update, dim3(GS), dim3(256), 0, c->stream, mr ? vs01 : vs, c->x32, c->r32,
-                                   c->z32, c->pA, c->pB, c->Ap, c->invd32);
-                if (mr) hipLaunchKernelGGL(k_mr_update2<false>, dim3(GS), dim3(256), 0, c->stream, c->mr_list2,
-                                           c->mr_n2, vs, c->x32, c->r32, c->z32, c->pA, c->pB, c->Ap, c->invd32));
+                hipLaunchKernelGGL(k_pcg_update, dim3(GS), dim3(256), 0, c->stream, vs, c->x32, c->r32, c->z32, c->pA,
+                                   c->pB, c->Ap, c->invd32));
           hipLaunchKernelGGL(k_pcg_beta, dim3(1), dim3(256), 0, c->stream, c->partial, (int)GS, c->sc);
         }
       }
@@ -1133,8 +1153,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         }
         continue;
       }
-      hipLaunchKernelGGL(k_pcg_load, dim3(G), dim3(256), 0, c->stream, va, c->r64, c->x32, c->r32, c->z32,
-                         breakdown ? c->pA : nullptr, c->invd32, learned ? 1 : 0);
+      load(c->r64, breakdown ? c->pA : nullptr);
       LAUNCH_CHECK(c);
       if (learned) {
         st = papply(nullptr);
@@ -1142,7 +1161,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       }
       if (breakdown) {
         if (learned)
-          hipLaunchKernelGGL(k_pcg_start_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, (int)GT, c->sc,
+          hipLaunchKernelGGL(k_pcg_start_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)GL, (int)GT, c->sc,
                              delta * delta, tol2_abs, max_iters - total, between);
         else
           hipLaunchKernelGGL(k_pcg_start, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, c->sc, delta * delta,
@@ -1150,7 +1169,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         iter_base = total;
         iter_before = 0;
       } else if (learned) {
-        hipLaunchKernelGGL(k_pcg_resume_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, (int)GT, c->sc);
+        hipLaunchKernelGGL(k_pcg_resume_flex, dim3(1), dim3(256), 0, c->stream, c->partial, (int)GL, (int)GT, c->sc);
       } else {
         hipLaunchKernelGGL(k_pcg_resume, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, c->sc);
       }

@@ -207,8 +207,7 @@ struct Ctx {
   long long mr_leaves_cap = 0;
   uint8_t* mr_lvl = nullptr;        // level byte per fine cell
   uint8_t* mr_valid[3] = {};        // enumerated fine faces
-  float* mr_cf32[3] = {};           // coupling conductance per fine face
-  double* mr_cf64[3] = {};
+  double* mr_cf64[3] = {};          // coupling conductance per fine face (reference-order solve)
   double* mr_vol64 = nullptr;       // leaf-cell volume at FLUID anchors
   double* mr_pfull = nullptr;       // FP64 pressure per fine cell
   int* mr_bbox = nullptr;           // particle cell boxes (device)
@@ -221,11 +220,7 @@ struct Ctx {
   pf_mr_solve_detail mr_detail{};
   double* mrf = nullptr;            // 15 fine FP64 vectors (ncell each)
   double* mrc = nullptr;            // 6 coarse FP64 vectors
-  // the multires cycle's block lists: levels 0-1 (a wave per block) and level 2 (four
-  // blocks per wave), split from the fluid list per solve
-  uint8_t *mr_f01 = nullptr, *mr_f2 = nullptr;
-  uint32_t *mr_list01 = nullptr, *mr_list2 = nullptr;
-  long long mr_n01 = 0, mr_n2 = 0;
+  uint8_t* mr_info = nullptr;       // per block: its level and which neighbours have level 2 (pf_mr_row.hip)
   long long mrc_cap = 0;
   long long* mr_pin_dev = nullptr;  // pinned anchor (block-major index) or -1
   long long* mr_pin_host = nullptr;

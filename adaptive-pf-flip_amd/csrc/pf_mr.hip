@@ -18,9 +18,10 @@
 // over its fine face patches p (multires_pressure3d.cpp:783-812).  Multiplying row a
 // by V_a gives a symmetric conductance Laplacian S x = V rhs with the same solution,
 // so the FP32 inner PCG runs on S (Jacobi on S equals Jacobi on the reference's
-// rows).  The unknown of a leaf cell lives at its anchor (lowest) fine cell; c_p is
-// stored per fine face (cf, zero unless the face couples two FLUID leaf cells, neither
-// pinned) and the Dirichlet part of the diagonal per anchor (cd).  The FP64 residual
+// rows), by cell rows in pf_mr_row.hip.  In the reference-order solve the unknown of a
+// leaf cell lives at its anchor (lowest) fine cell; c_p is stored per fine face (cf, zero
+// unless the face couples two FLUID leaf cells, neither pinned) and the Dirichlet part of
+// the diagonal per anchor (cd).  The FP64 residual
 // reports |rhs - A x|_inf = |(V rhs - S x) / V|_inf for the reference's stop rule.
 #include "pf_internal.h"
 
@@ -129,7 +130,6 @@ struct MrAsm {
   uint32_t* pin;          // [0] touches AIR, [1] pinned cell linear id (all ones: none), [4] FLUID leaf cells
   const float *u, *v, *w, *mu, *mv, *mw;
   double *b64, *cd64, *cf64[3], *vol64;
-  float *cd32, *cf32[3], *invd32;
   double* part;
   uint32_t* order_key;    // FLUID anchors: the reference's leafCells order (for the pin)
   // optional, the reference's own row quantities (for the reference-order solve):
@@ -205,15 +205,18 @@ __global__ void __launch_bounds__(256) k_mr_pin(MrAsm a) {
     int bx, by, bz;
     block_coords(a.m.dc, b, bx, by, bz);
     const int i = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3), k = bz * 4 + (lane >> 4);
-    int L;
+    const int L = mr_level(a.m, bx * 4, by * 4, bz * 4);  // (wave-uniform: a block lies in one leaf)
+    const int mask = (1 << (L < 0 ? 0 : L)) - 1;
     bool air = false;
-    if (i < a.m.g.nx && j < a.m.g.ny && k < a.m.g.nz && mr_is_anchor(a.m, i, j, k, L) &&
-        a.m.marker[b * kBlockVol + lane] == CELL_FLUID) {
-      ++cnt;
-      mn = min(mn, mr_order_key(a.m, i, j, k, L));
-      mr_patches(a.m, i, j, k, 1 << L, [&](int, int, int, int, int ni, int nj, int nk, double) {
-        air = air || (mr_level(a.m, ni, nj, nk) >= 0 && mr_marker(a.m, ni, nj, nk) == CELL_AIR);
-      });
+    // a lane per fine cell: an AIR cell next to a FLUID one lies in another leaf cell
+    if (L >= 0 && i < a.m.g.nx && j < a.m.g.ny && k < a.m.g.nz && a.m.marker[b * kBlockVol + lane] == CELL_FLUID) {
+      if (((i | j | k) & mask) == 0) {
+        ++cnt;
+        mn = min(mn, mr_order_key(a.m, i, j, k, L));
+      }
+      const int nb[6][3] = {{i - 1, j, k}, {i + 1, j, k}, {i, j - 1, k}, {i, j + 1, k}, {i, j, k - 1}, {i, j, k + 1}};
+#pragma unroll
+      for (int q = 0; q < 6; ++q) air = air || mr_marker(a.m, nb[q][0], nb[q][1], nb[q][2]) == CELL_AIR;
     }
     anyair = anyair || __any(air);
   }
@@ -226,16 +229,20 @@ __global__ void __launch_bounds__(256) k_mr_pin(MrAsm a) {
   if (lane == 0) { s_air[w] = anyair; s_min[w] = mn; s_cnt[w] = cnt; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    if (s_air[0] | s_air[1] | s_air[2] | s_air[3]) atomicOr(&a.pin[0], 1u);
+    // (the flag and the minimum settle early: look before the atomic)
+    if ((s_air[0] | s_air[1] | s_air[2] | s_air[3]) &&
+        !__hip_atomic_load(&a.pin[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicOr(&a.pin[0], 1u);
     const uint32_t m4 = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
-    if (m4 != 0xffffffffu) atomicMin(&a.pin[1], m4);
+    if (m4 < __hip_atomic_load(&a.pin[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&a.pin[1], m4);
     const uint32_t c4 = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     if (c4) atomicAdd(&a.pin[4], c4);
   }
 }
 
 // rows (multires_pressure3d.cpp:783-812) scaled by the cell volume: cd (Dirichlet
-// diagonal), cf per fine face (coupling), 1/diag, V rhs; FP64 and FP32 copies
+// diagonal), cf per fine face (coupling), V rhs, in the reference's patch order: for the
+// reference-order solve (the fast ones use k_mr_assemble_cells)
 __global__ void __launch_bounds__(256) k_mr_assemble(MrAsm a) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
@@ -278,7 +285,7 @@ __global__ void __launch_bounds__(256) k_mr_assemble(MrAsm a) {
         }
         if (!coupled) cd += cond;
         // a coupling face is written by both of its cells with the same value
-        if (coupled) { a.cf64[axis][fi] = cond; a.cf32[axis][fi] = (float)cond; }
+        if (coupled) a.cf64[axis][fi] = cond;
         div += sign * (double)mr_face_vel(a, axis, fi) * area / V;
       });
       rhs = pinned ? 0.0 : -div + a.cdiv;
@@ -291,8 +298,6 @@ __global__ void __launch_bounds__(256) k_mr_assemble(MrAsm a) {
     a.b64[c] = V * rhs;
     a.vol64[c] = anchor ? V : 0.0;
     a.cd64[c] = cd;
-    a.cd32[c] = (float)cd;
-    a.invd32[c] = diag > 0.0 ? (float)(1.0 / diag) : 0.f;
     bb += V * rhs * V * rhs;
   }
   double v[1] = {bb};
@@ -300,10 +305,6 @@ __global__ void __launch_bounds__(256) k_mr_assemble(MrAsm a) {
   block_reduce_store<1>(v, mx, a.part, kMaxPartials);
 }
 
-struct MrOp {
-  MrGrid m;
-  const float *cd, *cf[3];
-};
 struct MrOp64 {
   MrGrid m;
   const double *cd, *cf[3], *vol;
@@ -387,49 +388,6 @@ __device__ inline T mr_apply_row_coop(const MrGrid& m, const T* const* cf, int i
     acc += __shfl_xor(acc, 16 << bit, 64);
   }
   return acc;
-}
-
-// multires twin of k_pcg_spmv: p_new = z + beta p_old (recomputed at the neighbour
-// anchors), Ap = S p_new, partial p.Ap
-__global__ void __launch_bounds__(256) k_mr_spmv(VecArgs a, MrOp op, const float* __restrict__ z, float* __restrict__ pA,
-                                                 float* __restrict__ pB, float* __restrict__ Ap) {
-  if (a.sc->done) return;
-  const int lane = threadIdx.x & 63;
-  const bool odd = a.sc->iter & 1;
-  const float* __restrict__ pold = odd ? pB : pA;
-  float* __restrict__ pnew = odd ? pA : pB;
-  const float beta = (float)a.sc->beta;
-  double pap = 0.0;
-  FOR_LIST_BLOCKS(a, b, lane) {
-    const long long c = b * kBlockVol + lane;
-    const float pc = fmaf(beta, pold[c], z[c]);
-    float ap = 0.f;
-    {
-      // every anchor: a non-FLUID one has no couplings and cd = 0, so Ap = 0 there
-      int bx, by, bz;
-      block_coords(op.m.dc, b, bx, by, bz);
-      const int i = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3), k = bz * 4 + (lane >> 4);
-      const bool in = i < op.m.g.nx && j < op.m.g.ny && k < op.m.g.nz;
-      auto pval = [&](long long n) { return fmaf(beta, pold[n], z[n]); };
-      const int Lb = mr_level(op.m, bx * 4, by * 4, bz * 4);
-      if (Lb >= 0 && Lb <= 2) {
-        const int s = 1 << Lb;
-        const long long anc = bm_index(op.m.dc, i & ~(s - 1), j & ~(s - 1), k & ~(s - 1));
-        const float sum = mr_apply_row_coop<float>(op.m, op.cf, i, j, k, Lb, in, in ? pval(anc) : 0.f, pval);
-        if (in && ((i | j | k) & (s - 1)) == 0) ap = op.cd[c] * pc + sum;
-      } else {
-        int L;
-        if (in && mr_is_anchor(op.m, i, j, k, L))
-          ap = op.cd[c] * pc + mr_apply_row<float>(op.m, op.cf, i, j, k, 1 << L, pc, pval);
-      }
-    }
-    pnew[c] = pc;
-    Ap[c] = ap;
-    pap += (double)pc * (double)ap;
-  }
-  double v[1] = {pap};
-  const bool mx[1] = {false};
-  block_reduce_store<1>(v, mx, a.part, kMaxPartials);
 }
 
 // FP64 residual r = V rhs - S x; partial sums of r^2, max |r / V| (the reference's

@@ -1,0 +1,93 @@
+"""The multires operator by cell rows (pf_mr_row.hip) where its layout can go wrong: leaf
+cells clipped by a ragged domain, blocks of every level next to every other, a refined box
+at a corner, one refined block, no refinement at all.
+
+Bars: both fast solves (Jacobi PCG and multigrid), to a max residual of 1e-11, against the
+exact FP64 solution of the oracle's rows: those of the three-level tests, pressure within
+1e-6 and faces within 1e-5 norm-wise relative.
+"""
+import numpy as np
+import pytest
+
+import pfflip_amd as G
+import pyoracle as O
+from _helpers import rel_err
+from test_multires3_oracle import _system, exact_solution
+
+pytestmark = pytest.mark.gpu
+
+
+def _phase():
+    ph = O.Phase(1.0, 0.01, 1.0, 1.0)
+    ph.rho_tilde_0 = O.calibrate_rho_tilde0(ph, 1.0)
+    return ph, G.Phase(ph.rho_l, ph.rho_g, ph.alpha_phi, ph.rho_tilde_0)
+
+
+def _particles(dims, seed=4):
+    """8 jittered particles per cell below 0.6 of the height, a gas ball in them"""
+    nx, ny, nz = dims
+    k, j, i = np.meshgrid(np.arange(1, nz - 1), np.arange(1, max(2, int(0.6 * ny))), np.arange(1, nx - 1), indexing="ij")
+    c = np.repeat(np.stack([i.ravel(), j.ravel(), k.ravel()], 1), 8, axis=0)
+    r = np.random.default_rng(seed)
+    p = (c + r.uniform(0.01, 0.99, c.shape)).astype(np.float32)
+    v = r.normal(scale=0.3, size=p.shape).astype(np.float32)
+    t = (((p - np.array([nx / 2, ny * 0.25, nz / 2])) ** 2).sum(1) < (0.15 * nx) ** 2).astype(np.uint8)
+    return tuple(np.ascontiguousarray(q) for q in (*p.T, *v.T)) + (t,)
+
+
+def _to_projection(ctx, gph, dt):
+    ctx.mr_mark_cells()
+    ctx.mr_p2g(gph, 1.0)
+    ctx.apply_gravity(dt, -9.81)
+    ctx.apply_walls()
+
+
+@pytest.mark.parametrize("dims,level,boxes", [
+    ((17, 10, 9), 1, ([4, 3, 2, 13, 9, 8],)), ((24, 20, 28), 1, ([0, 0, 0, 9, 9, 9],)),
+    ((21, 19, 30), 1, ([8, 4, 8, 12, 8, 12],)), ((33, 18, 20), 1, ()), ((26, 25, 23), 1, ([0, 9, 0, 26, 20, 23],)),
+    ((40, 36, 24), 2, ([0, 14, 0, 40, 24, 24], [16, 0, 8, 24, 12, 16])),
+    ((37, 30, 33), 2, ([10, 12, 10, 20, 30, 20],) * 2)])
+def test_fast_solves_match_the_exact_solution(dims, level, boxes):
+    print(f"[mr rows] {dims} {level} {boxes}", flush=True)
+    dt = 0.02
+    ph, gph = _phase()
+    leaves = G.mr_layout_fine_box(*dims, level=level)
+    for b in boxes:
+        leaves = G.mr_layout_refine(*dims, leaves, b)
+    parts = _particles(dims)
+    ctx = G.MRContext(*dims, 1.0)
+    ctx.set_layout(leaves)
+    ctx.upload(*parts)
+    g = O.MRGrid(*dims, 1.0, faithful=False)
+    g.set_leaves(leaves)
+    ps = O.Particles(*parts[:6], type=parts[6])
+    g.mark_cells(ps)
+    g.p2g(ps, ph, 1.0)
+    g.apply_gravity(dt, -9.81)
+    g.apply_walls()
+    cells, A, rhs, pin, vol = _system(g, ph, dt)
+    g.apply_pressure(ph, dt, exact_solution(A, rhs, vol))
+    for mode in (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID):
+        _to_projection(ctx, gph, dt)
+        st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-11, 0.0, mode=mode))
+        assert st.converged == 1 and st.true_max_residual < 1e-11 and st.fallback_used == 0
+        assert st.fluid_cells == len(cells) and st.pinned_cell == pin
+        assert rel_err(ctx.field(G.FIELD_P), g.dense(O.P)) < 1e-6
+        for f in range(3):
+            assert rel_err(ctx.field(f), g.dense(f)) < 1e-5, f
+
+
+def test_fluid_above_level_2_is_refused_and_the_context_stays_usable():
+    dims, dt = (64, 64, 64), 0.02
+    _, gph = _phase()
+    ctx = G.MRContext(*dims, 1.0)
+    ctx.set_layout(G.mr_layout_fine_box(*dims, level=3))
+    ctx.upload(*_particles(dims))
+    for mode in (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID):
+        _to_projection(ctx, gph, dt)
+        with pytest.raises(G.PfError):
+            ctx.mr_project(gph, dt, G.mr_solve_cfg(2000, 1e-9, 0.0, mode=mode))
+    ctx.set_layout(G.mr_layout_fine_box(*dims, level=2))
+    _to_projection(ctx, gph, dt)
+    st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-9, 0.0))
+    assert st.converged == 1 and np.isfinite(ctx.field(G.FIELD_P)).all()
