@@ -144,17 +144,19 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   for (int col = 0; col < 8; ++col) {
     a.list = c->color_list + (long long)col * c->color_cap;
     a.count = c->color_cnt + col;
-    const dim3 grid((unsigned)std::max<long long>(c->color_cap, 1));
+    // (the list's length is on the device: offer the split by axes where it may be short)
+    const dim3 grid((unsigned)std::max<long long>(c->color_cap, 1), c->color_cap <= 8 * kSplitBlocks ? 3 : 1);
     const P2GShared sh = p2g_shared_args(a);
     const P2GField f0 = p2g_field_args(a, 0), f1 = p2g_field_args(a, 1), f2 = p2g_field_args(a, 2);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(64), 0, c->stream, sh, f0, f1, f2); };
+    const long long ki = kbegin(c, PF_K_P2G);
     if (mr)
-      TIMED(c, PF_K_P2G, hipLaunchKernelGGL((k_p2g_color<2, false>), grid, dim3(64), 0, c->stream, sh, f0, f1, f2));
+      a.fast32 ? launch(k_p2g_color<2, true>) : launch(k_p2g_color<2, false>);
     else if (single)
-      TIMED(c, PF_K_P2G, hipLaunchKernelGGL((k_p2g_color<1, false>), grid, dim3(64), 0, c->stream, sh, f0, f1, f2));
-    else if (a.fast32)
-      TIMED(c, PF_K_P2G, hipLaunchKernelGGL((k_p2g_color<0, true>), grid, dim3(64), 0, c->stream, sh, f0, f1, f2));
+      a.fast32 ? launch(k_p2g_color<1, true>) : launch(k_p2g_color<1, false>);
     else
-      TIMED(c, PF_K_P2G, hipLaunchKernelGGL((k_p2g_color<0, false>), grid, dim3(64), 0, c->stream, sh, f0, f1, f2));
+      a.fast32 ? launch(k_p2g_color<0, true>) : launch(k_p2g_color<0, false>);
+    kend(c, ki);
     LAUNCH_CHECK(c);
   }
   return PF_OK;

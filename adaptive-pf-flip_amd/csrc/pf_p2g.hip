@@ -152,30 +152,53 @@ __device__ inline float exact_weight(double ddx, double ddy, double ddz, bool& a
 // activates its block, zero weights included.  For a particle in cell c the nodes
 // lie in c..c+1 along the face axis and c-1..c+1 across it, inside the cubic
 // kernel's register window, so both kernels share the region and flush logic.
+//
+// The window's weights along one axis: nodes c, c+1 (entries 1, 2) on the face axis, two
+// of the three entries across it, so 18 nodes can take weight and every index is a
+// constant (with the eight nodes indexed by their offset the sums went through scratch:
+// 94 us a launch on 2.7 million particles).  lo: the first entry with a node.
+template <bool FACE>
+__device__ inline void trilinear_axis(double g, int c, double (&w)[3], int& lo) {
+  const double f0 = floor(g), f = g - f0;
+  if (FACE) {  // (floor(g) is the particle's cell)
+    w[0] = 1.0 - f;
+    w[1] = f;
+    w[2] = 0.0;
+    lo = 1;
+  } else {
+    lo = (int)f0 - c + 1;
+    w[0] = lo == 0 ? 1.0 - f : 0.0;
+    w[1] = lo == 0 ? f : 1.0 - f;
+    w[2] = lo == 0 ? 0.0 : f;
+  }
+}
+
+// one particle's 18 weights into the lane's node sums, and its stencil's activation bits
 template <int AX>
-__device__ inline void trilinear_weights(double gx, double gy, double gz, int i, int j, int k,
-                                         const bool* vx, const bool* vy, const bool* vz, float* wt,
-                                         uint64_t& fbits) {
+__device__ inline void trilinear_add(double gx, double gy, double gz, int i, int j, int k, float vel, float* am,
+                                     float* aq, uint64_t& fbits) {
   using A = Ax<AX>;
-  const int i0 = (int)floor(gx), j0 = (int)floor(gy), k0 = (int)floor(gz);
-  const double fx = gx - i0, fy = gy - j0, fz = gz - k0;
-  const double wx[2] = {1.0 - fx, fx}, wy[2] = {1.0 - fy, fy}, wz[2] = {1.0 - fz, fz};
+  double wx[3], wy[3], wz[3];
+  int ox0, oy0, oz0;
+  trilinear_axis<AX == 0>(gx, i, wx, ox0);
+  trilinear_axis<AX == 1>(gy, j, wy, oy0);
+  trilinear_axis<AX == 2>(gz, k, wz, oz0);
+  // (entry e of an axis is window offset e, or e + 1 on the face axis)
 #pragma unroll
-  for (int n = 0; n < A::NN; ++n) wt[n] = 0.f;
+  for (int ez = 0; ez < (AX == 2 ? 2 : 3); ++ez)
 #pragma unroll
-  for (int dk = 0; dk < 2; ++dk)
+    for (int ey = 0; ey < (AX == 1 ? 2 : 3); ++ey)
 #pragma unroll
-    for (int dj = 0; dj < 2; ++dj)
-#pragma unroll
-      for (int di = 0; di < 2; ++di) {
-        // window offsets (node - cell + 1); node indices of the window are in range
-        const int ox = i0 + di - i + 1, oy = j0 + dj - j + 1, oz = k0 + dk - k + 1;
-        if (ox < 0 || ox >= A::NX || oy < 0 || oy >= A::NY || oz < 0 || oz >= A::NZ) continue;
-        if (!(vx[ox] && vy[oy] && vz[oz])) continue;
-        const int n = ox + A::NX * (oy + A::NY * oz);
-        wt[n] = (float)(__dmul_rn(__dmul_rn(wx[di], wy[dj]), wz[dk]));
-        fbits |= (1ull << n);
+      for (int ex = 0; ex < (AX == 0 ? 2 : 3); ++ex) {
+        const int n = (ex + (AX == 0)) + A::NX * ((ey + (AX == 1)) + A::NY * (ez + (AX == 2)));
+        const float w = (float)__dmul_rn(__dmul_rn(wx[ex], wy[ey]), wz[ez]);
+        // mass += (float)(w * 1.0) = w; momentum += (float)(w * v), v exact in FP64: the
+        // product of two FP32 values is exact there, so this is the FP32 product
+        am[n] += w;
+        aq[n] = __fadd_rn(aq[n], __fmul_rn(w, vel));
       }
+  constexpr uint64_t row = 3ull, two = row | (row << A::NX), cube = two | (two << (A::NX * A::NY));
+  fbits |= cube << (ox0 + A::NX * (oy0 + A::NY * oz0));
 }
 
 // One particle's weights by the per-node path: the FP32 d^2 with the FP64 predicate and
@@ -217,7 +240,7 @@ __device__ inline float node_weights(const float* dx2, const float* dy2, const f
 // A lane splats its cell's particles (in ascending caller index) into its 36 node sums
 // of one face axis, then adds them into the block's LDS region.
 //
-// KT = 0 runs two loops.  The first covers cells of at most kFastMax particles in
+// Two loops.  The first covers cells of at most kFastMax particles in
 // caller-index order, with the next particle's data loaded while this one
 // computes, and evaluates the cubic in the separable FP32 form
 // t = (1 - (dx^2 + dy^2)/2.25) - dz^2/2.25, w = max(t, 0)^3 -- one subtraction per
@@ -227,8 +250,9 @@ __device__ inline float node_weights(const float* dx2, const float* dy2, const f
 // particle of a fuller cell (in memory order up to kSortedMax particles, else selected
 // by ascending caller index) through node_weights.
 // Keeping the rare paths out of the first loop keeps its registers to what it needs.
-// KT = 2 (multires, enumerated faces only) and KT = 1 (trilinear) use the second loop
-// for every particle.
+// KT = 2 (multires) masks the weights of faces that are not enumerated in both loops; KT =
+// 1 (trilinear) marks nothing.  (Both took the second loop for every particle before: 1.32
+// ms a launch on 14 million particles of three levels.)
 //
 // F32: origin 0, a power-of-two dx and fewer than 2^22 cells a side, where x/dx is
 // exact in FP32 and each offset from the lane's cell is either exact or one correctly
@@ -265,6 +289,18 @@ __device__ inline void splat_axis(const P2GShared& a, const P2GField& f, int i, 
 #pragma unroll
   for (int o = 0; o < A::NZ; ++o) penz[o] = vz[o] ? 0.f : kOutside;
   const float* vp = f.vel;
+  // multires: only the enumerated faces take (and normalise) weights
+  // (collectWeightedFaces, multires_ops3d_tp.cpp:62-75); s_flag holds the region's (bit 1)
+  uint64_t vbits = ~0ull;
+  if (KT == 2) {
+    vbits = 0;
+#pragma unroll
+    for (int n = 0; n < A::NN; ++n) {
+      const int ox = n % A::NX, oy = (n / A::NX) % A::NY, oz = n / (A::NX * A::NY);
+      vbits |= (uint64_t)(s_flag[lx + ox + A::RX * (ly + oy + A::RY * (lz + oz))] >> 1) << n;
+    }
+  }
+  const uint32_t vlo = (uint32_t)vbits, vhi = (uint32_t)(vbits >> 32);
 
   // offsets of a particle from the lane's cell along this axis' face grid
   // (sparse_ops3d_tp.cpp:117-122), and the FP64 stencil coordinates when asked
@@ -315,7 +351,7 @@ __device__ inline void splat_axis(const P2GShared& a, const P2GField& f, int i, 
   const bool masked = cnt <= kFastMax;  // ranked or sorted
   auto slot = [&](uint32_t r) -> uint32_t { return ranked ? (uint32_t)ord[r] : r; };
   uint64_t marked = 0;  // ranks (bit it) left to the second loop
-  if (KT == 0 && masked && cnt > 0) {
+  if (masked && cnt > 0) {
     // the particle of rank r (its data for the next iteration load while this one
     // computes)
     auto fetch = [&](uint32_t r, float& px, float& py, float& pz, float& vel, uint8_t& ty, float& pvol) {
@@ -330,6 +366,12 @@ __device__ inline void splat_axis(const P2GShared& a, const P2GField& f, int i, 
       const float px = nx_, py = ny_, pz = nz_, vel = nv_, pvol = nvol_;
       const uint8_t ty = nty_;
       if (it + 1 < cnt) fetch(it + 1, nx_, ny_, nz_, nv_, nty_, nvol_);
+      if (KT == 1) {
+        double gx, gy, gz;
+        coords64(px, py, pz, gx, gy, gz);
+        trilinear_add<AX>(gx, gy, gz, i, j, k, vel, am, aq, fbits);
+        continue;
+      }
       float fx, fy, fz;
       offsets(px, py, pz, fx, fy, fz);
       float dx2[A::NX], dy2[A::NY], dz2[A::NZ];
@@ -360,7 +402,11 @@ __device__ inline void splat_axis(const P2GShared& a, const P2GField& f, int i, 
             tmin = fminf(tmin, fabsf(t));
             // max(t, 0) as one median (t <= 1 here); fmaxf would first quiet a NaN t
             const float tp = __builtin_amdgcn_fmed3f(t, 0.f, 1.f);
-            const float w = tp * tp * tp;
+            float w = tp * tp * tp;
+            // (multires: no weight on a face that is not enumerated)
+            if (KT == 2)
+              w = __uint_as_float(__float_as_uint(w) &
+                                  (uint32_t)__builtin_amdgcn_sbfe((int)(n < 32 ? vlo : vhi), n & 31, 1));
             wt[n] = w;
             wsum += w;
           }
@@ -373,26 +419,10 @@ __device__ inline void splat_axis(const P2GShared& a, const P2GField& f, int i, 
       }
       accumulate(wt, wsum, mp, vel);
     }
-  } else if (masked && cnt > 0) {
-    marked = (cnt >= 64u) ? ~0ull : ((1ull << cnt) - 1ull);
   }
 
   // the second loop: marked particles in rank order, then every particle of a cell of
   // more than kFastMax particles, in memory order or by selection
-  uint64_t vbits = ~0ull;
-  if (KT == 2) {
-    // multires: only the enumerated faces take (and normalise) weights
-    // (collectWeightedFaces, multires_ops3d_tp.cpp:62-75)
-    vbits = 0;
-#pragma unroll
-    for (int oz = 0; oz < A::NZ; ++oz)
-#pragma unroll
-      for (int oy = 0; oy < A::NY; ++oy)
-#pragma unroll
-        for (int ox = 0; ox < A::NX; ++ox)
-          if (vx[ox] && vy[oy] && vz[oz] && f.valid[bm_index(fd, i + ox - 1, j + oy - 1, k + oz - 1)])
-            vbits |= 1ull << (ox + A::NX * (oy + A::NY * oz));
-  }
   const uint32_t nsecond = masked ? (uint32_t)__popcll(marked) : cnt;
   uint32_t last = 0;
   bool first = true;
@@ -419,17 +449,11 @@ __device__ inline void splat_axis(const P2GShared& a, const P2GField& f, int i, 
     const uint8_t ty = a.type[q];
     double gx, gy, gz;
     coords64(px, py, pz, gx, gy, gz);
-    float wt[A::NN];
     if (KT == 1) {
-      trilinear_weights<AX>(gx, gy, gz, i, j, k, vx, vy, vz, wt, fbits);
-      // mass += (float)(w * 1.0) = w; momentum += (float)(w * v) with v exact in FP64
-#pragma unroll
-      for (int n = 0; n < A::NN; ++n) {
-        am[n] += wt[n];
-        aq[n] += (float)((double)wt[n] * (double)vel);
-      }
+      trilinear_add<AX>(gx, gy, gz, i, j, k, vel, am, aq, fbits);
       continue;
     }
+    float wt[A::NN];
     float fx, fy, fz;
     offsets(px, py, pz, fx, fy, fz);
     float dx2[A::NX], dy2[A::NY], dz2[A::NZ];
@@ -497,7 +521,7 @@ __device__ inline void flush_axis(const P2GField& f, int bx, int by, int bz, flo
   for (int e = 0; e < kPer; ++e) {
     const int r = lane + 64 * e;
     if (r >= A::RN) continue;
-    if (s_flag[r]) {
+    if (s_flag[r] & 1) {
       const int rx = r % A::RX, ry = (r / A::RX) % A::RY, rz = r / (A::RX * A::RY);
       const int ni = bx * 4 - 1 + rx, nj = by * 4 - 1 + ry, nk = bz * 4 - 1 + rz;
       if (ni >= 0 && nj >= 0 && nk >= 0 && ni < fd.nx && nj < fd.ny && nk < fd.nz) {
@@ -515,17 +539,56 @@ __device__ inline void flush_axis(const P2GField& f, int bx, int by, int bz, flo
   }
 }
 
+// KT = 2: the enumerated faces of the block's region as bit 1 of its flags
+template <int AX>
+__device__ inline void load_valid(const P2GField& f, int bx, int by, int bz, uint8_t* s_flag, int lane) {
+  using A = Ax<AX>;
+  const Dims& fd = f.df;
+#pragma unroll
+  for (int e = 0; e < (A::RN + 63) / 64; ++e) {
+    const int r = lane + 64 * e;
+    if (r >= A::RN) continue;
+    const int rx = r % A::RX, ry = (r / A::RX) % A::RY, rz = r / (A::RX * A::RY);
+    const int ni = bx * 4 - 1 + rx, nj = by * 4 - 1 + ry, nk = bz * 4 - 1 + rz;
+    const bool in = ni >= 0 && nj >= 0 && nk >= 0 && ni < fd.nx && nj < fd.ny && nk < fd.nz;
+    s_flag[r] = in && f.valid[bm_index(fd, ni, nj, nk)] ? 2 : 0;
+  }
+}
+
+// one face axis of the block
+template <int AX, int KT, bool F32>
+__device__ inline void p2g_axis(const P2GShared& a, const P2GField& f, int bx, int by, int bz, uint32_t s0, uint32_t cnt,
+                                const uint8_t* ord, float2* s_node, uint8_t* s_flag, int lane) {
+  const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
+  if (KT == 2) {
+    load_valid<AX>(f, bx, by, bz, s_flag, lane);
+    __syncthreads();
+  }
+  splat_axis<AX, KT, F32>(a, f, bx * 4 + lx, by * 4 + ly, bz * 4 + lz, s0, cnt, ord, s_node, s_flag, lx, ly, lz);
+  __syncthreads();
+  flush_axis<AX>(f, bx, by, bz, s_node, s_flag, lane);
+  __syncthreads();
+}
+
 // KT = 0: normalized cubic (two-phase); KT = 1: trilinear, unit mass (single-phase);
 // KT = 2: normalized cubic over the enumerated multires faces.  One launch per colour:
 // a block's particles are ranked once and splatted into the three face fields in turn
-// through one LDS node region (12.3 KB of LDS per workgroup with the id ranking).
+// through one LDS node region (12.3 KB of LDS per workgroup with the id ranking).  With
+// few blocks of a colour (kSplitBlocks) each axis takes a workgroup of its own: the chip
+// is not full then and the launch lasts as long as one workgroup.
+constexpr uint32_t kSplitBlocks = 2048;
 template <int KT, bool F32>
 __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
   __shared__ uint32_t s_ids[kOrdMax * 64];
   __shared__ uint8_t s_ord[64 * kOrdMax];
   __shared__ float2 s_node[256];  // the region's (momentum, mass) sums per node
   __shared__ uint8_t s_flag[256];
-  if (blockIdx.x >= *a.count) return;
+  const uint32_t nblk = *a.count;
+  if (blockIdx.x >= nblk) return;
+  // (three workgroups to a block where the launch has them and the colour is short)
+  const bool split = gridDim.y == 3 && nblk <= kSplitBlocks;
+  if (!split && blockIdx.y > 0) return;
+  const int only = split ? (int)blockIdx.y : -1;
   const uint32_t b = a.list[blockIdx.x];
   const int lane = threadIdx.x;
   for (int t = lane; t < 256; t += 64) {
@@ -534,8 +597,6 @@ __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GF
   }
   int bx, by, bz;
   block_coords(a.dc, b, bx, by, bz);
-  const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
-  const int i = bx * 4 + lx, j = by * 4 + ly, k = bz * 4 + lz;
   const long long c = (long long)b * kBlockVol + lane;
   const uint32_t s0 = a.start[c];
   const uint32_t cnt = a.start[c + 1] - s0;
@@ -557,17 +618,9 @@ __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GF
     ord[0] = 0;
   }
   __syncthreads();
-  splat_axis<0, KT, F32>(a, fu, i, j, k, s0, cnt, ord, s_node, s_flag, lx, ly, lz);
-  __syncthreads();
-  flush_axis<0>(fu, bx, by, bz, s_node, s_flag, lane);
-  __syncthreads();
-  splat_axis<1, KT, F32>(a, fv, i, j, k, s0, cnt, ord, s_node, s_flag, lx, ly, lz);
-  __syncthreads();
-  flush_axis<1>(fv, bx, by, bz, s_node, s_flag, lane);
-  __syncthreads();
-  splat_axis<2, KT, F32>(a, fw, i, j, k, s0, cnt, ord, s_node, s_flag, lx, ly, lz);
-  __syncthreads();
-  flush_axis<2>(fw, bx, by, bz, s_node, s_flag, lane);
+  if (only <= 0) p2g_axis<0, KT, F32>(a, fu, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
+  if (only < 0 || only == 1) p2g_axis<1, KT, F32>(a, fv, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
+  if (only < 0 || only == 2) p2g_axis<2, KT, F32>(a, fw, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
 }
 
 }  // namespace pf
