@@ -573,10 +573,19 @@ __device__ inline void p2g_axis(const P2GShared& a, const P2GField& f, int bx, i
 // KT = 0: normalized cubic (two-phase); KT = 1: trilinear, unit mass (single-phase);
 // KT = 2: normalized cubic over the enumerated multires faces.  One launch per colour:
 // a block's particles are ranked once and splatted into the three face fields in turn
-// through one LDS node region (12.3 KB of LDS per workgroup with the id ranking).  With
-// few blocks of a colour (kSplitBlocks) each axis takes a workgroup of its own: the chip
-// is not full then and the launch lasts as long as one workgroup.
-constexpr uint32_t kSplitBlocks = 2048;
+// through one LDS node region (12.3 KB of LDS per workgroup with the id ranking).
+//
+// Or each axis takes a workgroup of its own, where that ends the launch sooner.  12
+// workgroups fit a CU (registers and LDS alike), so n blocks take ceil(n / 3072) rounds of
+// the chip, or ceil(3 n / 3072) rounds a third as long plus a tenth for ranking three
+// times: 64^3 (512 blocks a colour) 53 -> 31 us a launch, 144 x 101 x 131 (3600) 134 ->
+// 120; not at 128^3 x 0.6 (2400), 85 -> 91.
+constexpr uint32_t kP2GResident = 256 * 12;
+constexpr uint32_t kP2GSplitMost = 5 * kP2GResident;  // (past five rounds the last one matters little)
+__device__ inline bool p2g_split(uint32_t n) {
+  const uint32_t whole = (n + kP2GResident - 1) / kP2GResident, third = (3 * n + kP2GResident - 1) / kP2GResident;
+  return n <= kP2GSplitMost && 11 * third < 30 * whole;
+}
 template <int KT, bool F32>
 __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
   __shared__ uint32_t s_ids[kOrdMax * 64];
@@ -585,8 +594,7 @@ __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GF
   __shared__ uint8_t s_flag[256];
   const uint32_t nblk = *a.count;
   if (blockIdx.x >= nblk) return;
-  // (three workgroups to a block where the launch has them and the colour is short)
-  const bool split = gridDim.y == 3 && nblk <= kSplitBlocks;
+  const bool split = gridDim.y == 3 && p2g_split(nblk);
   if (!split && blockIdx.y > 0) return;
   const int only = split ? (int)blockIdx.y : -1;
   const uint32_t b = a.list[blockIdx.x];
