@@ -15,7 +15,10 @@
 // So before a G2P each face axis is packed into quads (vel, vel+x, saved, saved+x) of a
 // face and its +x neighbour: the two x-taps of a (j, k) pair are one 16-byte gather for
 // both fields and one 8-byte gather for vel alone, 24 gathers per particle instead of
-// 72, with the same values, weights and order of operations (the same bits).
+// 72, with the same values, weights and order of operations (the same bits).  Advection
+// alone packs pairs (vel, vel+x): 24 gathers instead of 48.
+#include <type_traits>
+
 #include "pf_internal.h"
 #include "pf_speed.h"
 
@@ -24,9 +27,7 @@ namespace pf {
 struct G2PArgs {
   Geom g;
   Dims df[3];
-  const float* vel[3];    // post-projection u, v, w
-  const float* saved[3];  // pre-gravity u, v, w
-  const float4* quad[3];  // per face (vel, vel+x, saved, saved+x): it and its +x neighbour
+  const void* field[3];   // per face float4 (vel, vel+x, saved, saved+x), float2 (vel, vel+x) or float vel
   PBuf P;
   long long n;
   float inv_dx, ox, oy, oz;
@@ -38,43 +39,24 @@ struct G2PArgs {
   uint32_t* vmax_bits;    // max |v| (float bits) after the update
 };
 
-// trilinear sample with per-tap index clamp, sparse_ops3d_common.h:30-51.  The
-// block-major offset is separable, bm_index(i, j, k) = X(i) + Y(j) + Z(k), so the 8
-// taps take 6 clamped terms instead of 8 full index computations.
-__device__ inline float sample(const float* __restrict__ f, const Dims& d, float gx, float gy, float gz) {
-  float fi = floorf(gx), fj = floorf(gy), fk = floorf(gz);
-  int i0 = (int)fi, j0 = (int)fj, k0 = (int)fk;
-  float fx = gx - fi, fy = gy - fj, fz = gz - fk;
-  float wx[2] = {1.f - fx, fx}, wy[2] = {1.f - fy, fy}, wz[2] = {1.f - fz, fz};
-  const long long sy = (long long)d.nbx * kBlockVol, sz = sy * d.nby;
-  long long X[2], Y[2], Z[2];
-#pragma unroll
-  for (int e = 0; e < 2; ++e) {
-    const int i = min(max(i0 + e, 0), d.nx - 1);
-    const int j = min(max(j0 + e, 0), d.ny - 1);
-    const int k = min(max(k0 + e, 0), d.nz - 1);
-    X[e] = (long long)(i >> 2) * kBlockVol + (i & 3);
-    Y[e] = (long long)(j >> 2) * sy + 4 * (j & 3);
-    Z[e] = (long long)(k >> 2) * sz + 16 * (k & 3);
-  }
-  float s = 0.f;
-#pragma unroll
-  for (int dk = 0; dk < 2; ++dk)
-#pragma unroll
-    for (int dj = 0; dj < 2; ++dj)
-#pragma unroll
-      for (int di = 0; di < 2; ++di) s = fmaf(wx[di] * wy[dj] * wz[dk], f[X[di] + Y[dj] + Z[dk]], s);
-  return s;
+// The trilinear sample with per-tap index clamp (sparse_ops3d_common.h:30-51) from a packed
+// field: Q[q] = (vel[q], vel[q+], saved[q], saved[q+]) or (vel[q], vel[q+]), q+ the face
+// one step along x (q itself at the last x), so one gather of 16 or 8 bytes serves the two
+// x-taps of a (j, k) pair.  The block-major offset is separable, bm_index(i, j, k) = X(i) +
+// Y(j) + Z(k).  For i0 >= nx - 1 the partner is the face itself (as packed); for i0 < 0
+// both taps are face 0, taken from the entry's first half.  Same weights and order of
+// operations as the tap-by-tap sum.  WS (quads): also the saved field's sample.
+// (A plain field, Q = float, takes the two taps one by one.)
+__device__ inline float4 x_taps(const float4* __restrict__ f, long long at, long long) { return f[at]; }
+__device__ inline float4 x_taps(const float2* __restrict__ f, long long at, long long) {
+  const float2 q = f[at];
+  return make_float4(q.x, q.y, 0.f, 0.f);
 }
-
-// The same trilinear sample from a quad field Q[q] = (vel[q], vel[q+], saved[q], saved[q+]),
-// q+ the face one step along x (q itself at the last x): one 16-byte gather serves the
-// two x-taps of a (j, k) pair for both fields, one 8-byte gather for vel alone.  The per-tap clamps are the sample's:
-// for i0 >= nx - 1 the partner is the face itself (as packed); for i0 < 0 both taps are
-// face 0, taken from the quad's first half.  Same weights and order of operations as
-// two calls of sample: the same bits.  ws: also the saved field's sample.
-template <bool WS>
-__device__ inline float2 sample_q(const float4* __restrict__ f, const Dims& d, float gx, float gy, float gz) {
+__device__ inline float4 x_taps(const float* __restrict__ f, long long at, long long next) {
+  return make_float4(f[at], f[next], 0.f, 0.f);
+}
+template <bool WS, typename Q>
+__device__ inline float2 sample_q(const Q* __restrict__ f, const Dims& d, float gx, float gy, float gz) {
   float fi = floorf(gx), fj = floorf(gy), fk = floorf(gz);
   int i0 = (int)fi, j0 = (int)fj, k0 = (int)fk;
   float fx = gx - fi, fy = gy - fj, fz = gz - fk;
@@ -82,7 +64,8 @@ __device__ inline float2 sample_q(const float4* __restrict__ f, const Dims& d, f
   const long long sy = (long long)d.nbx * kBlockVol, sz = sy * d.nby;
   const int ia = min(max(i0, 0), d.nx - 1);
   const bool lo = i0 < 0;
-  const long long X = (long long)(ia >> 2) * kBlockVol + (ia & 3);
+  const int ib = min(ia + 1, d.nx - 1);
+  const long long X = (long long)(ia >> 2) * kBlockVol + (ia & 3), X1 = (long long)(ib >> 2) * kBlockVol + (ib & 3);
   long long Y[2], Z[2];
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
@@ -96,7 +79,7 @@ __device__ inline float2 sample_q(const float4* __restrict__ f, const Dims& d, f
   for (int dk = 0; dk < 2; ++dk)
 #pragma unroll
     for (int dj = 0; dj < 2; ++dj) {
-      const float4 q = f[X + Y[dj] + Z[dk]];
+      const float4 q = x_taps(f, X + Y[dj] + Z[dk], X1 + Y[dj] + Z[dk]);
       const float v1 = lo ? q.x : q.y, s1 = lo ? q.z : q.w;
       const float w0 = wx[0] * wy[dj] * wz[dk], w1 = wx[1] * wy[dj] * wz[dk];
       sv = fmaf(w0, q.x, sv);
@@ -107,20 +90,14 @@ __device__ inline float2 sample_q(const float4* __restrict__ f, const Dims& d, f
   return make_float2(sv, ss);
 }
 
-__device__ inline void sample_vel(const G2PArgs& a, const float* const* f, float x, float y, float z, float out[3]) {
+// u, v, w (and, WS, the saved u, v, w) at a point from the packed fields
+template <bool WS, typename Q>
+__device__ inline void sample_vel(const G2PArgs& a, float x, float y, float z, float out[3], float sav[3]) {
   float px = (x - a.ox) * a.inv_dx, py = (y - a.oy) * a.inv_dx, pz = (z - a.oz) * a.inv_dx;
-  out[0] = sample(f[0], a.df[0], px, py - 0.5f, pz - 0.5f);
-  out[1] = sample(f[1], a.df[1], px - 0.5f, py, pz - 0.5f);
-  out[2] = sample(f[2], a.df[2], px - 0.5f, py - 0.5f, pz);
-}
-
-// u, v, w (and, WS, the saved u, v, w) at a point from the quad fields
-template <bool WS>
-__device__ inline void sample_vel_q(const G2PArgs& a, float x, float y, float z, float out[3], float sav[3]) {
-  float px = (x - a.ox) * a.inv_dx, py = (y - a.oy) * a.inv_dx, pz = (z - a.oz) * a.inv_dx;
-  const float2 s0 = sample_q<WS>(a.quad[0], a.df[0], px, py - 0.5f, pz - 0.5f);
-  const float2 s1 = sample_q<WS>(a.quad[1], a.df[1], px - 0.5f, py, pz - 0.5f);
-  const float2 s2 = sample_q<WS>(a.quad[2], a.df[2], px - 0.5f, py - 0.5f, pz);
+  auto field = [&](int ax) { return static_cast<const Q*>(a.field[ax]); };
+  const float2 s0 = sample_q<WS>(field(0), a.df[0], px, py - 0.5f, pz - 0.5f);
+  const float2 s1 = sample_q<WS>(field(1), a.df[1], px - 0.5f, py, pz - 0.5f);
+  const float2 s2 = sample_q<WS>(field(2), a.df[2], px - 0.5f, py - 0.5f, pz);
   out[0] = s0.x; out[1] = s1.x; out[2] = s2.x;
   if (WS) { sav[0] = s0.y; sav[1] = s1.y; sav[2] = s2.y; }
 }
@@ -153,10 +130,13 @@ __device__ inline void block_flush_counters(int (&cnt)[8], float speed, int32_t*
   }
 }
 
-// grid-stride over particles (fixed grid), counters flushed once per workgroup.  QUAD
-// (the G2P with the quad fields packed): every sample from the quads.
-template <bool QUAD>
+// grid-stride over particles (fixed grid), counters flushed once per workgroup.  The
+// grid's fields packed as Q: quads (the G2P), pairs of the velocity (advection alone), or
+// the plain velocity (advection of fewer particles than cells, where packing the grid
+// costs more than it saves: 14 ps a cell against 13 a particle).
+template <typename Q>
 __global__ void __launch_bounds__(256) k_g2p_advect(G2PArgs a) {
+  constexpr bool QUAD = std::is_same<Q, float4>::value;
   int cnt[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   float speed = 0.f;
   // Workgroups are dealt round-robin to the 8 XCDs; workgroup w (XCD w % 8) walks
@@ -170,10 +150,7 @@ __global__ void __launch_bounds__(256) k_g2p_advect(G2PArgs a) {
     float x = a.P.x[p], y = a.P.y[p], z = a.P.z[p];
     uint8_t ty = a.P.type[p];
     float k1[3], sv[3];
-    if (QUAD)
-      sample_vel_q<true>(a, x, y, z, k1, sv);
-    else
-      sample_vel(a, a.vel, x, y, z, k1);
+    sample_vel<QUAD, Q>(a, x, y, z, k1, sv);
     if (QUAD) {
       float al = ty == 0 ? a.aL : a.aG;
       float u = a.P.u[p], v = a.P.v[p], w = a.P.w[p];
@@ -189,17 +166,14 @@ __global__ void __launch_bounds__(256) k_g2p_advect(G2PArgs a) {
       if (a.order == 3) {
         float q[3], k3[3];
         for (int c = 0; c < 3; ++c) q[c] = pos[c] + k1[c] * (0.5f * dt);
-        if (QUAD) sample_vel_q<false>(a, q[0], q[1], q[2], k2, nullptr);
-        else sample_vel(a, a.vel, q[0], q[1], q[2], k2);
+        sample_vel<false, Q>(a, q[0], q[1], q[2], k2, nullptr);
         for (int c = 0; c < 3; ++c) q[c] = (pos[c] - k1[c] * dt) + k2[c] * (2.f * dt);
-        if (QUAD) sample_vel_q<false>(a, q[0], q[1], q[2], k3, nullptr);
-        else sample_vel(a, a.vel, q[0], q[1], q[2], k3);
+        sample_vel<false, Q>(a, q[0], q[1], q[2], k3, nullptr);
         for (int c = 0; c < 3; ++c) nxt[c] = pos[c] + ((k1[c] + k2[c] * 4.f) + k3[c]) * (dt / 6.f);
       } else {
         float m[3];
         for (int c = 0; c < 3; ++c) m[c] = pos[c] + k1[c] * (0.5f * dt);
-        if (QUAD) sample_vel_q<false>(a, m[0], m[1], m[2], k2, nullptr);
-        else sample_vel(a, a.vel, m[0], m[1], m[2], k2);
+        sample_vel<false, Q>(a, m[0], m[1], m[2], k2, nullptr);
         for (int c = 0; c < 3; ++c) nxt[c] = pos[c] + k2[c] * dt;
       }
       bool any = false;
@@ -216,6 +190,18 @@ __global__ void __launch_bounds__(256) k_g2p_advect(G2PArgs a) {
     }
   }
   block_flush_counters(cnt, speed, a.esc, a.vmax_bits, a.do_advect, a.do_g2p);
+}
+
+// the pair field of one face axis: Q[q] = (vel of face q, vel of its +x neighbour)
+__global__ void __launch_bounds__(256) k_pack_pair(Dims d, const float* __restrict__ vel, float2* __restrict__ out) {
+  for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < d.nblocks * kBlockVol;
+       q += (long long)gridDim.x * 256) {
+    int bx, by, bz;
+    block_coords(d, q >> 6, bx, by, bz);
+    const int l = (int)(q & 63), i = bx * 4 + (l & 3);
+    const long long n = i + 1 < d.nx ? ((l & 3) < 3 ? q + 1 : q + kBlockVol - 3) : q;
+    out[q] = make_float2(vel[q], vel[n]);
+  }
 }
 
 // the quad field of one face axis: Q[q] = (vel, saved) of face q and of its +x

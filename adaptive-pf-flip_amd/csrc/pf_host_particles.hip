@@ -168,10 +168,6 @@ int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double d
   G2PArgs a;
   a.g = c->geom;
   a.df[0] = c->du; a.df[1] = c->dv; a.df[2] = c->dw;
-  for (int ax = 0; ax < 3; ++ax) {
-    a.vel[ax] = c->f[F_U + ax];
-    a.saved[ax] = c->f[F_SU + ax];
-  }
   a.P = c->pa;
   a.n = c->np;
   a.inv_dx = (float)(1.0 / c->geom.dx);
@@ -186,25 +182,32 @@ int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double d
   a.esc = c->esc_dev;
   a.vmax_bits = reinterpret_cast<uint32_t*>(c->vmax_dev);
   const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
-  if (g2p)
-    for (int ax = 0; ax < 3; ++ax) {
-      if (!c->g2p_quad[ax]) HIP_TRY(c, dalloc(&c->g2p_quad[ax], fd[ax]->nblocks * kBlockVol));
-      a.quad[ax] = c->g2p_quad[ax];
-    }
+  const bool pairs = !g2p && c->np >= (long long)g.nx * g.ny * g.nz;
+  for (int ax = 0; ax < 3; ++ax) {
+    if ((g2p || pairs) && !c->g2p_quad[ax]) HIP_TRY(c, dalloc(&c->g2p_quad[ax], fd[ax]->nblocks * kBlockVol));
+    a.field[ax] = g2p || pairs ? static_cast<const void*>(c->g2p_quad[ax]) : c->f[F_U + ax];
+  }
   // the G2P reduces the max speed of the velocities it writes (the next CFL scan's value)
   if (g2p) HIP_TRY(c, fill_u32(c->stream, reinterpret_cast<uint32_t*>(c->vmax_dev), 0u, 1));
   {
     // (the kernel timer covers the packing and the kernel)
     const long long ki = kbegin(c, PF_K_G2P_ADVECT);
     const unsigned grid = xcd_grid(c->np, 256, 8192);
-    if (g2p) {
-      for (int ax = 0; ax < 3; ++ax)
-        hipLaunchKernelGGL(k_pack_quad, dim3(std::min<unsigned>(grid_for(fd[ax]->nblocks * kBlockVol, 256), 8192u)),
-                           dim3(256), 0, c->stream, *fd[ax], c->f[F_U + ax], c->f[F_SU + ax], c->g2p_quad[ax]);
-      hipLaunchKernelGGL(k_g2p_advect<true>, dim3(grid), dim3(256), 0, c->stream, a);
-    } else {
-      hipLaunchKernelGGL(k_g2p_advect<false>, dim3(grid), dim3(256), 0, c->stream, a);
+    for (int ax = 0; ax < 3; ++ax) {
+      const dim3 gp(std::min<unsigned>(grid_for(fd[ax]->nblocks * kBlockVol, 256), 8192u));
+      if (g2p)
+        hipLaunchKernelGGL(k_pack_quad, gp, dim3(256), 0, c->stream, *fd[ax], c->f[F_U + ax], c->f[F_SU + ax],
+                           c->g2p_quad[ax]);
+      else if (pairs)
+        hipLaunchKernelGGL(k_pack_pair, gp, dim3(256), 0, c->stream, *fd[ax], c->f[F_U + ax],
+                           reinterpret_cast<float2*>(c->g2p_quad[ax]));
     }
+    if (g2p)
+      hipLaunchKernelGGL(k_g2p_advect<float4>, dim3(grid), dim3(256), 0, c->stream, a);
+    else if (pairs)
+      hipLaunchKernelGGL(k_g2p_advect<float2>, dim3(grid), dim3(256), 0, c->stream, a);
+    else
+      hipLaunchKernelGGL(k_g2p_advect<float>, dim3(grid), dim3(256), 0, c->stream, a);
     kend(c, ki);
   }
   LAUNCH_CHECK(c);
