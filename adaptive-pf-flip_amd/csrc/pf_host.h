@@ -18,8 +18,8 @@ struct pf_lpc {
   int adam_t = 0;
   long long cap = 0, cap_train = 0;
   __bf16 *X = nullptr, *h1 = nullptr, *h2 = nullptr, *h3 = nullptr, *d3 = nullptr, *d2 = nullptr, *d1 = nullptr;
-  float *o = nullptr, *go = nullptr, *scale = nullptr;
-  float* part = nullptr;
+  float *o = nullptr, *go = nullptr, *tmax = nullptr;
+  double* part = nullptr;
   long long part_cap = 0;
   float *zbuf = nullptr, *qbuf = nullptr, *gz = nullptr;
   // energy objective: the error vector e and r = A e

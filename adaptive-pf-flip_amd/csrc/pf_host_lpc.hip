@@ -6,16 +6,17 @@
 
 namespace {
 
-constexpr int kLpcWgradWGs = 512;
+// partial sums of a layer's weight gradient (three workgroups each), and of the head's
+constexpr int kLpcWgradParts = 256, kLpcHeadParts = 1024;
 
 int lpc_grow(pf_lpc* L, long long nt, bool train) {
   if (nt > L->cap) {
-    dfree(L->X); dfree(L->h1); dfree(L->h2); dfree(L->o); dfree(L->scale);
+    dfree(L->X); dfree(L->h1); dfree(L->h2); dfree(L->o); dfree(L->tmax);
     HIP_TRY(L, dalloc(&L->X, nt * kHaloVol * 4));
     HIP_TRY(L, dalloc(&L->h1, nt * kTileVol * 16));
     HIP_TRY(L, dalloc(&L->h2, nt * kTileVol * 32));
     HIP_TRY(L, dalloc(&L->o, nt * kTileVol));
-    HIP_TRY(L, dalloc(&L->scale, nt));
+    HIP_TRY(L, dalloc(&L->tmax, nt * 8));
     L->cap = nt;
   }
   if (train && nt > L->cap_train) {
@@ -27,7 +28,7 @@ int lpc_grow(pf_lpc* L, long long nt, bool train) {
     HIP_TRY(L, dalloc(&L->go, nt * kTileVol));
     L->cap_train = nt;
   }
-  const long long need = std::max<long long>((long long)kLpcWgradWGs * kNW2, 1024LL * 16);
+  const long long need = (long long)kLpcWgradParts * kOffWH + (long long)kLpcHeadParts * kNWH;
   if (need > L->part_cap) {
     dfree(L->part);
     HIP_TRY(L, dalloc(&L->part, need));
@@ -48,7 +49,7 @@ int lpc_prep(pf_lpc* L, hipStream_t s) {
 int lpc_forward(pf_lpc* L, hipStream_t s, long long nt, bool store_h3, const int* done) {
   int st = lpc_prep(L, s);
   if (st) return st;
-  const dim3 grid((unsigned)(nt * 4));
+  const dim3 grid((unsigned)(nt * 16));
   ConvArgs a{};
   a.ntiles = nt;
   a.done = done;
@@ -62,12 +63,11 @@ int lpc_forward(pf_lpc* L, hipStream_t s, long long nt, bool store_h3, const int
   return PF_OK;
 }
 
-template <int CIN, int COUT, bool PADDED>
-int lpc_wgrad(pf_lpc* L, hipStream_t s, const __bf16* in, const __bf16* g, long long nt, float* dst) {
-  const int nwg = (int)std::min<long long>(kLpcWgradWGs, nt * 16);
-  hipLaunchKernelGGL((k_lpc_wgrad<CIN, COUT, PADDED>), dim3(nwg), dim3(256), 0, s, in, g, nt, L->part);
-  const int n = 27 * CIN * COUT;
-  hipLaunchKernelGGL(k_lpc_sum_parts, dim3((n + 255) / 256), dim3(256), 0, s, L->part, nwg, n, dst);
+// partials of the layer at offset OFF of the weights, to L->part from kLpcWgradParts * OFF
+template <int CIN, int COUT, bool PADDED, int OFF>
+int lpc_wgrad(pf_lpc* L, hipStream_t s, const __bf16* in, const __bf16* g, long long nt, int np) {
+  hipLaunchKernelGGL((k_lpc_wgrad<CIN, COUT, PADDED>), dim3(3 * np), dim3(192), 0, s, in, g, nt,
+                     L->part + (long long)kLpcWgradParts * OFF);
   HIP_TRY(L, hipGetLastError());
   return PF_OK;
 }
@@ -75,10 +75,11 @@ int lpc_wgrad(pf_lpc* L, hipStream_t s, const __bf16* in, const __bf16* g, long 
 // L->grad = d(sum o * go)/dw, from the activations of the last lpc_forward(store_h3)
 int lpc_backward(pf_lpc* L, hipStream_t s, long long nt) {
   const long long ncells = nt * kTileVol;
-  const int hg = (int)std::min<long long>(1024, (ncells + 15) / 16);
-  hipLaunchKernelGGL(k_lpc_head_bwd, dim3(hg), dim3(256), 0, s, L->h3, L->go, L->bf.wh, ncells, L->d3, L->part);
-  hipLaunchKernelGGL(k_lpc_sum_parts, dim3(1), dim3(256), 0, s, L->part, hg, kNWH, L->grad + kOffWH);
-  const dim3 grid((unsigned)(nt * 4));
+  const int hg = (int)std::min<long long>(kLpcHeadParts, (ncells + 15) / 16);
+  const int np = (int)std::min<long long>(kLpcWgradParts, nt * 8);
+  hipLaunchKernelGGL(k_lpc_head_bwd, dim3(hg), dim3(256), 0, s, L->h3, L->go, L->bf.wh, ncells, L->d3,
+                     L->part + (long long)kLpcWgradParts * kOffWH);
+  const dim3 grid((unsigned)(nt * 16));
   ConvArgs a{};
   a.ntiles = nt;
   a.in = L->d3; a.wt = L->bf.w3b; a.out = L->d2; a.mask = L->h2;
@@ -86,10 +87,21 @@ int lpc_backward(pf_lpc* L, hipStream_t s, long long nt) {
   a.in = L->d2; a.wt = L->bf.w2b; a.out = L->d1; a.mask = L->h1;
   hipLaunchKernelGGL((k_lpc_conv<32, 16, false, EPI_MASK>), grid, dim3(256), 0, s, a);
   HIP_TRY(L, hipGetLastError());
-  int st = lpc_wgrad<32, 16, false>(L, s, L->h2, L->d3, nt, L->grad + kOffW3);
-  if (!st) st = lpc_wgrad<16, 32, false>(L, s, L->h1, L->d2, nt, L->grad + kOffW2);
-  if (!st) st = lpc_wgrad<4, 16, true>(L, s, L->X, L->d1, nt, L->grad + kOffW1);
-  return st;
+  int st = lpc_wgrad<32, 16, false, kOffW3>(L, s, L->h2, L->d3, nt, np);
+  if (!st) st = lpc_wgrad<16, 32, false, kOffW2>(L, s, L->h1, L->d2, nt, np);
+  if (!st) st = lpc_wgrad<4, 16, true, kOffW1>(L, s, L->X, L->d1, nt, np);
+  if (st) return st;
+  LpcParts p;
+  const int off[5] = {kOffW1, kOffW2, kOffW3, kOffWH, kNW};
+  for (int l = 0; l < 4; ++l) {
+    p.part[l] = L->part + (long long)kLpcWgradParts * off[l];
+    p.nparts[l] = l < 3 ? np : hg;
+    p.off[l] = off[l];
+  }
+  p.off[4] = kNW;
+  hipLaunchKernelGGL(k_lpc_sum_parts, dim3(kNW / 16), dim3(256), 0, s, p, L->grad);
+  HIP_TRY(L, hipGetLastError());
+  return PF_OK;
 }
 
 // level-1 extents (the 2x2x2 aggregates of the multigrid cycle)
@@ -135,10 +147,9 @@ CwArgs lpc_cw_args(pf_ctx* c) {
   a.marker = c->marker; a.fbeta = c->fbeta; a.fphi = c->fphi;
   a.cd = c->cd32; a.invd = c->invd32;
   a.X = c->lpc->X;
+  a.tmax = c->lpc->tmax;
   return a;
 }
-
-unsigned lpc_tile_grid(long long nt) { return (unsigned)std::max<long long>(1, std::min<long long>(nt, 1024)); }
 
 // the network's per-aggregate weights of the last assembled system into c->mg_cs_net
 // (s = sqrt(w), 1 outside the tiles); store: keep the activations for a backward pass.
@@ -154,11 +165,12 @@ int lpc_cw_weights(pf_ctx* c, bool store) {
   int st = lpc_grow(L, c->ntiles, store);
   if (st) return fail(c, st, "learned preconditioner: " + L->err);
   CwArgs a = lpc_cw_args(c);
-  hipLaunchKernelGGL(k_lpc_cw_gather, dim3((unsigned)c->ntiles), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_lpc_cw_max, dim3((unsigned)c->ntiles * 8), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_lpc_cw_gather, dim3((unsigned)c->ntiles * kCwGatherWGs), dim3(256), 0, c->stream, a);
   LAUNCH_CHECK(c);
   st = lpc_forward(L, c->stream, c->ntiles, store, nullptr);
   if (st) return fail(c, st, "learned preconditioner: " + L->err);
-  hipLaunchKernelGGL(k_lpc_cw_scatter, dim3(lpc_tile_grid(c->ntiles)), dim3(256), 0, c->stream, a, L->o,
+  hipLaunchKernelGGL(k_lpc_cw_scatter, dim3((unsigned)c->ntiles * 16), dim3(256), 0, c->stream, a, L->o,
                      c->mg_cs_net);
   LAUNCH_CHECK(c);
   return PF_OK;

@@ -58,7 +58,7 @@ int pf_lpc_destroy(pf_lpc* L) {
   dfree(L->bf.w1f); dfree(L->bf.w1b); dfree(L->bf.w2f); dfree(L->bf.w2b); dfree(L->bf.w3f); dfree(L->bf.w3b);
   dfree(L->bf.wh);
   dfree(L->X); dfree(L->h1); dfree(L->h2); dfree(L->h3); dfree(L->d3); dfree(L->d2); dfree(L->d1);
-  dfree(L->o); dfree(L->go); dfree(L->scale); dfree(L->part);
+  dfree(L->o); dfree(L->go); dfree(L->tmax); dfree(L->part);
   dfree(L->zbuf); dfree(L->qbuf); dfree(L->gz); dfree(L->ebuf); dfree(L->rbuf); dfree(L->stage);
   for (auto& p : L->l1) dfree(p);
   hipStreamDestroy(L->stream);
@@ -303,7 +303,7 @@ static int lpc_grad_eval(pf_lpc* L, pf_ctx* c, int k, double* loss_out) {
   hipLaunchKernelGGL(k_lpc_cw_grad, dim3(gd1), dim3(256), 0, c->stream, n1, L->l1[2], L->l1[1], L->l1[0], bw,
                      L->l1[4]);
   CwArgs a = lpc_cw_args(c);
-  hipLaunchKernelGGL(k_lpc_cw_gout, dim3(lpc_tile_grid(c->ntiles)), dim3(256), 0, c->stream, a, L->o, L->l1[4],
+  hipLaunchKernelGGL(k_lpc_cw_gout, dim3((unsigned)c->ntiles * 16), dim3(256), 0, c->stream, a, L->o, L->l1[4],
                      c->mg_cs_net, L->go);
   LAUNCH_CHECK(c);
   st = lpc_backward(L, c->stream, c->ntiles);

@@ -46,6 +46,7 @@ struct CwArgs {
   const float* cd;         // FP32 operator: Dirichlet part of the diagonal
   const float* invd;       // FP32 1 / diagonal (0 outside the system)
   __bf16* X;               // [tile][18^3][4]
+  float* tmax;             // [tile][8] largest child beta of the tile's 8 block layers
   const int* done;
 };
 
@@ -93,17 +94,21 @@ __device__ inline CwFeat cw_children(const CwArgs& a, int I, int J, int K) {
   return f;
 }
 
-// one workgroup per tile: the tile's largest child beta, then the 18^3 x 4 input
-__global__ void __launch_bounds__(256) k_lpc_cw_gather(CwArgs a) {
+// the largest child beta of a tile, a workgroup per layer of 8 x 8 fine blocks
+__global__ void __launch_bounds__(256) k_lpc_cw_max(CwArgs a) {
   __shared__ float s_max[256];
   if (a.done && *a.done) return;
-  const long long t = blockIdx.x;
+  const long long t = blockIdx.x >> 3;
   if (t >= a.ntiles) return;
   int I0, J0, K0;
   cw_tile_origin(a, t, I0, J0, K0);
   float bmax = 0.f;
-  for (int q = threadIdx.x; q < 32 * 32 * 32; q += 256) {
-    const int i = 2 * I0 + (q & 31), j = 2 * J0 + ((q >> 5) & 31), k = 2 * K0 + (q >> 10);
+  // 64 consecutive threads read a block's 64 consecutive cells
+#pragma unroll 4
+  for (int q = threadIdx.x; q < 64 * 64; q += 256) {
+    const int b = q >> 6, e = q & 63;
+    const int i = 2 * I0 + 4 * (b & 7) + (e & 3), j = 2 * J0 + 4 * (b >> 3) + ((e >> 2) & 3);
+    const int k = 2 * K0 + 4 * (int)(blockIdx.x & 7) + (e >> 4);
     if (i >= a.g.nx || j >= a.g.ny || k >= a.g.nz) continue;
     const long long c = bm_index(a.dc, i, j, k);
     if (a.marker[c] == CELL_FLUID) bmax = fmaxf(bmax, a.fbeta[c]);
@@ -114,63 +119,74 @@ __global__ void __launch_bounds__(256) k_lpc_cw_gather(CwArgs a) {
     if (threadIdx.x < w) s_max[threadIdx.x] = fmaxf(s_max[threadIdx.x], s_max[threadIdx.x + w]);
     __syncthreads();
   }
-  const float tmax = s_max[0];
+  if (threadIdx.x == 0) a.tmax[blockIdx.x] = s_max[0];
+}
+
+// the 18^3 x 4 input of a tile, an aggregate per thread.  Its 40 child reads are a chain
+// of latencies, so a tile is spread over 23 workgroups: 16 us (and 13 us for the
+// maxima) at 27 tiles, where one workgroup a tile took 153 us for both.
+constexpr int kCwGatherWGs = (5832 + 255) / 256;
+__global__ void __launch_bounds__(256) k_lpc_cw_gather(CwArgs a) {
+  if (a.done && *a.done) return;
+  const long long t = blockIdx.x / kCwGatherWGs;
+  const int q = (int)(blockIdx.x % kCwGatherWGs) * 256 + threadIdx.x;
+  if (t >= a.ntiles || q >= 5832) return;
+  int I0, J0, K0;
+  cw_tile_origin(a, t, I0, J0, K0);
+  float tmax = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) tmax = fmaxf(tmax, a.tmax[t * 8 + w]);
   __bf16* X = a.X + t * 5832LL * 4;
-  for (int q = threadIdx.x; q < 5832; q += 256) {
-    const int I = I0 + q % 18 - 1, J = J0 + (q / 18) % 18 - 1, K = K0 + q / 324 - 1;
-    float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
-    if (I >= 0 && J >= 0 && K >= 0 && I < a.nx1 && J < a.ny1 && K < a.nz1) {
-      const CwFeat f = cw_children(a, I, J, K);
-      if (f.n > 0 && tmax > 0.f) {
-        const float bm = f.bsum / (float)f.n;
-        v0 = fminf(fmaxf(1.f + log10f(fmaxf(bm / tmax, 1e-30f)) * (1.f / 3.f), 0.f), 1.f);
-        v1 = f.psum / (float)f.n;
-        v2 = fminf(fmaxf(log10f(f.bmax / fmaxf(f.bmin, 1e-30f)) * (1.f / 3.f), 0.f), 1.f);
-        v3 = f.dsum > 0.f ? fminf(fmaxf(f.cdsum / f.dsum, 0.f), 1.f) : 0.f;
-      }
+  const int I = I0 + q % 18 - 1, J = J0 + (q / 18) % 18 - 1, K = K0 + q / 324 - 1;
+  float v0 = 0.f, v1 = 0.f, v2 = 0.f, v3 = 0.f;
+  if (I >= 0 && J >= 0 && K >= 0 && I < a.nx1 && J < a.ny1 && K < a.nz1) {
+    const CwFeat f = cw_children(a, I, J, K);
+    if (f.n > 0 && tmax > 0.f) {
+      const float bm = f.bsum / (float)f.n;
+      v0 = fminf(fmaxf(1.f + log10f(fmaxf(bm / tmax, 1e-30f)) * (1.f / 3.f), 0.f), 1.f);
+      v1 = f.psum / (float)f.n;
+      v2 = fminf(fmaxf(log10f(f.bmax / fmaxf(f.bmin, 1e-30f)) * (1.f / 3.f), 0.f), 1.f);
+      v3 = f.dsum > 0.f ? fminf(fmaxf(f.cdsum / f.dsum, 0.f), 1.f) : 0.f;
     }
-    X[q * 4 + 0] = (__bf16)v0;
-    X[q * 4 + 1] = (__bf16)v1;
-    X[q * 4 + 2] = (__bf16)v2;
-    X[q * 4 + 3] = (__bf16)v3;
   }
+  X[q * 4 + 0] = (__bf16)v0;
+  X[q * 4 + 1] = (__bf16)v1;
+  X[q * 4 + 2] = (__bf16)v2;
+  X[q * 4 + 3] = (__bf16)v3;
 }
 
 // s = exp(clamp(o, -kCwMax, kCwMax) / 2) for the tiles' aggregates (the slab holds 1
-// elsewhere)
+// elsewhere); a workgroup per plane of a tile, a thread per aggregate
 __global__ void __launch_bounds__(256) k_lpc_cw_scatter(CwArgs a, const float* __restrict__ o,
                                                         float* __restrict__ s) {
   if (a.done && *a.done) return;
-  for (long long t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
-    int I0, J0, K0;
-    cw_tile_origin(a, t, I0, J0, K0);
-    for (int q = threadIdx.x; q < 4096; q += 256) {
-      const int I = I0 + (q & 15), J = J0 + ((q >> 4) & 15), K = K0 + (q >> 8);
-      if (I >= a.nx1 || J >= a.ny1 || K >= a.nz1) continue;
-      const float ov = fminf(fmaxf(o[t * 4096 + q], -kCwMax), kCwMax);
-      s[bm_index(a.d1, I, J, K)] = expf(0.5f * ov);
-    }
-  }
+  const long long t = blockIdx.x >> 4, q = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= a.ntiles) return;
+  int I0, J0, K0;
+  cw_tile_origin(a, t, I0, J0, K0);
+  const int I = I0 + (threadIdx.x & 15), J = J0 + (threadIdx.x >> 4), K = K0 + (blockIdx.x & 15);
+  if (I >= a.nx1 || J >= a.ny1 || K >= a.nz1) return;
+  const float ov = fminf(fmaxf(o[q], -kCwMax), kCwMax);
+  s[bm_index(a.d1, I, J, K)] = expf(0.5f * ov);
 }
 
-// go[tile][q] = dL/ds * s / 2 where the clamp is inactive (the chain rule through the scatter)
+// go[tile][q] = dL/ds * s / 2 where the clamp is inactive (the chain rule through the
+// scatter), split the same way
 __global__ void __launch_bounds__(256) k_lpc_cw_gout(CwArgs a, const float* __restrict__ o,
                                                      const float* __restrict__ gs, const float* __restrict__ s,
                                                      float* __restrict__ go) {
-  for (long long t = blockIdx.x; t < a.ntiles; t += gridDim.x) {
-    int I0, J0, K0;
-    cw_tile_origin(a, t, I0, J0, K0);
-    for (int q = threadIdx.x; q < 4096; q += 256) {
-      const int I = I0 + (q & 15), J = J0 + ((q >> 4) & 15), K = K0 + (q >> 8);
-      float v = 0.f;
-      if (I < a.nx1 && J < a.ny1 && K < a.nz1) {
-        const long long c = bm_index(a.d1, I, J, K);
-        const float ov = o[t * 4096 + q];
-        if (ov > -kCwMax && ov < kCwMax) v = gs[c] * s[c] * 0.5f;
-      }
-      go[t * 4096 + q] = v;
-    }
+  const long long t = blockIdx.x >> 4, q = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (t >= a.ntiles) return;
+  int I0, J0, K0;
+  cw_tile_origin(a, t, I0, J0, K0);
+  const int I = I0 + (threadIdx.x & 15), J = J0 + (threadIdx.x >> 4), K = K0 + (blockIdx.x & 15);
+  float v = 0.f;
+  if (I < a.nx1 && J < a.ny1 && K < a.nz1) {
+    const long long c = bm_index(a.d1, I, J, K);
+    const float ov = o[q];
+    if (ov > -kCwMax && ov < kCwMax) v = gs[c] * s[c] * 0.5f;
   }
+  go[q] = v;
 }
 
 // t = invd (.) v over a dense slab (zero outside the system, where invd = 0)
