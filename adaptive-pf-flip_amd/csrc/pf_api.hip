@@ -191,7 +191,7 @@ int pf_destroy(pf_ctx* c) {
   hipStreamSynchronize(c->stream);
   for (int f = 0; f < F_N; ++f) { hipFree(c->f[f]); hipFree(c->act[f]); }
   hipFree(c->marker); hipFree(c->cell_count); hipFree(c->cell_start);
-  hipFree(c->color_list); hipFree(c->color_cnt); dfree(c->crowd_list); hipFree(c->pblk); hipFree(c->pblk_prev);
+  hipFree(c->color_list); hipFree(c->color_cnt); hipFree(c->p2g_regions); dfree(c->crowd_list); hipFree(c->pblk); hipFree(c->pblk_prev);
   hipFree(c->blk_flag32); hipFree(c->blk_scan); hipFree(c->morton_flags);
   PBuf* bufs[2] = {&c->pa, &c->pb};
   for (PBuf* b : bufs) {
@@ -583,7 +583,7 @@ int pf_bin_counts(pf_ctx* c, uint32_t* dense) {
 
 int pf_color_lists(pf_ctx* c, int32_t* lists, int64_t capacity, int64_t counts[8]) {
   if (!c || !counts) return PF_ERR_ARG;
-  int st = ensure_binned(c);
+  int st = ensure_color_lists(c);
   if (st) return st;
   HIP_TRY(c, hipMemcpyAsync(c->u32_host, c->color_cnt, sizeof(uint32_t) * 8, hipMemcpyDeviceToHost, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));

@@ -29,7 +29,7 @@ int grow_particles(pf_ctx* c, long long n, bool vol) {
   return PF_OK;
 }
 
-// counting sort of particles by block-major cell index + per-colour source lists
+// counting sort of particles by block-major cell index
 int ensure_binned(pf_ctx* c) {
   if (c->binned) return PF_OK;
   c->mark_order_valid = false;
@@ -67,11 +67,20 @@ int ensure_binned(pf_ctx* c) {
                        c->cell_start, c->pa, c->has_vol);
     LAUNCH_CHECK(c);
   }
+  c->binned = true;
+  c->colors_valid = false;
+  return PF_OK;
+}
+
+// the binned particles' source blocks per colour (large grids' P2G, pf_color_lists)
+int ensure_color_lists(pf_ctx* c) {
+  int st = ensure_binned(c);
+  if (st || c->colors_valid) return st;
   HIP_TRY(c, fill_u32(c->stream, c->color_cnt, 0u, 8));
   hipLaunchKernelGGL(k_color_lists, dim3(grid_for(c->dc.nblocks, 256)), dim3(256), 0, c->stream, c->dc,
                      c->cell_start, c->color_cnt, c->color_list, c->color_cap);
   LAUNCH_CHECK(c);
-  c->binned = true;
+  c->colors_valid = true;
   return PF_OK;
 }
 
@@ -113,7 +122,17 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   int st = ensure_binned(c);
   if (st) return st;
   const Dims* d[3] = {&c->du, &c->dv, &c->dw};
-  for (int ax = 0; ax < 3; ++ax) {
+  const long long nb = c->dc.nblocks;
+  if (nb <= kP2GRegionMost && c->np > 0 && !c->p2g_regions && !c->p2g_no_regions) {
+    // (without the memory for them: by colours)
+    if (hipMalloc((void**)&c->p2g_regions, sizeof(float2) * 3 * 256 * (size_t)nb) != hipSuccess) {
+      (void)hipGetLastError();
+      c->p2g_regions = nullptr;
+      c->p2g_no_regions = true;
+    }
+  }
+  const bool regions = c->p2g_regions && c->np > 0;
+  for (int ax = 0; ax < 3 && !regions; ++ax) {
     HIP_TRY(c, fill_f32(c->stream, c->f[F_U + ax], 0.f, d[ax]->nblocks * kBlockVol));
     HIP_TRY(c, fill_f32(c->stream, c->f[F_MU + ax], 0.f, d[ax]->nblocks * kBlockVol));
     HIP_TRY(c, fill_u8(c->stream, c->act[F_U + ax], 0, d[ax]->nblocks));
@@ -141,6 +160,29 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   a.mp_l = single ? 1.f : (float)(ph->rho_l * Vp);
   a.mp_g = single ? 1.f : (float)(ph->rho_g * Vp);
   if (c->np == 0) return PF_OK;
+  a.regions = c->p2g_regions;
+  if (regions) {
+    // (how many blocks hold particles is on the device; 8 particles a cell is usual)
+    const bool split = p2g_split((uint32_t)std::min<long long>(nb, c->np / 512 + 1));
+    const P2GShared sh = p2g_shared_args(a);
+    const P2GField f0 = p2g_field_args(a, 0), f1 = p2g_field_args(a, 1), f2 = p2g_field_args(a, 2);
+    const dim3 grid((unsigned)nb, split ? 3 : 1);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(64), 0, c->stream, sh, f0, f1, f2); };
+    const long long ki = kbegin(c, PF_K_P2G);
+    if (mr)
+      a.fast32 ? launch(k_p2g_block<2, true>) : launch(k_p2g_block<2, false>);
+    else if (single)
+      a.fast32 ? launch(k_p2g_block<1, true>) : launch(k_p2g_block<1, false>);
+    else
+      a.fast32 ? launch(k_p2g_block<0, true>) : launch(k_p2g_block<0, false>);
+    const long long nf = std::max({d[0]->nblocks, d[1]->nblocks, d[2]->nblocks});
+    hipLaunchKernelGGL(k_p2g_gather, dim3(grid_for(nf, 4), 3), dim3(256), 0, c->stream, sh, f0, f1, f2);
+    kend(c, ki);
+    LAUNCH_CHECK(c);
+    return PF_OK;
+  }
+  st = ensure_color_lists(c);
+  if (st) return st;
   for (int col = 0; col < 8; ++col) {
     a.list = c->color_list + (long long)col * c->color_cap;
     a.count = c->color_cnt + col;

@@ -138,6 +138,9 @@ struct Ctx {
   uint32_t* color_list = nullptr;   // 8 * color_cap
   uint32_t* color_cnt = nullptr;    // 8
   long long color_cap = 0;
+  bool colors_valid = false;        // the lists are those of the last binning
+  float2* p2g_regions = nullptr;    // P2G node sums per source block, for grids of up to kP2GRegionMost blocks
+  bool p2g_no_regions = false;      // no memory for them
   uint32_t* crowd_list = nullptr;   // cells of kRankMax < count <= kSortedMax particles (sorted by id)
   long long crowd_cap = 0;
   uint32_t* pblk = nullptr;         // sorted list of fluid cell blocks

@@ -22,6 +22,8 @@
 //   least 8 cells apart and never overlap, so within one of the 8 colour launches a
 //   node takes at most one addition from a region: a no-return L2 float atomic adds it
 //   into HBM in the same order as a read-modify-write would, without the wave waiting.
+//   Up to kP2GRegionMost blocks the regions go to memory instead, all blocks in one
+//   launch, and a second one adds them up in the same order, colour by colour.
 // * The activation predicate kern(d^2) > 0 is d^2 < 2.25 (exact: d^2/2.25 < 1 in
 //   correctly rounded FP64 iff d^2 < 2.25).  It is evaluated in FP32 and recomputed
 //   in FP64 inside a 1e-5 band around 2.25, so active-block sets match the FP64
@@ -51,6 +53,7 @@ struct P2GArgs {
   float inv_dx_f;
   float mp_l, mp_g;       // rho * Vp per phase
   const uint8_t* valid[3];  // KT = 2 (multires): the enumerated fine faces per axis
+  float2* regions;
 };
 
 // The launch's arguments: what all three face axes share (grid, block list, particle
@@ -69,6 +72,7 @@ struct P2GShared {
   float inv_dx_f;
   float mp_l, mp_g;
   bool has_vol, pow2, fast32;
+  float2* regions;  // the gathered form: [block][axis][256] (momentum, mass) node sums
 };
 
 struct P2GField {
@@ -96,6 +100,7 @@ inline P2GShared p2g_shared_args(const P2GArgs& a) {
   r.inv_dx_f = a.inv_dx_f;
   r.mp_l = a.mp_l; r.mp_g = a.mp_g;
   r.has_vol = a.has_vol; r.pow2 = a.pow2; r.fast32 = a.fast32;
+  r.regions = a.regions;
   return r;
 }
 
@@ -539,6 +544,22 @@ __device__ inline void flush_axis(const P2GField& f, int bx, int by, int bz, flo
   }
 }
 
+// Or stores the region for k_p2g_gather; a node without a contribution holds mass -0
+// (a sum that starts from +0 never is).
+template <int AX>
+__device__ inline void store_axis(float2* out, float2* s_node, uint8_t* s_flag, int lane) {
+  using A = Ax<AX>;
+#pragma unroll
+  for (int e = 0; e < (A::RN + 63) / 64; ++e) {
+    const int r = lane + 64 * e;
+    if (r >= A::RN) continue;
+    const float2 v = s_node[r];
+    out[r] = (s_flag[r] & 1) ? v : make_float2(0.f, -0.f);
+    s_node[r] = make_float2(0.f, 0.f);
+    s_flag[r] = 0;
+  }
+}
+
 // KT = 2: the enumerated faces of the block's region as bit 1 of its flags
 template <int AX>
 __device__ inline void load_valid(const P2GField& f, int bx, int by, int bz, uint8_t* s_flag, int lane) {
@@ -556,9 +577,9 @@ __device__ inline void load_valid(const P2GField& f, int bx, int by, int bz, uin
 }
 
 // one face axis of the block
-template <int AX, int KT, bool F32>
-__device__ inline void p2g_axis(const P2GShared& a, const P2GField& f, int bx, int by, int bz, uint32_t s0, uint32_t cnt,
-                                const uint8_t* ord, float2* s_node, uint8_t* s_flag, int lane) {
+template <int AX, int KT, bool F32, bool REG>
+__device__ inline void p2g_axis(const P2GShared& a, const P2GField& f, uint32_t b, int bx, int by, int bz, uint32_t s0,
+                                uint32_t cnt, const uint8_t* ord, float2* s_node, uint8_t* s_flag, int lane) {
   const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
   if (KT == 2) {
     load_valid<AX>(f, bx, by, bz, s_flag, lane);
@@ -566,38 +587,24 @@ __device__ inline void p2g_axis(const P2GShared& a, const P2GField& f, int bx, i
   }
   splat_axis<AX, KT, F32>(a, f, bx * 4 + lx, by * 4 + ly, bz * 4 + lz, s0, cnt, ord, s_node, s_flag, lx, ly, lz);
   __syncthreads();
-  flush_axis<AX>(f, bx, by, bz, s_node, s_flag, lane);
+  if (REG)
+    store_axis<AX>(a.regions + ((long long)b * 3 + AX) * 256, s_node, s_flag, lane);
+  else
+    flush_axis<AX>(f, bx, by, bz, s_node, s_flag, lane);
   __syncthreads();
 }
 
 // KT = 0: normalized cubic (two-phase); KT = 1: trilinear, unit mass (single-phase);
-// KT = 2: normalized cubic over the enumerated multires faces.  One launch per colour:
-// a block's particles are ranked once and splatted into the three face fields in turn
-// through one LDS node region (12.3 KB of LDS per workgroup with the id ranking).
-//
-// Or each axis takes a workgroup of its own, where that ends the launch sooner.  12
-// workgroups fit a CU (registers and LDS alike), so n blocks take ceil(n / 3072) rounds of
-// the chip, or ceil(3 n / 3072) rounds a third as long plus a tenth for ranking three
-// times: 64^3 (512 blocks a colour) 53 -> 31 us a launch, 144 x 101 x 131 (3600) 134 ->
-// 120; not at 128^3 x 0.6 (2400), 85 -> 91.
-constexpr uint32_t kP2GResident = 256 * 12;
-constexpr uint32_t kP2GSplitMost = 5 * kP2GResident;  // (past five rounds the last one matters little)
-__device__ inline bool p2g_split(uint32_t n) {
-  const uint32_t whole = (n + kP2GResident - 1) / kP2GResident, third = (3 * n + kP2GResident - 1) / kP2GResident;
-  return n <= kP2GSplitMost && 11 * third < 30 * whole;
-}
-template <int KT, bool F32>
-__global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
+// KT = 2: normalized cubic over the enumerated multires faces.  A block's particles are
+// ranked once and splatted into the three face fields in turn (only < 0), or into one of
+// them, through one LDS node region (12.3 KB of LDS per workgroup with the id ranking).
+template <int KT, bool F32, bool REG>
+__device__ inline void p2g_block(const P2GShared& a, const P2GField& fu, const P2GField& fv, const P2GField& fw,
+                                 uint32_t b, int only) {
   __shared__ uint32_t s_ids[kOrdMax * 64];
   __shared__ uint8_t s_ord[64 * kOrdMax];
   __shared__ float2 s_node[256];  // the region's (momentum, mass) sums per node
   __shared__ uint8_t s_flag[256];
-  const uint32_t nblk = *a.count;
-  if (blockIdx.x >= nblk) return;
-  const bool split = gridDim.y == 3 && p2g_split(nblk);
-  if (!split && blockIdx.y > 0) return;
-  const int only = split ? (int)blockIdx.y : -1;
-  const uint32_t b = a.list[blockIdx.x];
   const int lane = threadIdx.x;
   for (int t = lane; t < 256; t += 64) {
     s_node[t] = make_float2(0.f, 0.f);
@@ -626,9 +633,107 @@ __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GF
     ord[0] = 0;
   }
   __syncthreads();
-  if (only <= 0) p2g_axis<0, KT, F32>(a, fu, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
-  if (only < 0 || only == 1) p2g_axis<1, KT, F32>(a, fv, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
-  if (only < 0 || only == 2) p2g_axis<2, KT, F32>(a, fw, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
+  if (only <= 0) p2g_axis<0, KT, F32, REG>(a, fu, b, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
+  if (only < 0 || only == 1) p2g_axis<1, KT, F32, REG>(a, fv, b, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
+  if (only < 0 || only == 2) p2g_axis<2, KT, F32, REG>(a, fw, b, bx, by, bz, s0, cnt, ord, s_node, s_flag, lane);
+}
+
+// An axis a workgroup, where that ends the launch sooner: 12 workgroups fit a CU
+// (registers and LDS alike), so n blocks take ceil(n / 3072) rounds of the chip, or
+// ceil(3 n / 3072) rounds a third as long plus a tenth for ranking three times.
+constexpr uint32_t kP2GResident = 256 * 12;
+constexpr uint32_t kP2GSplitMost = 5 * kP2GResident;  // (past five rounds the last one matters little)
+__host__ __device__ inline bool p2g_split(uint32_t n) {
+  const uint32_t whole = (n + kP2GResident - 1) / kP2GResident, third = (3 * n + kP2GResident - 1) / kP2GResident;
+  return n <= kP2GSplitMost && 11 * third < 30 * whole;
+}
+
+// Every block in one launch, its region sums to memory, for grids of up to
+// kP2GRegionMost blocks; k_p2g_gather adds them up.  Launches by colour leave the chip
+// partly idle at the end of each of the eight, wait for their atomics and need cleared
+// fields.  Bound by the vector ALU while the fullest cells of a wave last.  By colour ->
+// block + gather: 64^3 248 -> 98 + 13 us, 144 x 101 x 131 1075 -> 617 + 77, 128^3 x 0.6
+// 675 -> 391 + 58, 256^3 6670 -> 4757 + 595 (and a fill of six fields saved).
+constexpr long long kP2GRegionMost = 262144;  // 256^3 cells, 1.6 GB of regions
+template <int KT, bool F32>
+__global__ void __launch_bounds__(64) k_p2g_block(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
+  const uint32_t b = blockIdx.x;
+  if (a.start[(long long)b * kBlockVol] == a.start[((long long)b + 1) * kBlockVol]) return;
+  p2g_block<KT, F32, true>(a, fu, fv, fw, b, gridDim.y == 3 ? (int)blockIdx.y : -1);
+}
+
+// One launch per colour for larger grids, without the regions' memory.
+template <int KT, bool F32>
+__global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
+  const uint32_t nblk = *a.count;
+  if (blockIdx.x >= nblk) return;
+  const bool split = gridDim.y == 3 && p2g_split(nblk);
+  if (!split && blockIdx.y > 0) return;
+  p2g_block<KT, F32, false>(a, fu, fv, fw, a.list[blockIdx.x], split ? (int)blockIdx.y : -1);
+}
+
+// A wave per block of a face field: a node lies in the regions of at most two source
+// blocks per direction, of opposite parity, so of at most one block per colour; their
+// sums are added in colour order, as the launches by colour do.  Writes every node and
+// the block's activation, so the fields need no clearing.
+template <int AX>
+__device__ inline void p2g_gather_axis(const P2GShared& a, const P2GField& f, long long fb, int lane) {
+  using A = Ax<AX>;
+  int Bx, By, Bz;
+  block_coords(f.df, fb, Bx, By, Bz);
+  bool occ = false;
+  if (lane < 27) {
+    const int sx = Bx + lane % 3 - 1, sy = By + (lane / 3) % 3 - 1, sz = Bz + lane / 9 - 1;
+    if (sx >= 0 && sy >= 0 && sz >= 0 && sx < a.dc.nbx && sy < a.dc.nby && sz < a.dc.nbz) {
+      const long long b = sx + a.dc.nbx * (sy + (long long)a.dc.nby * sz);
+      occ = a.start[b * kBlockVol] != a.start[(b + 1) * kBlockVol];
+    }
+  }
+  const uint32_t near = (uint32_t)__ballot(occ);  // the 27 blocks around that hold particles
+  const int lx = lane & 3, ly = (lane >> 2) & 3, lz = lane >> 4;
+  float mom = 0.f, mass = 0.f;
+  bool any = false;
+  if (near != 0 && Bx * 4 + lx < f.df.nx && By * 4 + ly < f.df.ny && Bz * 4 + lz < f.df.nz) {
+    // the region coordinate of node l in its own block (d = 0), or in the neighbour d that
+    // also reaches it; -1: none does
+    auto other = [](int l, int R, int& d) {
+      d = l == 3 ? 1 : -1;
+      return l == 3 ? 0 : (l + 5 < R ? l + 5 : -1);
+    };
+    int ox, oy, oz;
+    const int qx = other(lx, A::RX, ox), qy = other(ly, A::RY, oy), qz = other(lz, A::RZ, oz);
+    float2 v[8];
+#pragma unroll
+    for (int col = 0; col < 8; ++col) {
+      const bool px = (col & 1) == (Bx & 1), py = ((col >> 1) & 1) == (By & 1), pz = (col >> 2) == (Bz & 1);
+      const int rx = px ? lx + 1 : qx, ry = py ? ly + 1 : qy, rz = pz ? lz + 1 : qz;
+      const int dx = px ? 0 : ox, dy = py ? 0 : oy, dz = pz ? 0 : oz;
+      v[col] = make_float2(0.f, -0.f);
+      if (rx >= 0 && ry >= 0 && rz >= 0 && ((near >> (dx + 1 + 3 * (dy + 1) + 9 * (dz + 1))) & 1u)) {
+        const long long b = (Bx + dx) + a.dc.nbx * ((By + dy) + (long long)a.dc.nby * (Bz + dz));
+        v[col] = a.regions[(b * 3 + AX) * 256 + rx + A::RX * (ry + A::RY * rz)];
+      }
+    }
+#pragma unroll
+    for (int col = 0; col < 8; ++col)
+      if (__float_as_uint(v[col].y) != 0x80000000u) {
+        mom += v[col].x;
+        mass += v[col].y;
+        any = true;
+      }
+  }
+  f.mom[fb * kBlockVol + lane] = mom;
+  f.mass[fb * kBlockVol + lane] = mass;
+  const bool act = __any(any);
+  if (lane == 0) f.act_vel[fb] = f.act_mass[fb] = act ? 1 : 0;
+}
+
+__global__ void __launch_bounds__(256) k_p2g_gather(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
+  const long long fb = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (blockIdx.y == 0 && fb < fu.df.nblocks) p2g_gather_axis<0>(a, fu, fb, lane);
+  if (blockIdx.y == 1 && fb < fv.df.nblocks) p2g_gather_axis<1>(a, fv, fb, lane);
+  if (blockIdx.y == 2 && fb < fw.df.nblocks) p2g_gather_axis<2>(a, fw, fb, lane);
 }
 
 }  // namespace pf

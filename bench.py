@@ -430,17 +430,19 @@ def main():
         dominant = max(single, key=lambda k: single[k]["total_ms"]) if single else None
         nl, ms = live["p2g"]
         if nl:
-            # one launch per colour: each carries an eighth of the step's algorithmic P2G bytes
+            # a launch per colour carries an eighth of the step's algorithmic P2G bytes (smaller
+            # grids: one launch, timed with the gather of its regions)
             avg = ms / nl
-            per_launch = (P2G_BYTES[0] * npart + P2G_BYTES[1] * fluid) / 8
+            launches = nl // args.steps
+            per_launch = (P2G_BYTES[0] * npart + P2G_BYTES[1] * fluid) / launches
             achieved = per_launch / (avg * 1e-3) / 1e9
             tf = os.path.join(ROOT, "profiles", "p2g_color_rt256_traffic.md")
-            roofline = {"bound": "hbm", "kernel": "k_p2g_color<0, true>", "achieved": round(achieved, 1),
+            roofline = {"bound": "hbm", "kernel": "k_p2g_color<0, true>" if launches == 8 else "k_p2g_block<0, true> + k_p2g_gather", "achieved": round(achieved, 1),
                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                         "traffic": read_traffic(tf) if (os.path.exists(tf) and n == 256) else None,
                         "bytes_per_launch": int(per_launch), "avg_launch_ms": round(avg, 5),
                         "launches_timed": nl, "dominant_kernel_in_step_table": dominant,
-                        "note": "bytes = (25 B/particle + 24 B/fluid cell) / 8 colour launches; the kernel is "
+                        "note": f"bytes = (25 B/particle + 24 B/fluid cell) / {launches} launches; the kernel is "
                                 "VALU-bound: valu_busy and waves_per_simd are the SQ counters of the committed "
                                 "256^3 counter summary"}
             if os.path.exists(tf) and n == 256:
