@@ -18,7 +18,7 @@
 // start, the sums, the row's loads, the reduction), above it HBM (52 B/cell).  The
 // separate form (SpMV, alpha, update, beta: four launches of 2 to 5 us) took, per
 // iteration, 12.6 us at 48^3, 17.7 at 64^3, 33 at 128^3 and 225 to 260 at 256^3; this one
-// 6.9, 7.3, 24 and 233.
+// 6.4, 6.9, 24 and 233.
 #include "pf_internal.h"
 
 namespace pf {
@@ -49,12 +49,6 @@ struct CgRow {
   uint32_t o, xp, xm, y, z;    // byte offsets, kNoLoad where there is nothing to read
   int ly, lz;
 };
-
-__device__ inline double buf_ld_f64(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
-  return __hiloint2double((int)q.y, (int)q.x);
-}
 
 __device__ inline CgRow cg_row(const Dims& dc, uint32_t sy, uint32_t sz, uint32_t b, bool valid, int row) {
   CgRow R;
@@ -291,7 +285,7 @@ struct CgLoads {
 };
 
 // PRE: the first row's loads are issued before the sums are waited for, which hides
-// their latency (64^3: 7.8 -> 7.3 us) for 170 registers, two workgroups to a CU, instead
+// their latency (64^3: 7.8 -> 7.3 us with the sums as they were then) for 170 registers, two workgroups to a CU, instead
 // of 91: better while every workgroup is resident at once, so up to 512 of them (96^3,
 // 864 workgroups: 13.9 us without, 17.4 with; 128^3: 25.9 and 26.5).
 template <bool PRE>

@@ -216,9 +216,9 @@ static int lpc_loss_eval(pf_lpc* L, pf_ctx* c, int k, bool learned, bool store, 
                      c->cy32, c->cz32, 1.f);
   if (energy) {
     hipLaunchKernelGGL(k_lpc_dots3, dim3(G), dim3(256), 0, c->stream, va, L->ebuf, L->qbuf, L->zbuf, r);
-    hipLaunchKernelGGL(k_reduce_slots, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, 3, 0u, c->red);
+    hipLaunchKernelGGL(k_reduce_slots, dim3(3), dim3(256), 0, c->stream, c->partial, (int)G, 0u, c->red);
   } else {
-    hipLaunchKernelGGL(k_reduce_slots, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, 2, 0u, c->red);
+    hipLaunchKernelGGL(k_reduce_slots, dim3(2), dim3(256), 0, c->stream, c->partial, (int)G, 0u, c->red);
   }
   LAUNCH_CHECK(c);
   st = read_small(c);

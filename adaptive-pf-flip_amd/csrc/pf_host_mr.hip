@@ -339,7 +339,7 @@ int mr_reference_solve(pf_ctx* c, const pf_mr_solve_cfg& cf, unsigned G, const V
   const long long N = nfluid;
 
   auto reduce = [&](unsigned g, int nslots, unsigned mask) -> int {
-    hipLaunchKernelGGL(k_reduce_slots, dim3(1), dim3(256), 0, c->stream, c->partial, (int)g, nslots, mask, c->red);
+    hipLaunchKernelGGL(k_reduce_slots, dim3(nslots), dim3(256), 0, c->stream, c->partial, (int)g, mask, c->red);
     LAUNCH_CHECK(c);
     return read_small(c);
   };

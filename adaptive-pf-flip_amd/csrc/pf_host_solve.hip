@@ -840,7 +840,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   if (want_mx) c->mg_mx_n = (int)G;
   }
   // red[2] = sum b^2; red[3] = max |b| (sparse assembly only)
-  hipLaunchKernelGGL(k_reduce_slots, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, mr ? 1 : 2, 2u,
+  hipLaunchKernelGGL(k_reduce_slots, dim3(mr ? 1 : 2), dim3(256), 0, c->stream, c->partial, (int)G, 2u,
                      c->red + 2);
   LAUNCH_CHECK(c);
   record(c, timing, ev_assemble);
@@ -874,7 +874,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
           hipLaunchKernelGGL(k_residual64, dim3(G), dim3(256), 0, c->stream, va, c->b64, c->x64, c->r64, c->cd64,
                              c->cx64, c->cy64, c->cz64));
     LAUNCH_CHECK(c);
-    hipLaunchKernelGGL(k_reduce_slots, dim3(1), dim3(256), 0, c->stream, c->partial, (int)G, 2, 2u, c->red);
+    hipLaunchKernelGGL(k_reduce_slots, dim3(2), dim3(256), 0, c->stream, c->partial, (int)G, 2u, c->red);
     LAUNCH_CHECK(c);
     r_src = c->r64;
     return read_small(c);

@@ -81,17 +81,47 @@ __device__ inline uint8_t marker_at(const uint8_t* mk, const Dims& dc, const Geo
   return mk[bm_index(dc, i, j, k)];
 }
 
+// raw buffer access over a whole array of fewer than 2^31 bytes: 32-bit byte offsets
+// from a scalar descriptor; an offset at or past the array's size reads 0 and touches
+// no memory (the masked loads below use kNoLoad)
+constexpr uint32_t kNoLoad = 0x80000000u;
+__device__ inline __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+
 // ---------------------------------------------------------------- reductions
 
+// A wave's sum or maximum over DPP lane moves (rows of 16 by shifts, then the two row
+// broadcasts; lane 63 has it), which stay in the vector ALU: a butterfly through LDS
+// permutes waits about 100 cycles for each of its six steps.  k_cg_iter at 64^3 (two rounds of
+// five sums) 7.4 -> 6.9 us.
+template <int CTRL, int ROWS>
+__device__ inline double dpp_move(double v, double rest) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(rest), __double2loint(v), CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(rest), __double2hiint(v), CTRL, ROWS, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ inline double wave_last(double v) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), 63),
+                          __builtin_amdgcn_readlane(__double2loint(v), 63));
+}
 __device__ inline double wave_sum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += dpp_move<0x111, 0xf>(v, 0.0);  // row_shr 1, 2, 4, 8
+  v += dpp_move<0x112, 0xf>(v, 0.0);
+  v += dpp_move<0x114, 0xf>(v, 0.0);
+  v += dpp_move<0x118, 0xf>(v, 0.0);
+  v += dpp_move<0x142, 0xa>(v, 0.0);  // row_bcast 15 into rows 1 and 3, 31 into 2 and 3
+  v += dpp_move<0x143, 0xc>(v, 0.0);
+  return wave_last(v);
 }
 __device__ inline double wave_max(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
+  v = fmax(v, dpp_move<0x111, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x112, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x114, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x118, 0xf>(v, v));
+  v = fmax(v, dpp_move<0x142, 0xa>(v, v));
+  v = fmax(v, dpp_move<0x143, 0xc>(v, v));
+  return wave_last(v);
 }
 
 // sum (or max) of NV values per thread over a 256-thread workgroup -> part[slot*stride + blockIdx]
@@ -116,43 +146,64 @@ __device__ inline void block_reduce_store(double (&v)[NV], const bool (&is_max)[
   }
 }
 
-// fixed-order sum of part[0..n) by one 256-thread workgroup: strided per-thread
-// sums, then a wave butterfly and a 4-way combine (n <= 1024 in the solver loop)
-__device__ inline double block_sum_fast(const double* part, int n) {
+// an FP64 element of a buffer of partial sums, 0 past its end
+__device__ inline double buf_ld_f64(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+  return __hiloint2double((int)q.y, (int)q.x);
+}
+
+// fixed-order sums of NS slots of partials, part[q][0..n[q]), by one 256-thread workgroup:
+// per-thread sums, then a wave's and a 4-way combine.  The loads of 1024 partials of
+// every slot are issued before any is waited for (each takes 1 to 2 us where another
+// XCD just wrote it): k_pcg_beta_flex at 128^3 x 0.6 5.6 -> 2.8 us, k_pcg_alpha 3.3 -> 2.6.
+template <int NS>
+__device__ inline void block_sums(const double* const (&part)[NS], const int (&n)[NS], double (&out)[NS]) {
+  __shared__ double s_w[4][NS];
+  double acc[NS] = {};
+  int most = n[0];
+#pragma unroll
+  for (int q = 1; q < NS; ++q) most = max(most, n[q]);
+  for (int base = 0; base < most; base += 1024) {
+    double w[NS][4];
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+      const auto r = buf_rsrc(part[q], (uint32_t)n[q] * 8);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[q][j] = buf_ld_f64(r, (uint32_t)(base + 256 * j + (int)threadIdx.x) * 8);
+    }
+#pragma unroll
+    for (int q = 0; q < NS; ++q) acc[q] += (w[q][0] + w[q][1]) + (w[q][2] + w[q][3]);
+  }
+#pragma unroll
+  for (int q = 0; q < NS; ++q) acc[q] = wave_sum(acc[q]);
+  if ((threadIdx.x & 63) == 0)
+#pragma unroll
+    for (int q = 0; q < NS; ++q) s_w[threadIdx.x >> 6][q] = acc[q];
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NS; ++q) out[q] = (s_w[0][q] + s_w[1][q]) + (s_w[2][q] + s_w[3][q]);
+}
+
+// red[q] = the sum, or the maximum of non-negative values, of slot q (a workgroup each: 10.7 -> 2.4
+// to 4 us against one workgroup that takes the slots in turn)
+__global__ void __launch_bounds__(256) k_reduce_slots(const double* part, int n, unsigned max_mask, double* red) {
   __shared__ double s_w[4];
+  const int q = blockIdx.x;
+  const bool is_max = (max_mask >> q) & 1u;
+  const auto r = buf_rsrc(part + (long long)q * kMaxPartials, (uint32_t)n * 8);
   double acc = 0.0;
-  for (int t = threadIdx.x; t < n; t += 256) acc += part[t];
-  acc = wave_sum(acc);
+  for (int base = 0; base < n; base += 1024) {
+    double w[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = buf_ld_f64(r, (uint32_t)(base + 256 * j + (int)threadIdx.x) * 8);
+    acc = is_max ? fmax(acc, fmax(fmax(w[0], w[1]), fmax(w[2], w[3]))) : acc + ((w[0] + w[1]) + (w[2] + w[3]));
+  }
+  acc = is_max ? wave_max(acc) : wave_sum(acc);
   if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = acc;
   __syncthreads();
-  const double r = (s_w[0] + s_w[1]) + (s_w[2] + s_w[3]);
-  __syncthreads();
-  return r;
-}
-
-// one workgroup sums part[slot*stride + 0..n) in a fixed order
-__device__ inline double block_sum_partials(const double* part, int n, bool is_max) {
-  __shared__ double s[256];
-  double acc = is_max ? 0.0 : 0.0;
-  for (int t = threadIdx.x; t < n; t += 256) acc = is_max ? fmax(acc, part[t]) : acc + part[t];
-  s[threadIdx.x] = acc;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) s[threadIdx.x] = is_max ? fmax(s[threadIdx.x], s[threadIdx.x + w]) : s[threadIdx.x] + s[threadIdx.x + w];
-    __syncthreads();
-  }
-  double r = s[0];
-  __syncthreads();
-  return r;
-}
-
-// red[q] = reduction of slot q (NV slots)
-__global__ void __launch_bounds__(256) k_reduce_slots(const double* part, int n, int nslots,
-                                                      unsigned max_mask, double* red) {
-  for (int q = 0; q < nslots; ++q) {
-    double r = block_sum_partials(part + (long long)q * kMaxPartials, n, (max_mask >> q) & 1u);
-    if (threadIdx.x == 0) red[q] = r;
-  }
+  if (threadIdx.x == 0)
+    red[q] = is_max ? fmax(fmax(s_w[0], s_w[1]), fmax(s_w[2], s_w[3])) : (s_w[0] + s_w[1]) + (s_w[2] + s_w[3]);
 }
 
 // ------------------------------------------------------------ set-up kernels
@@ -490,8 +541,11 @@ __global__ void __launch_bounds__(256) k_pcg_load(VecArgs a, const double* __res
 // fresh start: scalars from the loaded residual
 __global__ void __launch_bounds__(256) k_pcg_start(const double* part, int n, SolveScalars* sc, double delta2,
                                                    double tol2_abs, int max_iter, int between) {
-  double rz = block_sum_partials(part, n, false);
-  double rr = block_sum_partials(part + kMaxPartials, n, false);
+  const double* const slot[2] = {part, part + kMaxPartials};
+  const int num[2] = {n, n};
+  double sum[2];
+  block_sums<2>(slot, num, sum);
+  const double rz = sum[0], rr = sum[1];
   if (threadIdx.x == 0) {
     sc->rz = rz; sc->rr = rr; sc->rr0 = rr; sc->rr_best = rr; sc->tol2 = delta2;
     sc->rr_ref = rr; sc->tol2_abs = tol2_abs;
@@ -504,8 +558,11 @@ __global__ void __launch_bounds__(256) k_pcg_start(const double* part, int n, So
 
 // after a residual replacement: beta from the replaced residual, same direction
 __global__ void __launch_bounds__(256) k_pcg_resume(const double* part, int n, SolveScalars* sc) {
-  double rz = block_sum_partials(part, n, false);
-  double rr = block_sum_partials(part + kMaxPartials, n, false);
+  const double* const slot[2] = {part, part + kMaxPartials};
+  const int num[2] = {n, n};
+  double sum[2];
+  block_sums<2>(slot, num, sum);
+  const double rz = sum[0], rr = sum[1];
   if (threadIdx.x == 0) {
     sc->beta = sc->rz != 0.0 ? rz / sc->rz : 0.0;
     sc->rz = rz; sc->rr = rr; sc->rr_ref = rr;
@@ -553,13 +610,6 @@ __global__ void __launch_bounds__(256) k_pcg_spmv_gather(VecArgs a, const float*
   block_reduce_store<1>(v, mx, a.part, kMaxPartials);
 }
 
-// raw buffer access over a whole array of fewer than 2^31 bytes: 32-bit byte offsets
-// from a scalar descriptor; an offset at or past the array's size reads 0 and touches
-// no memory (the masked loads below use kNoLoad)
-constexpr uint32_t kNoLoad = 0x80000000u;
-__device__ inline __amdgpu_buffer_rsrc_t buf_rsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
 __device__ inline float buf_ld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   return __uint_as_float((uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
 }
@@ -742,7 +792,11 @@ __global__ void __launch_bounds__(256) k_pcg_spmv(VecArgs a, const float* __rest
 // alpha = r.z / p.Ap from the SpMV partials (one workgroup)
 __global__ void __launch_bounds__(256) k_pcg_alpha(const double* part, int n, SolveScalars* sc) {
   if (sc->done) return;
-  const double pap = block_sum_fast(part, n);
+  const double* const slot[1] = {part};
+  const int num[1] = {n};
+  double sum[1];
+  block_sums<1>(slot, num, sum);
+  const double pap = sum[0];
   if (threadIdx.x == 0) {
     sc->pAp = pap;
     if (!(pap > 0.0) || !isfinite(pap)) {
@@ -824,8 +878,11 @@ __global__ void __launch_bounds__(256) k_pcg_update(VecArgs a, float* __restrict
 
 __global__ void __launch_bounds__(256) k_pcg_beta(const double* part, int n, SolveScalars* sc) {
   if (sc->done) return;
-  const double rz = block_sum_fast(part, n);
-  const double rr = block_sum_fast(part + kMaxPartials, n);
+  const double* const slot[2] = {part, part + kMaxPartials};
+  const int num[2] = {n, n};
+  double sum[2];
+  block_sums<2>(slot, num, sum);
+  const double rz = sum[0], rr = sum[1];
   if (threadIdx.x == 0) finish_iteration(sc, rz, rr);
 }
 
@@ -863,9 +920,11 @@ __global__ void __launch_bounds__(256) k_pcg_update_flex(VecArgs a, float* __res
 // iteration end with the flexible beta: slot 2 (nz partials) r.z_new, slots 0/1 (n)
 __global__ void __launch_bounds__(256) k_pcg_beta_flex(const double* part, int n, int nz, SolveScalars* sc) {
   if (sc->done) return;
-  const double rzo = block_sum_fast(part, n);
-  const double rr = block_sum_fast(part + kMaxPartials, n);
-  const double rz = block_sum_fast(part + 2 * kMaxPartials, nz);
+  const double* const slot[3] = {part, part + kMaxPartials, part + 2 * kMaxPartials};
+  const int num[3] = {n, n, nz};
+  double sum[3];
+  block_sums<3>(slot, num, sum);
+  const double rzo = sum[0], rr = sum[1], rz = sum[2];
   if (threadIdx.x == 0) {
     const double beta = flexible_beta(rz, rzo, sc->rz);
     sc->rz_cross = rzo;  // kept for the resume after a residual replacement
@@ -877,8 +936,11 @@ __global__ void __launch_bounds__(256) k_pcg_beta_flex(const double* part, int n
 // fresh start / resume for the flexible solve (z from the network, slot 2)
 __global__ void __launch_bounds__(256) k_pcg_start_flex(const double* part, int n, int nz, SolveScalars* sc,
                                                         double delta2, double tol2_abs, int max_iter, int between) {
-  const double rr = block_sum_partials(part + kMaxPartials, n, false);
-  const double rz = block_sum_partials(part + 2 * kMaxPartials, nz, false);
+  const double* const slot[2] = {part + kMaxPartials, part + 2 * kMaxPartials};
+  const int num[2] = {n, nz};
+  double sum[2];
+  block_sums<2>(slot, num, sum);
+  const double rr = sum[0], rz = sum[1];
   if (threadIdx.x == 0) {
     sc->rz = rz; sc->rr = rr; sc->rr0 = rr; sc->rr_best = rr; sc->tol2 = delta2;
     sc->rr_ref = rr; sc->tol2_abs = tol2_abs;
@@ -894,8 +956,11 @@ __global__ void __launch_bounds__(256) k_pcg_start_flex(const double* part, int 
 // (the replaced residual differs from it by the FP32 drift only).
 __global__ void __launch_bounds__(256) k_pcg_resume_flex(const double* part, int n, int nz, SolveScalars* sc) {
   const double rzo = sc->rz_cross;
-  const double rr = block_sum_partials(part + kMaxPartials, n, false);
-  const double rz = block_sum_partials(part + 2 * kMaxPartials, nz, false);
+  const double* const slot[2] = {part + kMaxPartials, part + 2 * kMaxPartials};
+  const int num[2] = {n, nz};
+  double sum[2];
+  block_sums<2>(slot, num, sum);
+  const double rr = sum[0], rz = sum[1];
   if (threadIdx.x == 0) {
     sc->beta = flexible_beta(rz, rzo, sc->rz);
     sc->rz = rz; sc->rr = rr; sc->rr_ref = rr;
