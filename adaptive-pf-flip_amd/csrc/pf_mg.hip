@@ -370,6 +370,11 @@ __device__ inline float mg_ldh1(__amdgpu_buffer_rsrc_t r, uint32_t off, float sc
 //   MG_RESTRICT  level 1's residual P^T (r - A x): the two aggregates of a row are
 //                pairs of its registers, their y and z partners lanes ^1 and ^4
 // SWEEP and PSWEEP add the partial r . out when part is set.
+// Every load of a slot is masked by its offset instead of a branch (a branch waits for
+// what it loads before the next one is reached) and one load serves both y faces, one
+// both z faces: level 0 at 160^3 / 256^3 FIRST2 13 -> 10.9 / 97 -> 86 us, PSWEEP 20 -> 12.2 /
+// 120 -> 91.  HBM from there (14 B read and 4 written a cell for FIRST2; 22 in all
+// for the sweeps).
 enum { MG_FIRST2 = 0, MG_SWEEP = 1, MG_PSWEEP = 2, MG_RESTRICT = 3 };
 
 struct MgRowArgs {
@@ -410,10 +415,18 @@ __device__ inline float mg_u1(const MgRowBufs& B, float omega, float ui, uint32_
   return buf_ld(B.x, off);
 }
 
-// level 1's correction at aggregates (I, J, K) and (I + 1, J, K), I even: adjacent
+// byte offset of aggregate (I, J, K) in the next level's slab
+__device__ inline uint32_t mg_coff(const Dims& d, int I, int J, int K) {
+  const uint32_t b = (uint32_t)(I >> 2) + (uint32_t)d.nbx * ((uint32_t)(J >> 2) + (uint32_t)d.nby * (uint32_t)(K >> 2));
+  return (b * kBlockVol + (uint32_t)((I & 3) + 4 * (J & 3) + 16 * (K & 3))) * 4;
+}
+
+// the next level's correction at aggregates (I, J, K) and (I + 1, J, K), I even: adjacent
 // in the slab
-__device__ inline float2 mg_cpair(const MgRowArgs& a, int I, int J, int K) {
-  return *reinterpret_cast<const float2*>(a.xc + bm_index(a.dc, I, J, K));
+__device__ inline float2 buf_ld2(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 q = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+  return make_float2(__uint_as_float(q.x), __uint_as_float(q.y));
 }
 
 template <int MODE>
@@ -454,49 +467,34 @@ __global__ void __launch_bounds__(256) k_mg_row(MgRowArgs a) {
     block_coords(a.d, b, bx, by, bz);
     const uint32_t o = valid ? (b * kBlockVol + 4 * row) * 4 : kNoLoad;
     const bool fxp = valid && bx + 1 < a.d.nbx, fxm = valid && bx > 0;
-    const bool fyp = valid && ly == 3 && by + 1 < a.d.nby, fym = valid && ly == 0 && by > 0;
-    const bool fzp = valid && lz == 3 && bz + 1 < a.d.nbz, fzm = valid && lz == 0 && bz > 0;
+    // a row lies on one y face and on one z face at most: one masked load serves both sides
+    const bool fy = valid && ((ly == 3 && by + 1 < a.d.nby) || (ly == 0 && by > 0));
+    const bool fz = valid && ((lz == 3 && bz + 1 < a.d.nbz) || (lz == 0 && bz > 0));
     const uint32_t oxp = fxp ? o + kBlockVol * 4 : kNoLoad, oxm = fxm ? o - kBlockVol * 4 + 12 : kNoLoad;
-    const uint32_t oyp = fyp ? o + sy - 48 : kNoLoad, oym = fym ? o - sy + 48 : kNoLoad;
-    const uint32_t ozp = fzp ? o + sz - 192 : kNoLoad, ozm = fzm ? o - sz + 192 : kNoLoad;
+    const uint32_t oy = fy ? (ly == 3 ? o + sy - 48 : o - sy + 48) : kNoLoad;
+    const uint32_t oz = fz ? (lz == 3 ? o + sz - 192 : o - sz + 192) : kNoLoad;
     const F4 cd = mg_ldh4(B.cd, o, ua), cx = mg_ldh4(B.cx, o, ua), cy = mg_ldh4(B.cy, o, ua);
     const F4 cz = mg_ldh4(B.cz, o, ua);
     const F4 iv = mg_ldh4(B.inv, o, ui), rr = buf_ld4(B.r, o);
     F4 u = mg_u4<MODE>(B, omu, ui, o);
     float uxp = mg_u1<MODE>(B, omu, ui, oxp), uxm = mg_u1<MODE>(B, omu, ui, oxm);
     const float cxxm = mg_ldh1(B.cx, oxm, ua);
-    F4 uyp = mg_u4<MODE>(B, omu, ui, oyp), uym = mg_u4<MODE>(B, omu, ui, oym);
-    F4 uzp = mg_u4<MODE>(B, omu, ui, ozp), uzm = mg_u4<MODE>(B, omu, ui, ozm);
-    const F4 cyym = mg_ldh4(B.cy, oym, ua), czzm = mg_ldh4(B.cz, ozm, ua);
+    F4 uy = mg_u4<MODE>(B, omu, ui, oy), uz = mg_u4<MODE>(B, omu, ui, oz);
+    const F4 cyym = mg_ldh4(B.cy, ly == 0 ? oy : kNoLoad, ua), czzm = mg_ldh4(B.cz, lz == 0 ? oz : kNoLoad, ua);
     const int J = (4 * by + ly) >> 1, K = (4 * bz + lz) >> 1, I0 = 2 * bx;
     if (MODE == MG_PSWEEP) {
-      if (valid) {
-        const float2 c0 = mg_cpair(a, I0, J, K);
+      // masked loads, all in flight with the rest (0 where there is nothing to add)
+      const auto bc = buf_rsrc(a.xc, (uint32_t)(a.dc.nblocks * kBlockVol * 4));
+      const float2 c0 = buf_ld2(bc, valid ? mg_coff(a.dc, I0, J, K) : kNoLoad);
+      const float2 c1 = buf_ld2(bc, fy ? mg_coff(a.dc, I0, ly == 3 ? 2 * by + 2 : 2 * by - 1, K) : kNoLoad);
+      const float2 c2 = buf_ld2(bc, fz ? mg_coff(a.dc, I0, J, lz == 3 ? 2 * bz + 2 : 2 * bz - 1) : kNoLoad);
+      uxp = fmaf(omc, buf_ld(bc, fxp ? mg_coff(a.dc, I0 + 2, J, K) : kNoLoad), uxp);
+      uxm = fmaf(omc, buf_ld(bc, fxm ? mg_coff(a.dc, I0 - 1, J, K) : kNoLoad), uxm);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (iv.v[i] != 0.0f) u.v[i] = fmaf(omc, i < 2 ? c0.x : c0.y, u.v[i]);
-      }
-      if (fxp) uxp = fmaf(omc, a.xc[bm_index(a.dc, I0 + 2, J, K)], uxp);
-      if (fxm) uxm = fmaf(omc, a.xc[bm_index(a.dc, I0 - 1, J, K)], uxm);
-      if (fyp) {
-        const float2 c = mg_cpair(a, I0, 2 * by + 2, K);
-        uyp.v[0] = fmaf(omc, c.x, uyp.v[0]); uyp.v[1] = fmaf(omc, c.x, uyp.v[1]);
-        uyp.v[2] = fmaf(omc, c.y, uyp.v[2]); uyp.v[3] = fmaf(omc, c.y, uyp.v[3]);
-      }
-      if (fym) {
-        const float2 c = mg_cpair(a, I0, 2 * by - 1, K);
-        uym.v[0] = fmaf(omc, c.x, uym.v[0]); uym.v[1] = fmaf(omc, c.x, uym.v[1]);
-        uym.v[2] = fmaf(omc, c.y, uym.v[2]); uym.v[3] = fmaf(omc, c.y, uym.v[3]);
-      }
-      if (fzp) {
-        const float2 c = mg_cpair(a, I0, J, 2 * bz + 2);
-        uzp.v[0] = fmaf(omc, c.x, uzp.v[0]); uzp.v[1] = fmaf(omc, c.x, uzp.v[1]);
-        uzp.v[2] = fmaf(omc, c.y, uzp.v[2]); uzp.v[3] = fmaf(omc, c.y, uzp.v[3]);
-      }
-      if (fzm) {
-        const float2 c = mg_cpair(a, I0, J, 2 * bz - 1);
-        uzm.v[0] = fmaf(omc, c.x, uzm.v[0]); uzm.v[1] = fmaf(omc, c.x, uzm.v[1]);
-        uzm.v[2] = fmaf(omc, c.y, uzm.v[2]); uzm.v[3] = fmaf(omc, c.y, uzm.v[3]);
+      for (int i = 0; i < 4; ++i) {
+        if (iv.v[i] != 0.0f) u.v[i] = fmaf(omc, i < 2 ? c0.x : c0.y, u.v[i]);
+        uy.v[i] = fmaf(omc, i < 2 ? c1.x : c1.y, uy.v[i]);
+        uz.v[i] = fmaf(omc, i < 2 ? c2.x : c2.y, uz.v[i]);
       }
     }
     // (A u) per cell, in mg_ax's order of terms
@@ -510,12 +508,12 @@ __global__ void __launch_bounds__(256) k_mg_row(MgRowArgs a) {
       const float pxp = i < 3 ? u.v[i + 1] : (fxp ? uxp : uc);
       const float pxm = i > 0 ? u.v[i - 1] : (fxm ? uxm : uc);
       const float cxm = i > 0 ? cx.v[i - 1] : (fxm ? cxxm : 0.f);
-      const float pyp = ly < 3 ? syp : (fyp ? uyp.v[i] : uc);
-      const float pym = ly > 0 ? sym : (fym ? uym.v[i] : uc);
-      const float cym = ly > 0 ? scy : (fym ? cyym.v[i] : 0.f);
-      const float pzp = lz < 3 ? szp : (fzp ? uzp.v[i] : uc);
-      const float pzm = lz > 0 ? szm : (fzm ? uzm.v[i] : uc);
-      const float czm = lz > 0 ? scz : (fzm ? czzm.v[i] : 0.f);
+      const float pyp = ly < 3 ? syp : (fy ? uy.v[i] : uc);
+      const float pym = ly > 0 ? sym : (fy ? uy.v[i] : uc);
+      const float cym = ly > 0 ? scy : cyym.v[i];
+      const float pzp = lz < 3 ? szp : (fz ? uz.v[i] : uc);
+      const float pzm = lz > 0 ? szm : (fz ? uz.v[i] : uc);
+      const float czm = lz > 0 ? scz : czzm.v[i];
       float ax = cd.v[i] * uc;
       ax = fmaf(cx.v[i], uc - pxp, ax);
       ax = fmaf(cxm, uc - pxm, ax);

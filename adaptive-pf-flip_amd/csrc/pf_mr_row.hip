@@ -439,15 +439,13 @@ __global__ void __launch_bounds__(256) k_mr_cycle(MrCycleArgs a) {
     }
     if (MODE == MG_PSWEEP) {
       // (a missing neighbour takes the block's own correction, times a zero coupling)
+      // (loads without a branch, in flight with the rest)
       auto corr = [&](int bx, int by, int bz) { return a.omega_c * a.xc[bm_index(a.dcc, bx, by, bz)]; };
-      const float c = corr(R.bx, R.by, R.bz);
-      uxp += R.bx + 1 < op.dc.nbx ? corr(R.bx + 1, R.by, R.bz) : c;
-      uxm += R.bx > 0 ? corr(R.bx - 1, R.by, R.bz) : c;
-      float cy = c, cz = c;
-      if (R.ly == 3 && R.by + 1 < op.dc.nby) cy = corr(R.bx, R.by + 1, R.bz);
-      if (R.ly == 0 && R.by > 0) cy = corr(R.bx, R.by - 1, R.bz);
-      if (R.lz == 3 && R.bz + 1 < op.dc.nbz) cz = corr(R.bx, R.by, R.bz + 1);
-      if (R.lz == 0 && R.bz > 0) cz = corr(R.bx, R.by, R.bz - 1);
+      const int ny = R.ly == 3 ? min(R.by + 1, op.dc.nby - 1) : (R.ly == 0 ? max(R.by - 1, 0) : R.by);
+      const int nz = R.lz == 3 ? min(R.bz + 1, op.dc.nbz - 1) : (R.lz == 0 ? max(R.bz - 1, 0) : R.bz);
+      const float c = corr(R.bx, R.by, R.bz), cy = corr(R.bx, ny, R.bz), cz = corr(R.bx, R.by, nz);
+      uxp += corr(min(R.bx + 1, op.dc.nbx - 1), R.by, R.bz);
+      uxm += corr(max(R.bx - 1, 0), R.by, R.bz);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         if (inv.v[i] != 0.f) u.v[i] += c;
