@@ -171,6 +171,7 @@ int mr_apply_layout(pf_ctx* c, std::vector<Leaf> lv) {
       HIP_TRY(c, dalloc(&c->mr_valid[a], fd[a]->nblocks * kBlockVol));
     }
     HIP_TRY(c, dalloc(&c->mr_info, c->dc.nblocks));
+    HIP_TRY(c, dalloc(&c->mr_cs, c->dc.nblocks));
     HIP_TRY(c, dalloc(&c->mr_vol64, ncell));
     HIP_TRY(c, dalloc(&c->mr_pfull, ncell));
   }

@@ -471,6 +471,7 @@ MrRowOp mr_row_op(const pf_ctx* c) {
   o.dc = c->dc;
   o.info = c->mr_info;
   o.cd = c->cd32; o.cx = c->cx32; o.cy = c->cy32; o.cz = c->cz32; o.inv = c->invd32;
+  o.cs = c->mr_cs;
   return o;
 }
 
@@ -810,6 +811,9 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       mo.b64 = c->b64; mo.cd64 = c->cd64; mo.cx64 = c->cx64; mo.cy64 = c->cy64; mo.cz64 = c->cz64;
       mo.vol64 = c->mr_vol64;
       mo.cd32 = c->cd32; mo.cx32 = c->cx32; mo.cy32 = c->cy32; mo.cz32 = c->cz32; mo.inv32 = c->invd32;
+      mo.cs = c->mr_cs;
+      // (a neighbour outside the list has no couplings)
+      HIP_TRY(c, fill_f32(c->stream, reinterpret_cast<float*>(c->mr_cs), 0.f, 4 * c->dc.nblocks));
       TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble_cells, dim3(G), dim3(256), 0, c->stream, ma, mo));
     }
     LAUNCH_CHECK(c);

@@ -224,6 +224,7 @@ struct Ctx {
   double* mrf = nullptr;            // 15 fine FP64 vectors (ncell each)
   double* mrc = nullptr;            // 6 coarse FP64 vectors
   uint8_t* mr_info = nullptr;       // per block: its level and which neighbours have level 2 (pf_mr_row.hip)
+  float4* mr_cs = nullptr;          // per level-2 block: the sums of its couplings (pf_mr_row.hip)
   long long mrc_cap = 0;
   long long* mr_pin_dev = nullptr;  // pinned anchor (block-major index) or -1
   long long* mr_pin_host = nullptr;

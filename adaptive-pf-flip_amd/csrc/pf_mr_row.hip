@@ -13,8 +13,8 @@
 // What bounds it: the rows' loads from L2 and HBM.  The form it replaces went through
 // each leaf cell's patches one by one (level byte, face index and anchor of every patch)
 // and split the levels over two launches.  On 1.75 million leaf cells of three levels (256^3
-// effective, 131,000 blocks) an SpMV took 194 + 30 us and takes 59, a sweep of the cycle
-// 150 + 20 and takes 53, an FP64 residual 348 and takes 115.
+// effective, 131,000 blocks) an SpMV took 194 + 30 us and takes 49, a sweep of the cycle
+// 150 + 20 and takes 37, an FP64 residual 348 and takes 109.
 #include "pf_internal.h"
 
 namespace pf {
@@ -25,6 +25,7 @@ struct MrRowOp {
   Dims dc;
   const uint8_t* info;
   const float *cd, *cx, *cy, *cz, *inv;
+  const float4* cs;  // per block of level 2: the sums of cd, cx, cy and cz (0 in other blocks)
 };
 struct MrRowOp64 {
   Dims dc;
@@ -61,19 +62,19 @@ struct MrRow {
   uint32_t cxm, cy, cz;          // the lower neighbours' couplings
   bool hxm, hy, hz;              // ... that exist
   bool sy, sz;                   // the face row's values are one value
+  bool pure;                     // a level-2 block among level-2 blocks: one coupling a face
   bool valid;
   int L, ly, lz, row;
   int bx, by, bz;
   float w;                       // share of a leaf cell in one entry of a row
 };
 
-__device__ inline MrRow mr_row(const Dims& dc, const uint8_t* __restrict__ info, uint32_t b, bool valid, int row) {
+__device__ inline MrRow mr_row(const Dims& dc, unsigned f, uint32_t b, bool valid, int row) {
   MrRow R;
   R.valid = valid;
   R.row = row;
   R.ly = row & 3;
   R.lz = row >> 2;
-  const unsigned f = info[b];
   R.L = (int)(f & kMrLevelMask);
   R.w = !valid ? 0.f : (R.L == 0 ? 1.f : (R.L == 1 ? 0.125f : 0.015625f));
   block_coords(dc, b, R.bx, R.by, R.bz);
@@ -113,6 +114,8 @@ __device__ inline MrRow mr_row(const Dims& dc, const uint8_t* __restrict__ info,
     R.cz = base - sz + 48 + 4 * R.ly;
     R.z = R.sz ? base - sz : R.cz;
   }
+  R.pure = R.L == 2 && (f & 4 || R.bx + 1 >= dc.nbx) && (f & 8 || R.bx == 0) && (f & 16 || R.by + 1 >= dc.nby) &&
+           (f & 32 || R.by == 0) && (f & 64 || R.bz + 1 >= dc.nbz) && (f & 128 || R.bz == 0);
   return R;
 }
 
@@ -162,16 +165,47 @@ __device__ inline Row4<T> mr_leaf_sum(Row4<T> a, int L) {
 }
 
 // S u at the row's leaf cells: u its own values, uxp and uxm the cells past its ends, uy
-// and uz its face rows.  Every lane of the wave calls it.
-template <typename T>
-__device__ inline Row4<T> mr_apply(const MrRow& R, const T* __restrict__ cd, const T* __restrict__ cx,
-                                   const T* __restrict__ cy, const T* __restrict__ cz, const Row4<T>& u, T uxp, T uxm,
-                                   const Row4<T>& uy, const Row4<T>& uz) {
+// and uz its face rows.  Every lane of the wave calls it.  With SUMS a pure block's rows read
+// the sums of its 16 couplings a face (summed in FP64 by the assembly) instead of 1.2 KB of
+// couplings: its first row takes the cell's own term and the lower faces, its last row
+// the upper y and z faces.  On 256^3 effective (131,000
+// blocks of three levels) an SpMV 53 -> 49 us, the cycle's four passes 159 -> 146.  Not in the Jacobi
+// iteration, whose small grids wait for latencies: 7.3 -> 7.6 us with them.
+template <typename T, bool SUMS, typename Op>
+__device__ inline Row4<T> mr_apply(const MrRow& R, const Op& op, const Row4<T>& u, T uxp, T uxm, const Row4<T>& uy,
+                                   const Row4<T>& uz) {
   const int lane = threadIdx.x & 63;
-  const Row4<T> d = mr_ld4(cd + R.oc), c0 = mr_ld4(cx + R.oc), c1 = mr_ld4(cy + R.oc), c2 = mr_ld4(cz + R.oc);
-  const Row4<T> y0 = mr_ld4(cy + R.cy), z0 = mr_ld4(cz + R.cz);
-  const T xlo = R.hxm ? cx[R.cxm] : (T)0;
-  Row4<T> a;
+  const bool pure = SUMS && R.pure;
+  Row4<T> d = {}, c0 = {}, c1 = {}, c2 = {}, y0 = {}, z0 = {};
+  T xlo = (T)0;
+  if (!pure) {
+    d = mr_ld4(op.cd + R.oc);
+    c0 = mr_ld4(op.cx + R.oc);
+    c1 = mr_ld4(op.cy + R.oc);
+    c2 = mr_ld4(op.cz + R.oc);
+    y0 = mr_ld4(op.cy + R.cy);
+    z0 = mr_ld4(op.cz + R.cz);
+    if (R.hxm) xlo = op.cx[R.cxm];
+  }
+  Row4<T> a = {};
+  if constexpr (SUMS) {
+    if (pure && (R.row == 0 || R.row == 15)) {
+      const float4 q = op.cs[R.own >> 6];
+      if (R.row == 0) {
+        const float xl = R.hxm ? op.cs[R.xm >> 6].y : 0.f, yl = R.hy ? op.cs[R.y >> 6].z : 0.f,
+                    zl = R.hz ? op.cs[R.z >> 6].w : 0.f;
+        const float own = u.v[0];
+        float s = q.x * own;
+        s = fmaf(q.y, own - uxp, s);
+        s = fmaf(xl, own - uxm, s);
+        s = fmaf(yl, own - uy.v[0], s);
+        a.v[0] = fmaf(zl, own - uz.v[0], s);
+      } else {
+        a.v[0] = fmaf(q.z, u.v[0] - uy.v[0], q.w * (u.v[0] - uz.v[0]));
+      }
+    }
+    if (!__any(!pure)) return mr_leaf_sum(a, R.L);
+  }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const T own = u.v[i];
@@ -185,19 +219,54 @@ __device__ inline Row4<T> mr_apply(const MrRow& R, const T* __restrict__ cd, con
     s = fma(R.ly > 0 ? cyl : (R.hy ? y0.v[i] : (T)0), own - (R.ly > 0 ? ym : uy.v[i]), s);
     s = fma(c2.v[i], own - (R.lz < 3 ? zp : uz.v[i]), s);
     s = fma(R.lz > 0 ? czl : (R.hz ? z0.v[i] : (T)0), own - (R.lz > 0 ? zm : uz.v[i]), s);
-    a.v[i] = s;
+    if (!pure) a.v[i] = s;
   }
   return mr_leaf_sum(a, R.L);
 }
 
-// the list in slots of four blocks (one per 16 lanes), each XCD a contiguous eighth
-#define FOR_MR_ROWS(A, op, R)                                                                            \
-  for (uint32_t _seg = (uint32_t)(((A).nlist + 7) / 8), _s0 = (blockIdx.x & 7) * _seg,                   \
-                _e = min((uint32_t)(A).nlist, _s0 + _seg),                                               \
-                _t = _s0 + ((blockIdx.x >> 3) * 4 + (threadIdx.x >> 6)) * 4;                             \
-       _t < _e; _t += (gridDim.x >> 3) * 16)                                                             \
-    if (const MrRow R = mr_row((op).dc, (op).info, (A).list[min(_t + ((threadIdx.x & 63) >> 4), _e - 1)], \
-                               _t + ((threadIdx.x & 63) >> 4) < _e, threadIdx.x & 15); true)
+// The list in slots of four blocks (one per 16 lanes), each XCD a contiguous eighth.  The
+// next slot's info bytes and the one after's list entries load while a slot is worked
+// on (list, info and values would be three waits in a row): an update 36.5 ->
+// 32.6 us on those blocks, a Jacobi iteration on 80 x 72 x 80 7.34 -> 7.23.
+struct MrWalk {
+  const uint32_t* list;
+  const uint8_t* info;
+  uint32_t t, e, step, b, nb;
+  unsigned f, nf;
+  __device__ MrWalk(const uint32_t* list_, long long nlist, const uint8_t* info_) : list(list_), info(info_) {
+    const uint32_t seg = (uint32_t)((nlist + 7) / 8), s0 = (blockIdx.x & 7) * seg;
+    e = min((uint32_t)nlist, s0 + seg);
+    t = s0 + ((blockIdx.x >> 3) * 4 + (threadIdx.x >> 6)) * 4;
+    step = (gridDim.x >> 3) * 16;
+    b = nb = 0;
+    f = nf = 0;
+    if (t < e) {
+      b = at(t);
+      nb = at(t + step);
+      f = info[b];
+    }
+  }
+  __device__ uint32_t at(uint32_t s) const { return list[min(s + ((threadIdx.x & 63) >> 4), e - 1)]; }
+  __device__ bool more() const { return t < e; }
+  __device__ bool valid() const { return t + ((threadIdx.x & 63) >> 4) < e; }
+  // (call with the slot's b and f taken: prefetches the next)
+  __device__ uint32_t ahead() {
+    nf = info[nb];
+    return at(t + 2 * step);
+  }
+  __device__ void next(uint32_t nnb) {
+    t += step;
+    b = nb;
+    f = nf;
+    nb = nnb;
+  }
+};
+#define FOR_MR_WALK(W, op, R)                                                                    \
+  for (uint32_t _nn; (W).more() && ((_nn = (W).ahead()), true); (W).next(_nn))                    \
+    if (const MrRow R = mr_row((op).dc, (W).f, (W).b, (W).valid(), threadIdx.x & 15); true)
+#define FOR_MR_ROWS(A, op, R)                         \
+  MrWalk _walk((A).list, (A).nlist, (op).info);       \
+  FOR_MR_WALK(_walk, op, R)
 
 // Levels and neighbours' levels of every block (the whole slab), as info bytes.
 __global__ void __launch_bounds__(256) k_mr_info(MrGrid m, uint8_t* __restrict__ info) {
@@ -239,7 +308,7 @@ __global__ void __launch_bounds__(256) k_mr_spmv(VecArgs a, MrRowOp op, const fl
       py.v[i] = fmaf(beta, py.v[i], zy.v[i]);
       pz.v[i] = fmaf(beta, pz.v[i], zz.v[i]);
     }
-    const Row4<float> ap = mr_apply(R, op.cd, op.cx, op.cy, op.cz, p, xp, xm, py, pz);
+    const Row4<float> ap = mr_apply<float, true>(R, op, p, xp, xm, py, pz);
     mr_put(pnew, R, p);
     mr_put(Ap, R, ap);
     double s = 0.0;
@@ -319,12 +388,13 @@ __global__ void __launch_bounds__(256) k_mr_load(VecArgs a, MrRowOp op, const do
   }
 }
 
-// the Jacobi iteration in one kernel (k_cg_iter's twin): 7.7 us on 80 x 72 x 80 with two
+// the Jacobi iteration in one kernel (k_cg_iter's twin): 7.2 us on 80 x 72 x 80 with two
 // levels, where the six separate kernels took 35
 __global__ void __launch_bounds__(256) k_mr_cg_iter(CgArgs a, MrRowOp op) {
   __shared__ double sh[4][CG_SUMS];
   double w[4][CG_SUMS];
   cg_fetch(a, w);
+  MrWalk walk(a.list, a.nlist, op.info);
   SolveScalars S = cg_state(a.in);
   if (!cg_advance(a, w, S, sh)) return;
   const float alpha = (float)S.alpha, beta = (float)S.beta;
@@ -332,7 +402,7 @@ __global__ void __launch_bounds__(256) k_mr_cg_iter(CgArgs a, MrRowOp op) {
     return fmaf(beta, p, inv * fmaf(-alpha, q, r));
   };
   double v[CG_SUMS] = {};
-  FOR_MR_ROWS(a, op, R) {
+  FOR_MR_WALK(walk, op, R) {
     const Row4<float> r = mr_own(a.r, R), q = mr_own(a.q, R), p = mr_own(a.p, R), inv = mr_own(op.inv, R);
     const Row4<float> ry = mr_yrow(a.r, R), qy = mr_yrow(a.q, R), iy = mr_yrow(op.inv, R);
     const Row4<float> rz = mr_zrow(a.r, R), qz = mr_zrow(a.q, R), iz = mr_zrow(op.inv, R);
@@ -347,7 +417,7 @@ __global__ void __launch_bounds__(256) k_mr_cg_iter(CgArgs a, MrRowOp op) {
       py.v[i] = direction(ry.v[i], qy.v[i], py.v[i], iy.v[i]);
       pz.v[i] = direction(rz.v[i], qz.v[i], pz.v[i], iz.v[i]);
     }
-    const Row4<float> qn = mr_apply(R, op.cd, op.cx, op.cy, op.cz, pn, xp, xm, py, pz);
+    const Row4<float> qn = mr_apply<float, false>(R, op, pn, xp, xm, py, pz);
     mr_put(a.x, R, x);
     mr_put(a.rn, R, rn);
     mr_put(a.pn, R, pn);
@@ -375,7 +445,7 @@ __global__ void __launch_bounds__(256) k_mr_residual(VecArgs a, MrRowOp64 op, co
   double rr = 0.0, rm = 0.0;
   FOR_MR_ROWS(a, op, R) {
     const Row4<double> u = mr_own(x, R), uy = mr_yrow(x, R), uz = mr_zrow(x, R);
-    const Row4<double> sx = mr_apply(R, op.cd, op.cx, op.cy, op.cz, u, x[R.xp], x[R.xm], uy, uz);
+    const Row4<double> sx = mr_apply<double, false>(R, op, u, x[R.xp], x[R.xm], uy, uz);
     const Row4<double> vol = mr_ld4(op.vol + R.oc);
     Row4<double> res = mr_leaf_sum(mr_ld4(b64 + R.oc), R.L);
     double s = 0.0;
@@ -453,7 +523,7 @@ __global__ void __launch_bounds__(256) k_mr_cycle(MrCycleArgs a) {
         uz.v[i] += cz;
       }
     }
-    const Row4<float> ax = mr_apply(R, op.cd, op.cx, op.cy, op.cz, u, uxp, uxm, uy, uz);
+    const Row4<float> ax = mr_apply<float, true>(R, op, u, uxp, uxm, uy, uz);
     if (MODE == MG_RESTRICT) {
       float s = 0.f;
 #pragma unroll
@@ -529,6 +599,7 @@ __global__ void __launch_bounds__(256) k_mr_mg_coarse(MrRowOp op, Dims dcc, floa
 struct MrCellOut {
   double *b64, *cd64, *cx64, *cy64, *cz64, *vol64;
   float *cd32, *cx32, *cy32, *cz32, *inv32;
+  float4* cs;
 };
 
 // sum over the lanes (fine cells of a block) of each leaf cell, L wave-uniform
@@ -594,6 +665,10 @@ __global__ void __launch_bounds__(256) k_mr_assemble_cells(MrAsm a, MrCellOut o)
     const bool anchor = fluid && ((i | j | k) & mask) == 0;
     const double Vp = pinned ? 1.0 : V, rhs = pinned ? 0.0 : -div + a.cdiv;
     if (pinned) cd = diag = 1.0;
+    if (L == 2) {
+      const double sx = mr_lane_sum(cp[0], 2), sy = mr_lane_sum(cp[1], 2), sz = mr_lane_sum(cp[2], 2);
+      if (lane == 0) o.cs[b] = make_float4((float)cd, (float)sx, (float)sy, (float)sz);
+    }
     const double bv = anchor ? Vp * rhs : 0.0;
     o.b64[c] = bv;
     o.vol64[c] = anchor ? Vp : 0.0;
