@@ -89,7 +89,9 @@ __global__ void __launch_bounds__(256) k_mr_valid(MrGrid m, int axis, uint8_t* _
 
 // markCells (multires_sim3d_tp.cpp:39-70) per leaf cell: SOLID when one of its fine
 // cells lies in the boundary layer, else FLUID when one holds a particle, else AIR;
-// written to every fine cell of the leaf cell
+// written to every fine cell of the leaf cell.  A leaf cell of level 0 to 2 lies in one
+// block, so in one wave: ballots (256^3 effective: 56 us, 970 when each cell walked its
+// leaf cell); above that each cell walks the s^3 cells.
 __global__ void __launch_bounds__(256) k_mr_mark(MrGrid m, const uint32_t* __restrict__ start,
                                                  uint8_t* __restrict__ marker, uint8_t* __restrict__ act) {
   const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -101,8 +103,14 @@ __global__ void __launch_bounds__(256) k_mr_mark(MrGrid m, const uint32_t* __res
   const int i = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3), k = bz * 4 + (lane >> 4);
   if (i >= m.g.nx || j >= m.g.ny || k >= m.g.nz) return;
   const int L = mr_level(m, i, j, k);
+  const uint64_t walls = __ballot(i == 0 || j == 0 || k == 0 || i == m.g.nx - 1 || j == m.g.ny - 1 || k == m.g.nz - 1);
+  const uint64_t held = __ballot(start[q + 1] > start[q]);
   uint8_t mk = CELL_AIR;
-  if (L >= 0) {
+  if (L >= 0 && L <= 2) {
+    // the leaf cell's lanes: one cell, an aligned 2^3 of them, the block
+    const uint64_t leaf = L == 0 ? 1ull << lane : (L == 1 ? 0x330033ull << (lane & 42) : ~0ull);
+    mk = (walls & leaf) ? CELL_SOLID : ((held & leaf) ? CELL_FLUID : CELL_AIR);
+  } else if (L > 2) {
     const int s = 1 << L;
     const int x0 = i - i % s, y0 = j - j % s, z0 = k - k % s;
     bool solid = false, fluid = false;
