@@ -165,8 +165,9 @@ int lpc_cw_weights(pf_ctx* c, bool store) {
   int st = lpc_grow(L, c->ntiles, store);
   if (st) return fail(c, st, "learned preconditioner: " + L->err);
   CwArgs a = lpc_cw_args(c);
-  hipLaunchKernelGGL(k_lpc_cw_max, dim3((unsigned)c->ntiles * 8), dim3(256), 0, c->stream, a);
-  hipLaunchKernelGGL(k_lpc_cw_gather, dim3((unsigned)c->ntiles * kCwGatherWGs), dim3(256), 0, c->stream, a);
+  const unsigned slots = (unsigned)((c->ntiles + 7) / 8) * 8;
+  hipLaunchKernelGGL(k_lpc_cw_max, dim3(slots * 8), dim3(256), 0, c->stream, a);
+  hipLaunchKernelGGL(k_lpc_cw_gather, dim3(slots * kCwGatherWGs), dim3(256), 0, c->stream, a);
   LAUNCH_CHECK(c);
   st = lpc_forward(L, c->stream, c->ntiles, store, nullptr);
   if (st) return fail(c, st, "learned preconditioner: " + L->err);

@@ -94,11 +94,13 @@ __device__ inline CwFeat cw_children(const CwArgs& a, int I, int J, int K) {
   return f;
 }
 
-// the largest child beta of a tile, a workgroup per layer of 8 x 8 fine blocks
+// the largest child beta of a tile, a workgroup per layer of 8 x 8 fine blocks (a tile's
+// workgroups are 8 apart, on one XCD, here and in the gather)
 __global__ void __launch_bounds__(256) k_lpc_cw_max(CwArgs a) {
   __shared__ float s_max[256];
   if (a.done && *a.done) return;
-  const long long t = blockIdx.x >> 3;
+  const long long t = (blockIdx.x >> 6) * 8LL + (blockIdx.x & 7);
+  const int layer = (blockIdx.x >> 3) & 7;
   if (t >= a.ntiles) return;
   int I0, J0, K0;
   cw_tile_origin(a, t, I0, J0, K0);
@@ -108,7 +110,7 @@ __global__ void __launch_bounds__(256) k_lpc_cw_max(CwArgs a) {
   for (int q = threadIdx.x; q < 64 * 64; q += 256) {
     const int b = q >> 6, e = q & 63;
     const int i = 2 * I0 + 4 * (b & 7) + (e & 3), j = 2 * J0 + 4 * (b >> 3) + ((e >> 2) & 3);
-    const int k = 2 * K0 + 4 * (int)(blockIdx.x & 7) + (e >> 4);
+    const int k = 2 * K0 + 4 * layer + (e >> 4);
     if (i >= a.g.nx || j >= a.g.ny || k >= a.g.nz) continue;
     const long long c = bm_index(a.dc, i, j, k);
     if (a.marker[c] == CELL_FLUID) bmax = fmaxf(bmax, a.fbeta[c]);
@@ -119,7 +121,7 @@ __global__ void __launch_bounds__(256) k_lpc_cw_max(CwArgs a) {
     if (threadIdx.x < w) s_max[threadIdx.x] = fmaxf(s_max[threadIdx.x], s_max[threadIdx.x + w]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) a.tmax[blockIdx.x] = s_max[0];
+  if (threadIdx.x == 0) a.tmax[t * 8 + layer] = s_max[0];
 }
 
 // the 18^3 x 4 input of a tile, an aggregate per thread.  Its 40 child reads are a chain
@@ -128,8 +130,9 @@ __global__ void __launch_bounds__(256) k_lpc_cw_max(CwArgs a) {
 constexpr int kCwGatherWGs = (5832 + 255) / 256;
 __global__ void __launch_bounds__(256) k_lpc_cw_gather(CwArgs a) {
   if (a.done && *a.done) return;
-  const long long t = blockIdx.x / kCwGatherWGs;
-  const int q = (int)(blockIdx.x % kCwGatherWGs) * 256 + threadIdx.x;
+  const uint32_t slot = blockIdx.x >> 3;
+  const long long t = (slot / kCwGatherWGs) * 8LL + (blockIdx.x & 7);
+  const int q = (int)(slot % kCwGatherWGs) * 256 + threadIdx.x;
   if (t >= a.ntiles || q >= 5832) return;
   int I0, J0, K0;
   cw_tile_origin(a, t, I0, J0, K0);
@@ -149,10 +152,8 @@ __global__ void __launch_bounds__(256) k_lpc_cw_gather(CwArgs a) {
       v3 = f.dsum > 0.f ? fminf(fmaxf(f.cdsum / f.dsum, 0.f), 1.f) : 0.f;
     }
   }
-  X[q * 4 + 0] = (__bf16)v0;
-  X[q * 4 + 1] = (__bf16)v1;
-  X[q * 4 + 2] = (__bf16)v2;
-  X[q * 4 + 3] = (__bf16)v3;
+  const bf16x4 v = {(__bf16)v0, (__bf16)v1, (__bf16)v2, (__bf16)v3};
+  reinterpret_cast<bf16x4*>(X)[q] = v;
 }
 
 // s = exp(clamp(o, -kCwMax, kCwMax) / 2) for the tiles' aggregates (the slab holds 1
