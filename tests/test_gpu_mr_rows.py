@@ -77,16 +77,32 @@ def test_fast_solves_match_the_exact_solution(dims, level, boxes):
             assert rel_err(ctx.field(f), g.dense(f)) < 1e-5, f
 
 
-def test_fluid_above_level_2_is_refused_and_the_context_stays_usable():
+def test_fluid_above_level_2_takes_the_patch_walk():
+    """level-3 cells span blocks: the Jacobi solve goes patch by patch, the multigrid refuses,
+    and the context goes on with rows on the next layout"""
     dims, dt = (64, 64, 64), 0.02
-    _, gph = _phase()
+    ph, gph = _phase()
+    leaves = G.mr_layout_fine_box(*dims, level=3)
+    parts = _particles(dims)
     ctx = G.MRContext(*dims, 1.0)
-    ctx.set_layout(G.mr_layout_fine_box(*dims, level=3))
-    ctx.upload(*_particles(dims))
-    for mode in (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID):
-        _to_projection(ctx, gph, dt)
-        with pytest.raises(G.PfError):
-            ctx.mr_project(gph, dt, G.mr_solve_cfg(2000, 1e-9, 0.0, mode=mode))
+    ctx.set_layout(leaves)
+    ctx.upload(*parts)
+    g = O.MRGrid(*dims, 1.0, faithful=False)
+    g.set_leaves(leaves)
+    ps = O.Particles(*parts[:6], type=parts[6])
+    g.mark_cells(ps)
+    g.p2g(ps, ph, 1.0)
+    g.apply_gravity(dt, -9.81)
+    g.apply_walls()
+    cells, A, rhs, pin, vol = _system(g, ph, dt)
+    g.apply_pressure(ph, dt, exact_solution(A, rhs, vol))
+    _to_projection(ctx, gph, dt)
+    st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-11, 0.0))
+    assert st.converged == 1 and st.fluid_cells == len(cells) and st.pinned_cell == pin
+    assert rel_err(ctx.field(G.FIELD_P), g.dense(O.P)) < 1e-6
+    _to_projection(ctx, gph, dt)
+    with pytest.raises(G.PfError):
+        ctx.mr_project(gph, dt, G.mr_solve_cfg(2000, 1e-9, 0.0, mode=G.MR_SOLVE_MULTIGRID))
     ctx.set_layout(G.mr_layout_fine_box(*dims, level=2))
     _to_projection(ctx, gph, dt)
     st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-9, 0.0))
