@@ -766,9 +766,6 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   pa.single = single ? 1 : 0;
   const unsigned G = list_grid(npb);
   const bool refmode = mr && c->mr_cfg && c->mr_cfg->mode == PF_MR_SOLVE_REFERENCE;
-  // leaves above level 2: patch by patch instead of by cell rows (the multigrid refuses them)
-  bool walk = false;
-  for (size_t a = 0; mr && !refmode && a < c->mr_leaves.size(); a += 4) walk = walk || c->mr_leaves[a] > 2;
   if (mr) {
     c->mr_detail = pf_mr_solve_detail{};
     c->mr_detail.coarse_preconditioner_auto_disable_iteration = -1;
@@ -788,7 +785,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     ma.u = c->f[F_U]; ma.v = c->f[F_V]; ma.w = c->f[F_W];
     ma.mu = c->f[F_MU]; ma.mv = c->f[F_MV]; ma.mw = c->f[F_MW];
     ma.part = c->partial;
-    if (refmode || walk) {
+    if (refmode) {
       // the couplings are written per fine face, so the arrays start at zero
       const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
       for (int a = 0; a < 3; ++a) {
@@ -798,17 +795,16 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         ma.cf64[a] = c->mr_cf64[a];
       }
       ma.b64 = c->b64; ma.cd64 = c->cd64; ma.vol64 = c->mr_vol64;
-    }
-    if (refmode) {
       const long long ncell = c->dc.nblocks * kBlockVol;
       ma.rref = c->mrf + 12 * ncell;
       ma.dref = c->mrf + 13 * ncell;
       ma.vtrue = c->mrf + 14 * ncell;
       ma.pin_cell = c->mr_pin_dev;
     }
+    HIP_TRY(c, fill_u32(c->stream, c->u32_dev + 5, 0u, 1));
     hipLaunchKernelGGL(k_mr_pin, dim3(std::min(G, 512u)), dim3(256), 0, c->stream, ma);
     LAUNCH_CHECK(c);
-    if (refmode || walk) {
+    if (refmode) {
       TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble, dim3(G), dim3(256), 0, c->stream, ma));
     } else {
       MrCellOut mo;
@@ -856,6 +852,8 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   // 4. FP64 iterative refinement around the FP32 Jacobi PCG
   VecArgs va;
   va.dc = c->dc; va.list = c->pblk; va.nlist = npb; va.sc = c->sc; va.part = c->partial;
+  hipLaunchKernelGGL(k_ir_start, dim3(G), dim3(256), 0, c->stream, va, c->x64, c->invd32, cfg->warm_start);
+  LAUNCH_CHECK(c);
   MrRowOp mop{};
   MrRowOp64 mrow64{};
   MrOp64 mop64{};
@@ -866,13 +864,10 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     mop64.m = mr_grid(c);
     mop64.cd = c->cd64; mop64.vol = c->mr_vol64;
     for (int a = 0; a < 3; ++a) mop64.cf[a] = c->mr_cf64[a];
-    if (walk) hipLaunchKernelGGL(k_mr_walk_inv, dim3(G), dim3(256), 0, c->stream, va, mop64, c->invd32);
   }
-  hipLaunchKernelGGL(k_ir_start, dim3(G), dim3(256), 0, c->stream, va, c->x64, c->invd32, cfg->warm_start);
-  LAUNCH_CHECK(c);
   const double* r_src = c->r64;  // the FP64 residual the next (re)start loads
   auto residual = [&]() -> int {
-    if (mr && (refmode || walk))
+    if (mr && refmode)
       TIMED(c, PF_K_RESIDUAL64,
             hipLaunchKernelGGL(k_mr_residual64, dim3(G), dim3(256), 0, c->stream, va, mop64, c->b64, c->x64, c->r64));
     else if (mr)
@@ -940,6 +935,8 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
   // weights (z and partial r.z in slot 2, GT partials)
   bool learned = want_learned || want_mg;
   c->mg_cs_active = c->mg_cs;  // caller-set weights (pf_mg_set_correction_weights) or none
+  if (mr && !refmode && c->u32_host[5])
+    return fail(c, PF_ERR_STATE, "multires leaves above level 2 hold FLUID cells: the fast solves take levels 0 to 2");
   if (learned) {
     st = mr ? mr_mg_build(c, mop) : mg_build(c);
     if (st) return st;
@@ -982,11 +979,11 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     // the buffer-addressed kernels take 32-bit byte offsets: arrays below 2 GiB
     const bool spmv_buffers = c->dc.nblocks * kBlockVol * 4 < (1LL << 31);
     CgState cg;
-    const bool one_kernel = mr ? !walk : spmv_buffers;   // the Jacobi iteration as k_cg_iter or k_mr_cg_iter
-    const unsigned GL = mr && !walk ? cg_grid(npb) : G;    // workgroups of the load, one partial each
+    const bool one_kernel = mr || spmv_buffers;   // the Jacobi iteration as k_cg_iter or k_mr_cg_iter
+    const unsigned GL = mr ? cg_grid(npb) : G;    // workgroups of the load, one partial each
     // r32 from the FP64 residual, x32 = 0 (and p = 0)
     auto load = [&](const double* src, float* p) {
-      if (mr && !walk)
+      if (mr)
         hipLaunchKernelGGL(k_mr_load, dim3(GL), dim3(256), 0, c->stream, va, mop, src, c->x32, c->r32, p,
                            static_cast<float*>(nullptr), static_cast<const float*>(nullptr), 0);
       else
@@ -1016,7 +1013,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     if (st) return st;
     // the two iteration kernels use at most 1024 workgroups, so the per-iteration
     // scalar kernels sum few partials
-    const unsigned GS = mr && !walk ? cg_grid(npb) : std::min(G, 1024u);
+    const unsigned GS = mr ? cg_grid(npb) : std::min(G, 1024u);
     VecArgs vs = va;
     int iter_before = 0, iter_base = 0;
     double best_rr = rr, prev_rr = rr;
@@ -1037,10 +1034,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         if (st) return st;
       }
       for (int q = 0; q < (fused ? 0 : q_next); ++q) {
-        if (walk)
-          TIMED(c, PF_K_PCG_SPMV, hipLaunchKernelGGL(k_mr_walk_spmv, dim3(GS), dim3(256), 0, c->stream, vs, mop64,
-                                                     c->z32, c->pA, c->pB, c->Ap));
-        else if (mr)
+        if (mr)
           TIMED(c, PF_K_PCG_SPMV,
                 hipLaunchKernelGGL(k_mr_spmv, dim3(GS), dim3(256), 0, c->stream, vs, mop, c->z32, c->pA, c->pB, c->Ap));
         else if (spmv_buffers)

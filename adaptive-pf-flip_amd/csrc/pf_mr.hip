@@ -439,68 +439,6 @@ __global__ void __launch_bounds__(256) k_mr_residual64(VecArgs a, MrOp64 op, con
   block_reduce_store<2>(v, mx, a.part, kMaxPartials);
 }
 
-// Layouts with leaves above level 2 (their cells span blocks, so not by cell rows): the
-// fast Jacobi solve on the anchors' rows, patch by patch with the FP64 couplings.
-// 1 / diagonal at the FLUID anchors
-__global__ void __launch_bounds__(256) k_mr_walk_inv(VecArgs a, MrOp64 op, float* __restrict__ inv) {
-  const int lane = threadIdx.x & 63;
-  FOR_LIST_BLOCKS(a, b, lane) {
-    const long long c = b * kBlockVol + lane;
-    float v = 0.f;
-    if (op.vol[c] != 0.0) {
-      int bx, by, bz, L;
-      block_coords(op.m.dc, b, bx, by, bz);
-      const int i = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3), k = bz * 4 + (lane >> 4);
-      mr_is_anchor(op.m, i, j, k, L);
-      const double diag =
-          op.cd[c] + mr_apply_row<double>(op.m, op.cf, i, j, k, 1 << L, 1.0, [](long long) { return 0.0; });
-      v = diag > 0.0 ? (float)(1.0 / diag) : 0.f;
-    }
-    inv[c] = v;
-  }
-}
-
-// p_new = z + beta p_old (recomputed at the neighbour anchors), Ap = S p_new, partial p.Ap
-__global__ void __launch_bounds__(256) k_mr_walk_spmv(VecArgs a, MrOp64 op, const float* __restrict__ z,
-                                                      float* __restrict__ pA, float* __restrict__ pB,
-                                                      float* __restrict__ Ap) {
-  if (a.sc->done) return;
-  const int lane = threadIdx.x & 63;
-  const bool odd = a.sc->iter & 1;
-  const float* __restrict__ pold = odd ? pB : pA;
-  float* __restrict__ pnew = odd ? pA : pB;
-  const float beta = (float)a.sc->beta;
-  auto pval = [&](long long n) { return (double)fmaf(beta, pold[n], z[n]); };
-  double pap = 0.0;
-  FOR_LIST_BLOCKS(a, b, lane) {
-    const long long c = b * kBlockVol + lane;
-    const float pc = fmaf(beta, pold[c], z[c]);
-    float ap = 0.f;
-    int bx, by, bz;
-    block_coords(op.m.dc, b, bx, by, bz);
-    const int i = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3), k = bz * 4 + (lane >> 4);
-    const int Lb = mr_level(op.m, bx * 4, by * 4, bz * 4);
-    if (Lb >= 0 && Lb <= 2) {
-      const int s = 1 << Lb;
-      const bool in = i < op.m.g.nx && j < op.m.g.ny && k < op.m.g.nz;
-      const long long anc = bm_index(op.m.dc, i & ~(s - 1), j & ~(s - 1), k & ~(s - 1));
-      const bool live = in && op.vol[anc] != 0.0;
-      const double sum = mr_apply_row_coop<double>(op.m, op.cf, i, j, k, Lb, live, live ? pval(anc) : 0.0, pval);
-      if (live && anc == c) ap = (float)(op.cd[c] * (double)pc + sum);
-    } else if (op.vol[c] != 0.0) {
-      int L;
-      mr_is_anchor(op.m, i, j, k, L);
-      ap = (float)(op.cd[c] * (double)pc + mr_apply_row<double>(op.m, op.cf, i, j, k, 1 << L, (double)pc, pval));
-    }
-    pnew[c] = pc;
-    Ap[c] = ap;
-    pap += (double)pc * (double)ap;
-  }
-  double v[1] = {pap};
-  const bool mx[1] = {false};
-  block_reduce_store<1>(v, mx, a.part, kMaxPartials);
-}
-
 // pressure per fine cell: the solution at the anchor of its leaf cell on FLUID cells
 __global__ void __launch_bounds__(256) k_mr_store_pressure(MrGrid m, const double* __restrict__ x64, float* __restrict__ p,
                                                            double* __restrict__ pfull, uint8_t* __restrict__ act) {

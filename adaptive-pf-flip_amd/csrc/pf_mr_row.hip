@@ -629,6 +629,7 @@ __global__ void __launch_bounds__(256) k_mr_assemble_cells(MrAsm a, MrCellOut o)
     const int i = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3), k = bz * 4 + (lane >> 4);
     const int L = mr_level(a.m, bx * 4, by * 4, bz * 4);  // (wave-uniform)
     const int s = 1 << (L < 0 ? 0 : L), mask = s - 1;
+    if (L > 2 && lane == 0) a.pin[5] = 1;  // (the host refuses the solve)
     const bool fluid = L >= 0 && i < a.m.g.nx && j < a.m.g.ny && k < a.m.g.nz && a.m.marker[c] == CELL_FLUID;
     const double h = dx * (double)s, V = h * h * h;
     const bool pinned = fluid && pins && mr_order_key(a.m, i & ~mask, j & ~mask, k & ~mask, L) == pin_key;

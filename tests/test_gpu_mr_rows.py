@@ -42,18 +42,9 @@ def _to_projection(ctx, gph, dt):
     ctx.apply_walls()
 
 
-@pytest.mark.parametrize("dims,level,boxes", [
-    ((17, 10, 9), 1, ([4, 3, 2, 13, 9, 8],)), ((24, 20, 28), 1, ([0, 0, 0, 9, 9, 9],)),
-    ((21, 19, 30), 1, ([8, 4, 8, 12, 8, 12],)), ((33, 18, 20), 1, ()), ((26, 25, 23), 1, ([0, 9, 0, 26, 20, 23],)),
-    ((40, 36, 24), 2, ([0, 14, 0, 40, 24, 24], [16, 0, 8, 24, 12, 16])),
-    ((37, 30, 33), 2, ([10, 12, 10, 20, 30, 20],) * 2)])
-def test_fast_solves_match_the_exact_solution(dims, level, boxes):
-    print(f"[mr rows] {dims} {level} {boxes}", flush=True)
+def _against_exact(dims, leaves, modes):
     dt = 0.02
     ph, gph = _phase()
-    leaves = G.mr_layout_fine_box(*dims, level=level)
-    for b in boxes:
-        leaves = G.mr_layout_refine(*dims, leaves, b)
     parts = _particles(dims)
     ctx = G.MRContext(*dims, 1.0)
     ctx.set_layout(leaves)
@@ -67,7 +58,7 @@ def test_fast_solves_match_the_exact_solution(dims, level, boxes):
     g.apply_walls()
     cells, A, rhs, pin, vol = _system(g, ph, dt)
     g.apply_pressure(ph, dt, exact_solution(A, rhs, vol))
-    for mode in (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID):
+    for mode in modes:
         _to_projection(ctx, gph, dt)
         st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-11, 0.0, mode=mode))
         assert st.converged == 1 and st.true_max_residual < 1e-11 and st.fallback_used == 0
@@ -77,32 +68,40 @@ def test_fast_solves_match_the_exact_solution(dims, level, boxes):
             assert rel_err(ctx.field(f), g.dense(f)) < 1e-5, f
 
 
-def test_fluid_above_level_2_takes_the_patch_walk():
-    """level-3 cells span blocks: the Jacobi solve goes patch by patch, the multigrid refuses,
-    and the context goes on with rows on the next layout"""
-    dims, dt = (64, 64, 64), 0.02
-    ph, gph = _phase()
+@pytest.mark.parametrize("dims,level,boxes", [
+    ((17, 10, 9), 1, ([4, 3, 2, 13, 9, 8],)), ((24, 20, 28), 1, ([0, 0, 0, 9, 9, 9],)),
+    ((21, 19, 30), 1, ([8, 4, 8, 12, 8, 12],)), ((33, 18, 20), 1, ()), ((26, 25, 23), 1, ([0, 9, 0, 26, 20, 23],)),
+    ((40, 36, 24), 2, ([0, 14, 0, 40, 24, 24], [16, 0, 8, 24, 12, 16])),
+    ((37, 30, 33), 2, ([10, 12, 10, 20, 30, 20],) * 2)])
+def test_fast_solves_match_the_exact_solution(dims, level, boxes):
+    print(f"[mr rows] {dims} {level} {boxes}", flush=True)
+    leaves = G.mr_layout_fine_box(*dims, level=level)
+    for b in boxes:
+        leaves = G.mr_layout_refine(*dims, leaves, b)
+    _against_exact(dims, leaves, (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID))
+
+
+def test_level_3_leaves_of_air_alone():
+    """level-3 leaves above the water, beside blocks of levels 2, 1 and 0 that hold it"""
+    dims = (40, 104, 36)
     leaves = G.mr_layout_fine_box(*dims, level=3)
-    parts = _particles(dims)
+    for b in ([0, 0, 0, 40, 62, 36], [0, 40, 0, 18, 62, 36], [0, 52, 0, 10, 62, 20]):
+        leaves = G.mr_layout_refine(*dims, leaves, b)
+    top = [int(lv[2]) * (4 << int(lv[0])) for lv in leaves if lv[0] == 3]
+    assert sorted(set(leaves[:, 0])) == [0, 1, 2, 3] and min(top) == 64  # (the water reaches into y = 60..64)
+    _against_exact(dims, leaves, (G.MR_SOLVE_FAST,))
+
+
+def test_fluid_above_level_2_is_refused_and_the_context_stays_usable():
+    dims, dt = (64, 64, 64), 0.02
+    _, gph = _phase()
     ctx = G.MRContext(*dims, 1.0)
-    ctx.set_layout(leaves)
-    ctx.upload(*parts)
-    g = O.MRGrid(*dims, 1.0, faithful=False)
-    g.set_leaves(leaves)
-    ps = O.Particles(*parts[:6], type=parts[6])
-    g.mark_cells(ps)
-    g.p2g(ps, ph, 1.0)
-    g.apply_gravity(dt, -9.81)
-    g.apply_walls()
-    cells, A, rhs, pin, vol = _system(g, ph, dt)
-    g.apply_pressure(ph, dt, exact_solution(A, rhs, vol))
-    _to_projection(ctx, gph, dt)
-    st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-11, 0.0))
-    assert st.converged == 1 and st.fluid_cells == len(cells) and st.pinned_cell == pin
-    assert rel_err(ctx.field(G.FIELD_P), g.dense(O.P)) < 1e-6
-    _to_projection(ctx, gph, dt)
-    with pytest.raises(G.PfError):
-        ctx.mr_project(gph, dt, G.mr_solve_cfg(2000, 1e-9, 0.0, mode=G.MR_SOLVE_MULTIGRID))
+    ctx.set_layout(G.mr_layout_fine_box(*dims, level=3))
+    ctx.upload(*_particles(dims))
+    for mode in (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID):
+        _to_projection(ctx, gph, dt)
+        with pytest.raises(G.PfError):
+            ctx.mr_project(gph, dt, G.mr_solve_cfg(2000, 1e-9, 0.0, mode=mode))
     ctx.set_layout(G.mr_layout_fine_box(*dims, level=2))
     _to_projection(ctx, gph, dt)
     st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-9, 0.0))
