@@ -755,6 +755,16 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     if (!s2) s2 = lpc_cw_tiles(c, c->pblk, npb);
     if (s2) return s2;
   }
+  // From here on these blocks' arrays hold this system, so the next solve clears them,
+  // also after an error: a stale coupling in a block outside its list would join a listed
+  // neighbour's row.
+  struct Listed {
+    pf_ctx* c;
+    ~Listed() {
+      std::swap(c->pblk, c->pblk_prev);
+      c->npblk_prev = c->npblk;
+    }
+  } listed{c};
   ProjArgs pa;
   pa.g = g; pa.dc = c->dc; pa.du = c->du; pa.dv = c->dv; pa.dw = c->dw;
   pa.marker = c->marker; pa.list = c->pblk; pa.nlist = npb;
@@ -1203,8 +1213,6 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
                                mr_grid(c), a, c->mr_pfull, c->f[F_U + a], c->f[F_MU + a], pk, dt));
     LAUNCH_CHECK(c);
     record(c, timing, ev_vel);
-    std::swap(c->pblk, c->pblk_prev);
-    c->npblk_prev = npb;
     if (out) *out = S;
     return PF_OK;
   }
@@ -1228,8 +1236,6 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
         hipLaunchKernelGGL(k_velocity_update, dim3(grid_for(npb, 4)), dim3(256), 0, c->stream, vl));
   LAUNCH_CHECK(c);
   record(c, timing, ev_vel);
-  std::swap(c->pblk, c->pblk_prev);
-  c->npblk_prev = npb;
   if (out) *out = S;
   return PF_OK;
 }

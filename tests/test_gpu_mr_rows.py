@@ -106,3 +106,28 @@ def test_fluid_above_level_2_is_refused_and_the_context_stays_usable():
     _to_projection(ctx, gph, dt)
     st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-9, 0.0))
     assert st.converged == 1 and np.isfinite(ctx.field(G.FIELD_P)).all()
+
+
+def test_a_refused_solve_leaves_nothing_to_the_next():
+    """water everywhere on level 3 (refused once its rows are assembled), then at high x only
+    on level 1: its lowest blocks read couplings of blocks that only the first system listed"""
+    dims, dt = (64, 64, 64), 0.02
+    _, gph = _phase()
+    parts = _particles(dims)
+    some = tuple(np.ascontiguousarray(q[parts[0] > 33]) for q in parts)
+    out = []
+    for refused in (True, False):
+        ctx = G.MRContext(*dims, 1.0)
+        if refused:
+            ctx.set_layout(G.mr_layout_fine_box(*dims, level=3))
+            ctx.upload(*parts)
+            _to_projection(ctx, gph, dt)
+            with pytest.raises(G.PfError):
+                ctx.mr_project(gph, dt, G.mr_solve_cfg(2000, 1e-9, 0.0))
+        ctx.set_layout(G.mr_layout_fine_box(*dims, level=1))
+        ctx.upload(*some)
+        _to_projection(ctx, gph, dt)
+        st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, 1e-9, 0.0))
+        assert st.converged == 1
+        out.append((st.iterations, ctx.field(G.FIELD_P)))
+    assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
