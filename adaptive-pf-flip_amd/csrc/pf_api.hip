@@ -91,8 +91,8 @@ int pf_copy_probe(pf_ctx* c, int64_t n, double* ms) {
   if (!c || n <= 0 || (n & 3) != 0 || n > (1LL << 31)) return PF_ERR_ARG;
   // its own buffers (allocated here: a measurement hook, not a step stage)
   float *src = nullptr, *dst = nullptr;
-  HIP_TRY(c, dalloc(&src, n));
-  HIP_TRY(c, dalloc(&dst, n));
+  HIP_TRY(c, dalloc(c, &src, n));
+  HIP_TRY(c, dalloc(c, &dst, n));
   HIP_TRY(c, hipDeviceSynchronize());
   hipEvent_t a, b;
   HIP_TRY(c, hipEventCreate(&a));
@@ -615,7 +615,7 @@ int pf_face_phi(pf_ctx* c, const pf_phase* ph, int32_t axis, double* dense) {
   const Dims& d = axis == 0 ? c->du : (axis == 1 ? c->dv : c->dw);
   const long long n = (long long)d.nx * d.ny * d.nz;
   double* out = nullptr;
-  HIP_TRY(c, dalloc(&out, n));
+  HIP_TRY(c, dalloc(c, &out, n));
   hipLaunchKernelGGL(k_face_phi, dim3(grid_for(n, 256)), dim3(256), 0, c->stream, d, c->f[F_MU + axis],
                      phase_k(ph), out);
   hipError_t e = hipGetLastError();

@@ -85,10 +85,33 @@ hipError_t dalloc(T** p, long long n) {
   *p = nullptr;
   if (n <= 0) n = 1;
   hipError_t e = hipMalloc((void**)p, sizeof(T) * (size_t)n);
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess) {
+    (void)hipGetLastError();  // (reported here; a later launch check is not to find it)
+    *p = nullptr;
+    return e;
+  }
   e = hipMemsetAsync(*p, 0, sizeof(T) * (size_t)n, nullptr);
   if (e != hipSuccess) return e;
   return hipStreamSynchronize(nullptr);
+}
+
+template <typename T>
+void dfree(T*& p) {
+  if (p) (void)hipFree((void*)p);
+  p = nullptr;
+}
+
+// The same for a call on a context (or null): where memory runs out, the regions that the
+// context's splat keeps are given back first.  The splat takes them again when they
+// fit, and does without them otherwise.
+template <typename T>
+hipError_t dalloc(pf_ctx* c, T** p, long long n) {
+  hipError_t e = dalloc(p, n);
+  if (e == hipErrorOutOfMemory && c && c->p2g_regions && hipStreamSynchronize(c->stream) == hipSuccess) {
+    dfree(c->p2g_regions);
+    e = dalloc(p, n);
+  }
+  return e;
 }
 
 unsigned grid_for(long long work, long long per_block) {
@@ -157,12 +180,6 @@ PhaseK phase_k(const pf_phase* ph) {
   k.rmin = std::log(ph->rho_l / ph->rho_g) * ph->rho_g * ph->rho_tilde_0;
   k.den = ph->alpha_phi * ph->rho_tilde_0 * ph->rho_l;
   return k;
-}
-
-template <typename T>
-void dfree(T*& p) {
-  if (p) (void)hipFree((void*)p);
-  p = nullptr;
 }
 
 int read_small(pf_ctx* c) {

@@ -11,9 +11,9 @@ namespace {
 // a particle buffer of cap entries (with volumes)
 int alloc_pbuf(pf_ctx* c, PBuf& b, long long cap) {
   b = PBuf{};
-  HIP_TRY(c, dalloc(&b.x, cap)); HIP_TRY(c, dalloc(&b.y, cap)); HIP_TRY(c, dalloc(&b.z, cap));
-  HIP_TRY(c, dalloc(&b.u, cap)); HIP_TRY(c, dalloc(&b.v, cap)); HIP_TRY(c, dalloc(&b.w, cap));
-  HIP_TRY(c, dalloc(&b.type, cap)); HIP_TRY(c, dalloc(&b.id, cap)); HIP_TRY(c, dalloc(&b.vol, cap));
+  HIP_TRY(c, dalloc(c, &b.x, cap)); HIP_TRY(c, dalloc(c, &b.y, cap)); HIP_TRY(c, dalloc(c, &b.z, cap));
+  HIP_TRY(c, dalloc(c, &b.u, cap)); HIP_TRY(c, dalloc(c, &b.v, cap)); HIP_TRY(c, dalloc(c, &b.w, cap));
+  HIP_TRY(c, dalloc(c, &b.type, cap)); HIP_TRY(c, dalloc(c, &b.id, cap)); HIP_TRY(c, dalloc(c, &b.vol, cap));
   return PF_OK;
 }
 
@@ -30,7 +30,7 @@ int ensure_scan_capacity(pf_ctx* c, long long n) {
   hipFree(c->scan_tiles);
   c->scan_tiles = nullptr;
   c->scan_tile_cap = 0;
-  HIP_TRY(c, dalloc(&c->scan_tiles, need));
+  HIP_TRY(c, dalloc(c, &c->scan_tiles, need));
   c->scan_tile_cap = need;
   return PF_OK;
 }
@@ -70,19 +70,19 @@ int run_adaptivity(pf_ctx* c, const pf_adapt_cfg* cfg, pf_adapt_stats* out) {
   if (np > c->pa_cap) {
     dfree(c->pa_alive); dfree(c->pa_key); dfree(c->pa_by_id); dfree(c->pa_new_id);
     const long long cap = np + np / 4;
-    HIP_TRY(c, dalloc(&c->pa_alive, cap));
-    HIP_TRY(c, dalloc(&c->pa_key, cap));
-    HIP_TRY(c, dalloc(&c->pa_by_id, cap + 1));
-    HIP_TRY(c, dalloc(&c->pa_new_id, cap + 1));
+    HIP_TRY(c, dalloc(c, &c->pa_alive, cap));
+    HIP_TRY(c, dalloc(c, &c->pa_key, cap));
+    HIP_TRY(c, dalloc(c, &c->pa_by_id, cap + 1));
+    HIP_TRY(c, dalloc(c, &c->pa_new_id, cap + 1));
     c->pa_cap = cap;
   }
   if (!c->pa_cflag) {
-    HIP_TRY(c, dalloc(&c->pa_cflag, ncell));
-    HIP_TRY(c, dalloc(&c->pa_d1, ncell));
-    HIP_TRY(c, dalloc(&c->pa_d2, ncell));
-    HIP_TRY(c, dalloc(&c->pa_wanted, nlin + 1));
-    HIP_TRY(c, dalloc(&c->pa_wscan, nlin + 1));
-    HIP_TRY(c, dalloc(&c->pa_cnt, 32));
+    HIP_TRY(c, dalloc(c, &c->pa_cflag, ncell));
+    HIP_TRY(c, dalloc(c, &c->pa_d1, ncell));
+    HIP_TRY(c, dalloc(c, &c->pa_d2, ncell));
+    HIP_TRY(c, dalloc(c, &c->pa_wanted, nlin + 1));
+    HIP_TRY(c, dalloc(c, &c->pa_wscan, nlin + 1));
+    HIP_TRY(c, dalloc(c, &c->pa_cnt, 32));
   }
   // the coarsening and refill stages write volumes: start from 1.0 where none were given
   if (!c->has_vol && (cfg->gas_particle_coarsening || cfg->liquid_particle_coarsening || cfg->liquid_particle_refill)) {
@@ -207,7 +207,7 @@ int run_adaptivity(pf_ctx* c, const pf_adapt_cfg* cfg, pf_adapt_stats* out) {
     if (st) return st;
     hipFree(c->rank);
     c->rank = nullptr;
-    HIP_TRY(c, dalloc(&c->rank, cap));
+    HIP_TRY(c, dalloc(c, &c->rank, cap));
     c->pcap = cap;
   } else {
     std::swap(c->pa, c->pb);

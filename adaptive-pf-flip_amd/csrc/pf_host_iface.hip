@@ -15,8 +15,8 @@ constexpr int kIfaceFields = 9;
 int iface_fields(pf_ctx* c, const pf_phase* ph, IfaceArgs& a, bool mr) {
   const long long n = c->dc.nblocks * kBlockVol;
   if (!c->iface) {
-    HIP_TRY(c, dalloc(&c->iface, n * kIfaceFields));
-    HIP_TRY(c, dalloc(&c->iface_bad, 1));
+    HIP_TRY(c, dalloc(c, &c->iface, n * kIfaceFields));
+    HIP_TRY(c, dalloc(c, &c->iface_bad, 1));
   }
   a.dc = c->dc; a.du = c->du; a.dv = c->dv; a.dw = c->dw;
   a.g = c->geom;

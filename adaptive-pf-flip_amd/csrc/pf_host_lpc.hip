@@ -9,29 +9,30 @@ namespace {
 // partial sums of a layer's weight gradient (three workgroups each), and of the head's
 constexpr int kLpcWgradParts = 256, kLpcHeadParts = 1024;
 
-int lpc_grow(pf_lpc* L, long long nt, bool train) {
+// c: the context of the call, or null
+int lpc_grow(pf_lpc* L, pf_ctx* c, long long nt, bool train) {
   if (nt > L->cap) {
     dfree(L->X); dfree(L->h1); dfree(L->h2); dfree(L->o); dfree(L->tmax);
-    HIP_TRY(L, dalloc(&L->X, nt * kHaloVol * 4));
-    HIP_TRY(L, dalloc(&L->h1, nt * kTileVol * 16));
-    HIP_TRY(L, dalloc(&L->h2, nt * kTileVol * 32));
-    HIP_TRY(L, dalloc(&L->o, nt * kTileVol));
-    HIP_TRY(L, dalloc(&L->tmax, nt * 8));
+    HIP_TRY(L, dalloc(c, &L->X, nt * kHaloVol * 4));
+    HIP_TRY(L, dalloc(c, &L->h1, nt * kTileVol * 16));
+    HIP_TRY(L, dalloc(c, &L->h2, nt * kTileVol * 32));
+    HIP_TRY(L, dalloc(c, &L->o, nt * kTileVol));
+    HIP_TRY(L, dalloc(c, &L->tmax, nt * 8));
     L->cap = nt;
   }
   if (train && nt > L->cap_train) {
     dfree(L->h3); dfree(L->d3); dfree(L->d2); dfree(L->d1); dfree(L->go);
-    HIP_TRY(L, dalloc(&L->h3, nt * kTileVol * 16));
-    HIP_TRY(L, dalloc(&L->d3, nt * kTileVol * 16));
-    HIP_TRY(L, dalloc(&L->d2, nt * kTileVol * 32));
-    HIP_TRY(L, dalloc(&L->d1, nt * kTileVol * 16));
-    HIP_TRY(L, dalloc(&L->go, nt * kTileVol));
+    HIP_TRY(L, dalloc(c, &L->h3, nt * kTileVol * 16));
+    HIP_TRY(L, dalloc(c, &L->d3, nt * kTileVol * 16));
+    HIP_TRY(L, dalloc(c, &L->d2, nt * kTileVol * 32));
+    HIP_TRY(L, dalloc(c, &L->d1, nt * kTileVol * 16));
+    HIP_TRY(L, dalloc(c, &L->go, nt * kTileVol));
     L->cap_train = nt;
   }
   const long long need = (long long)kLpcWgradParts * kOffWH + (long long)kLpcHeadParts * kNWH;
   if (need > L->part_cap) {
     dfree(L->part);
-    HIP_TRY(L, dalloc(&L->part, need));
+    HIP_TRY(L, dalloc(c, &L->part, need));
     L->part_cap = need;
   }
   return PF_OK;
@@ -119,8 +120,8 @@ int lpc_cw_tiles(pf_ctx* c, const uint32_t* list, long long nlist) {
   const long long nall = (long long)c->ntx * c->nty * c->ntz;
   if (nall > c->ntiles_all) {
     dfree(c->tiles); dfree(c->tile_flags);
-    HIP_TRY(c, dalloc(&c->tiles, nall));
-    HIP_TRY(c, dalloc(&c->tile_flags, nall));
+    HIP_TRY(c, dalloc(c, &c->tiles, nall));
+    HIP_TRY(c, dalloc(c, &c->tile_flags, nall));
     c->ntiles_all = nall;
   }
   HIP_TRY(c, fill_u8(c->stream, c->tile_flags, 0, nall));
@@ -159,10 +160,10 @@ int lpc_cw_weights(pf_ctx* c, bool store) {
   if (!L) return fail(c, PF_ERR_STATE, "no network attached (pf_lpc_attach)");
   if (c->mg.empty()) return fail(c, PF_ERR_STATE, "learned preconditioner: the grid has no coarse level");
   const long long n1 = c->mg[0].d.nblocks * kBlockVol;
-  if (!c->mg_cs_net) HIP_TRY(c, dalloc(&c->mg_cs_net, n1));
+  if (!c->mg_cs_net) HIP_TRY(c, dalloc(c, &c->mg_cs_net, n1));
   HIP_TRY(c, fill_f32(c->stream, c->mg_cs_net, 1.f, n1));
   if (c->ntiles == 0) return PF_OK;
-  int st = lpc_grow(L, c->ntiles, store);
+  int st = lpc_grow(L, c, c->ntiles, store);
   if (st) return fail(c, st, "learned preconditioner: " + L->err);
   CwArgs a = lpc_cw_args(c);
   const unsigned slots = (unsigned)((c->ntiles + 7) / 8) * 8;
@@ -180,8 +181,8 @@ int lpc_cw_weights(pf_ctx* c, bool store) {
 int lpc_features_alloc(pf_ctx* c) {
   if (c->fbeta) return PF_OK;
   const long long ncell = c->dc.nblocks * kBlockVol;
-  HIP_TRY(c, dalloc(&c->fbeta, ncell));
-  HIP_TRY(c, dalloc(&c->fphi, ncell));
+  HIP_TRY(c, dalloc(c, &c->fbeta, ncell));
+  HIP_TRY(c, dalloc(c, &c->fphi, ncell));
   return PF_OK;
 }
 

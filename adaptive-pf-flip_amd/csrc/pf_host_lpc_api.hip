@@ -107,7 +107,7 @@ static int lpc_stage_input(pf_lpc* L, int64_t nt, const float* X) {
 
 int pf_lpc_forward_tiles(pf_lpc* L, int64_t nt, const float* X, float* O) {
   if (!L || !X || !O || nt <= 0) return PF_ERR_ARG;
-  int st = lpc_grow(L, nt, false);
+  int st = lpc_grow(L, nullptr, nt, false);
   if (!st) st = lpc_stage_input(L, nt, X);
   if (!st) st = lpc_forward(L, L->stream, nt, false, nullptr);
   if (st) return st;
@@ -118,7 +118,7 @@ int pf_lpc_forward_tiles(pf_lpc* L, int64_t nt, const float* X, float* O) {
 
 int pf_lpc_grad_tiles(pf_lpc* L, int64_t nt, const float* X, const float* gO, float* gW) {
   if (!L || !X || !gO || !gW || nt <= 0) return PF_ERR_ARG;
-  int st = lpc_grow(L, nt, true);
+  int st = lpc_grow(L, nullptr, nt, true);
   if (!st) st = lpc_stage_input(L, nt, X);
   if (!st) st = lpc_forward(L, L->stream, nt, true, nullptr);
   if (st) return st;
@@ -146,7 +146,7 @@ int pf_lpc_record(pf_ctx* c, int32_t max_snapshots, int32_t every) {
   c->snap_cap = 0;
   c->nsnap = 0;
   if (max_snapshots == 0) return PF_OK;
-  HIP_TRY(c, dalloc(&c->snaps, (long long)max_snapshots * c->dc.nblocks * kBlockVol));
+  HIP_TRY(c, dalloc(c, &c->snaps, (long long)max_snapshots * c->dc.nblocks * kBlockVol));
   c->snap_cap = max_snapshots;
   c->snap_every = std::max(every, 1);
   return PF_OK;
@@ -168,16 +168,16 @@ static int lpc_loss_eval(pf_lpc* L, pf_ctx* c, int k, bool learned, bool store, 
   const bool energy = L->objective == PF_LPC_OBJECTIVE_ENERGY;
   if (ncell > L->cell_cap) {
     dfree(L->zbuf); dfree(L->qbuf); dfree(L->gz); dfree(L->ebuf); dfree(L->rbuf);
-    HIP_TRY(L, dalloc(&L->zbuf, ncell));
-    HIP_TRY(L, dalloc(&L->qbuf, ncell));
-    HIP_TRY(L, dalloc(&L->gz, ncell));
-    HIP_TRY(L, dalloc(&L->ebuf, ncell));
-    HIP_TRY(L, dalloc(&L->rbuf, ncell));
+    HIP_TRY(L, dalloc(c, &L->zbuf, ncell));
+    HIP_TRY(L, dalloc(c, &L->qbuf, ncell));
+    HIP_TRY(L, dalloc(c, &L->gz, ncell));
+    HIP_TRY(L, dalloc(c, &L->ebuf, ncell));
+    HIP_TRY(L, dalloc(c, &L->rbuf, ncell));
     L->cell_cap = ncell;
   }
   if (n1 > L->l1_cap) {
     for (auto& p : L->l1) dfree(p);
-    for (auto& p : L->l1) HIP_TRY(L, dalloc(&p, n1));
+    for (auto& p : L->l1) HIP_TRY(L, dalloc(c, &p, n1));
     L->l1_cap = n1;
   }
   // stale values outside the system must stay finite: clear the work vectors

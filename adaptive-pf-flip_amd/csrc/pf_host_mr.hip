@@ -166,18 +166,18 @@ int mr_apply_layout(pf_ctx* c, std::vector<Leaf> lv) {
   const long long ncell = c->dc.nblocks * kBlockVol;
   const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
   if (!c->mr_lvl) {
-    HIP_TRY(c, dalloc(&c->mr_lvl, ncell));
+    HIP_TRY(c, dalloc(c, &c->mr_lvl, ncell));
     for (int a = 0; a < 3; ++a) {
-      HIP_TRY(c, dalloc(&c->mr_valid[a], fd[a]->nblocks * kBlockVol));
+      HIP_TRY(c, dalloc(c, &c->mr_valid[a], fd[a]->nblocks * kBlockVol));
     }
-    HIP_TRY(c, dalloc(&c->mr_info, c->dc.nblocks));
-    HIP_TRY(c, dalloc(&c->mr_cs, c->dc.nblocks));
-    HIP_TRY(c, dalloc(&c->mr_vol64, ncell));
-    HIP_TRY(c, dalloc(&c->mr_pfull, ncell));
+    HIP_TRY(c, dalloc(c, &c->mr_info, c->dc.nblocks));
+    HIP_TRY(c, dalloc(c, &c->mr_cs, c->dc.nblocks));
+    HIP_TRY(c, dalloc(c, &c->mr_vol64, ncell));
+    HIP_TRY(c, dalloc(c, &c->mr_pfull, ncell));
   }
   if ((long long)lv.size() > c->mr_leaves_cap) {
     dfree(c->mr_leaves_dev);
-    HIP_TRY(c, dalloc(&c->mr_leaves_dev, 4 * (long long)lv.size()));
+    HIP_TRY(c, dalloc(c, &c->mr_leaves_dev, 4 * (long long)lv.size()));
     c->mr_leaves_cap = (long long)lv.size();
   }
   c->mr_leaves.assign(4 * lv.size(), 0);
@@ -218,7 +218,7 @@ int mr_dynamic(pf_ctx* c, const pf_mr_refine_cfg* rc) {
   const Geom& g = c->geom;
   const int lim[3] = {g.nx, g.ny, g.nz};
   // the box buffers belong to refinement, which may run before any layout exists
-  if (!c->mr_bbox) HIP_TRY(c, dalloc(&c->mr_bbox, 16));
+  if (!c->mr_bbox) HIP_TRY(c, dalloc(c, &c->mr_bbox, 16));
   if (!c->mr_bbox_host) HIP_TRY(c, hipHostMalloc((void**)&c->mr_bbox_host, sizeof(int) * 16));
   if (c->np > 0 && !c->pa.x) return fail(c, PF_ERR_STATE, "particle buffers missing");
   HIP_TRY(c, fill_u32(c->stream, reinterpret_cast<uint32_t*>(c->mr_bbox), 0x7fffffffu, 12));
@@ -400,7 +400,7 @@ int mr_reference_solve(pf_ctx* c, const pf_mr_solve_cfg& cf, unsigned G, const V
       dfree(c->mrc);
       c->mrc = nullptr;
       c->mrc_cap = 0;
-      HIP_TRY(c, dalloc(&c->mrc, cg.nc * 6));
+      HIP_TRY(c, dalloc(c, &c->mrc, cg.nc * 6));
       c->mrc_cap = cg.nc * 6;
     }
     Vc = c->mrc;

@@ -71,8 +71,8 @@ int pf_mr_scene_bubbles(pf_ctx* c, uint64_t seed, int32_t nb, int32_t band, floa
   const unsigned grid = (unsigned)((nl + 3) / 4);
   uint32_t* cnt = nullptr;
   long long* off = nullptr;
-  HIP_TRY(c, dalloc(&cnt, nl));
-  if (hipMalloc((void**)&off, sizeof(long long) * (size_t)nl) != hipSuccess) {
+  HIP_TRY(c, dalloc(c, &cnt, nl));
+  if (dalloc(c, &off, nl) != hipSuccess) {
     dfree(cnt);
     return fail(c, PF_ERR_HIP, "pf_mr_scene_bubbles: allocation failed");
   }

@@ -15,15 +15,15 @@ int grow_particles(pf_ctx* c, long long n, bool vol) {
       hipFree(b->x); hipFree(b->y); hipFree(b->z); hipFree(b->u); hipFree(b->v); hipFree(b->w);
       hipFree(b->type); hipFree(b->id); hipFree(b->vol);
       *b = PBuf{};
-      HIP_TRY(c, dalloc(&b->x, cap)); HIP_TRY(c, dalloc(&b->y, cap)); HIP_TRY(c, dalloc(&b->z, cap));
-      HIP_TRY(c, dalloc(&b->u, cap)); HIP_TRY(c, dalloc(&b->v, cap)); HIP_TRY(c, dalloc(&b->w, cap));
-      HIP_TRY(c, dalloc(&b->type, cap)); HIP_TRY(c, dalloc(&b->id, cap));
+      HIP_TRY(c, dalloc(c, &b->x, cap)); HIP_TRY(c, dalloc(c, &b->y, cap)); HIP_TRY(c, dalloc(c, &b->z, cap));
+      HIP_TRY(c, dalloc(c, &b->u, cap)); HIP_TRY(c, dalloc(c, &b->v, cap)); HIP_TRY(c, dalloc(c, &b->w, cap));
+      HIP_TRY(c, dalloc(c, &b->type, cap)); HIP_TRY(c, dalloc(c, &b->id, cap));
     }
-    if (vol && !b->vol) HIP_TRY(c, dalloc(&b->vol, cap));
+    if (vol && !b->vol) HIP_TRY(c, dalloc(c, &b->vol, cap));
   }
   if (n > c->pcap) {
     hipFree(c->rank);
-    HIP_TRY(c, dalloc(&c->rank, cap));
+    HIP_TRY(c, dalloc(c, &c->rank, cap));
     c->pcap = cap;
   }
   return PF_OK;
@@ -57,7 +57,7 @@ int ensure_binned(pf_ctx* c) {
     const long long cap = c->np / (kRankMax + 1) + 1;
     if (cap > c->crowd_cap) {
       dfree(c->crowd_list);
-      HIP_TRY(c, dalloc(&c->crowd_list, cap));
+      HIP_TRY(c, dalloc(c, &c->crowd_list, cap));
       c->crowd_cap = cap;
     }
     HIP_TRY(c, fill_u32(c->stream, c->u32_dev + 16, 0u, 1));
@@ -226,7 +226,7 @@ int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double d
   const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
   const bool pairs = !g2p && c->np >= (long long)g.nx * g.ny * g.nz;
   for (int ax = 0; ax < 3; ++ax) {
-    if ((g2p || pairs) && !c->g2p_quad[ax]) HIP_TRY(c, dalloc(&c->g2p_quad[ax], fd[ax]->nblocks * kBlockVol));
+    if ((g2p || pairs) && !c->g2p_quad[ax]) HIP_TRY(c, dalloc(c, &c->g2p_quad[ax], fd[ax]->nblocks * kBlockVol));
     a.field[ax] = g2p || pairs ? static_cast<const void*>(c->g2p_quad[ax]) : c->f[F_U + ax];
   }
   // the G2P reduces the max speed of the velocities it writes (the next CFL scan's value)

@@ -29,8 +29,8 @@ int pf_write_render_cache(pf_ctx* c, const char* path, const pf_render_frame* m,
   const long long ncell = c->dc.nblocks * kBlockVol;
   // the cell phase field, then the field and the markers to the host
   if (!c->iface) {
-    HIP_TRY(c, dalloc(&c->iface, ncell * kIfaceFields));
-    HIP_TRY(c, dalloc(&c->iface_bad, 1));
+    HIP_TRY(c, dalloc(c, &c->iface, ncell * kIfaceFields));
+    HIP_TRY(c, dalloc(c, &c->iface_bad, 1));
   }
   IfaceArgs a;
   a.dc = c->dc; a.du = c->du; a.dv = c->dv; a.dw = c->dw;

@@ -70,18 +70,18 @@ int mg_alloc(pf_ctx* c) {
     const long long n = b.d.nblocks * kBlockVol;
     float** arrs[8] = {&b.cd, &b.cx, &b.cy, &b.cz, &b.inv, &b.x, &b.r, &b.t};
     for (float** a : arrs)
-      if (e == hipSuccess) e = dalloc(a, n);
+      if (e == hipSuccess) e = dalloc(c, a, n);
     for (auto& p : b.h)
-      if (e == hipSuccess) e = dalloc(&p, n);
-    if (e == hipSuccess) e = dalloc(&b.unscale, 2);
+      if (e == hipSuccess) e = dalloc(c, &p, n);
+    if (e == hipSuccess) e = dalloc(c, &b.unscale, 2);
     levels.push_back(b);
   }
   const long long n0 = c->dc.nblocks * kBlockVol;
-  if (e == hipSuccess) e = dalloc(&t0, n0);
+  if (e == hipSuccess) e = dalloc(c, &t0, n0);
   for (auto& p : h)
-    if (e == hipSuccess) e = dalloc(&p, n0);
-  if (e == hipSuccess) e = dalloc(&mx, 2 * kMaxPartials);
-  if (e == hipSuccess) e = dalloc(&unscale, 2);
+    if (e == hipSuccess) e = dalloc(c, &p, n0);
+  if (e == hipSuccess) e = dalloc(c, &mx, 2 * kMaxPartials);
+  if (e == hipSuccess) e = dalloc(c, &unscale, 2);
   if (e != hipSuccess) {
     release();
     return fail(c, PF_ERR_NOMEM, std::string("multigrid levels: ") + hipGetErrorString(e));
@@ -600,7 +600,7 @@ int cg_load(pf_ctx* c, CgState& g, VecArgs va, unsigned G, const double* r_src, 
 
 int cg_start(pf_ctx* c, CgState& g, const VecArgs& va, unsigned G, const double* r_src, double delta2,
              double tol2_abs, int budget, int between) {
-  if (!c->cgq) HIP_TRY(c, dalloc(&c->cgq, c->dc.nblocks * kBlockVol));
+  if (!c->cgq) HIP_TRY(c, dalloc(c, &c->cgq, c->dc.nblocks * kBlockVol));
   g.cur = g.par = 0;
   hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(1), 0, c->stream, c->sc, 1, delta2, tol2_abs, budget, between);
   return cg_load(c, g, va, G, r_src, true);
@@ -781,8 +781,8 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     c->mr_detail.coarse_preconditioner_auto_disable_iteration = -1;
   }
   if (refmode) {
-    if (!c->mrf) HIP_TRY(c, dalloc(&c->mrf, (long long)kMrfVectors * c->dc.nblocks * kBlockVol));
-    if (!c->mr_pin_dev) HIP_TRY(c, dalloc(&c->mr_pin_dev, 1));
+    if (!c->mrf) HIP_TRY(c, dalloc(c, &c->mrf, (long long)kMrfVectors * c->dc.nblocks * kBlockVol));
+    if (!c->mr_pin_dev) HIP_TRY(c, dalloc(c, &c->mr_pin_dev, 1));
     if (!c->mr_pin_host) HIP_TRY(c, hipHostMalloc((void**)&c->mr_pin_host, sizeof(long long)));
     HIP_TRY(c, fill_u32(c->stream, reinterpret_cast<uint32_t*>(c->mr_pin_dev), 0xffffffffu, 2));
   }
@@ -800,7 +800,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
       for (int a = 0; a < 3; ++a) {
         const long long n = fd[a]->nblocks * kBlockVol;
-        if (!c->mr_cf64[a]) HIP_TRY(c, dalloc(&c->mr_cf64[a], n));
+        if (!c->mr_cf64[a]) HIP_TRY(c, dalloc(c, &c->mr_cf64[a], n));
         HIP_TRY(c, fill_f64(c->stream, c->mr_cf64[a], 0.0, n));
         ma.cf64[a] = c->mr_cf64[a];
       }
@@ -1276,7 +1276,7 @@ int pf_mg_set_correction_weights(pf_ctx* c, const float* w, int64_t n) {
           return fail(c, PF_ERR_ARG, "pf_mg_set_correction_weights: weights must be positive and finite");
         s[(size_t)bm_index(d1, i, j, k)] = std::sqrt(v);
       }
-  if (!c->mg_cs) HIP_TRY(c, dalloc(&c->mg_cs, d1.nblocks * kBlockVol));
+  if (!c->mg_cs) HIP_TRY(c, dalloc(c, &c->mg_cs, d1.nblocks * kBlockVol));
   HIP_TRY(c, hipMemcpyAsync(c->mg_cs, s.data(), sizeof(float) * s.size(), hipMemcpyHostToDevice, c->stream));
   HIP_TRY(c, hipStreamSynchronize(c->stream));
   return PF_OK;
