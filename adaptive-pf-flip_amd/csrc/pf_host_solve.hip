@@ -600,7 +600,6 @@ int cg_load(pf_ctx* c, CgState& g, VecArgs va, unsigned G, const double* r_src, 
 
 int cg_start(pf_ctx* c, CgState& g, const VecArgs& va, unsigned G, const double* r_src, double delta2,
              double tol2_abs, int budget, int between) {
-  if (!c->cgq) HIP_TRY(c, dalloc(c, &c->cgq, c->dc.nblocks * kBlockVol));
   g.cur = g.par = 0;
   hipLaunchKernelGGL(k_cg_begin, dim3(1), dim3(1), 0, c->stream, c->sc, 1, delta2, tol2_abs, budget, between);
   return cg_load(c, g, va, G, r_src, true);
@@ -989,7 +988,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     // the buffer-addressed kernels take 32-bit byte offsets: arrays below 2 GiB
     const bool spmv_buffers = c->dc.nblocks * kBlockVol * 4 < (1LL << 31);
     CgState cg;
-    const bool one_kernel = mr || spmv_buffers;   // the Jacobi iteration as k_cg_iter or k_mr_cg_iter
+    bool one_kernel = mr || spmv_buffers;         // the Jacobi iteration as k_cg_iter or k_mr_cg_iter
     const unsigned GL = mr ? cg_grid(npb) : G;    // workgroups of the load, one partial each
     // r32 from the FP64 residual, x32 = 0 (and p = 0)
     auto load = [&](const double* src, float* p) {
@@ -1002,6 +1001,11 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     };
     // (re)start: r32 from r64, x32 = 0, p = 0, z = M(r)
     auto start = [&](int budget) -> int {
+      if (one_kernel && !learned && !c->cgq) {
+        const hipError_t e = dalloc(c, &c->cgq, ncell);
+        if (mr) HIP_TRY(c, e);
+        one_kernel = e == hipSuccess;  // (the separate kernels need no second A p)
+      }
       if (one_kernel && !learned) return cg_start(c, cg, va, G, r_src, delta * delta, tol2_abs, budget, between);
       load(r_src, c->pA);
       LAUNCH_CHECK(c);
