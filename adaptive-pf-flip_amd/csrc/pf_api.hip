@@ -229,6 +229,7 @@ int pf_destroy(pf_ctx* c) {
   dfree(c->cgq);
   hipFree(c->u32_dev); hipFree(c->esc_dev); hipFree(c->vmax_dev);
   for (auto* q : c->g2p_quad) hipFree(q);
+  for (auto* q : c->g2p_pair) hipFree(q);
   hipFree(c->scan_tiles); hipFree(c->stage_f);
   for (int e = 0; e <= PF_NSTAGES; ++e)
     if (c->ev[e]) hipEventDestroy(c->ev[e]);

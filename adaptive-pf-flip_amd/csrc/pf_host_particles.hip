@@ -204,6 +204,22 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   return PF_OK;
 }
 
+// Room for the velocity pairs of an advection without G2P: the G2P's quads where it has
+// allocated them, else arrays of their own (8 B a face).  False without the memory: the plain
+// gathers then, the same bits.
+bool g2p_pairs(pf_ctx* c, const Dims* const (&fd)[3], float2* (&pair)[3]) {
+  if (c->g2p_quad[2]) {
+    for (int ax = 0; ax < 3; ++ax) pair[ax] = reinterpret_cast<float2*>(c->g2p_quad[ax]);
+    return true;
+  }
+  for (int ax = 0; ax < 3 && !c->g2p_no_pairs; ++ax) {
+    if (!c->g2p_pair[ax]) c->g2p_no_pairs = dalloc(&c->g2p_pair[ax], fd[ax]->nblocks * kBlockVol) != hipSuccess;
+    pair[ax] = c->g2p_pair[ax];
+  }
+  if (c->g2p_no_pairs)
+    for (auto& q : c->g2p_pair) dfree(q);
+  return !c->g2p_no_pairs;
+}
 
 int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double dt, int order) {
   if (c->np == 0) return PF_OK;
@@ -224,10 +240,13 @@ int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double d
   a.esc = c->esc_dev;
   a.vmax_bits = reinterpret_cast<uint32_t*>(c->vmax_dev);
   const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
-  const bool pairs = !g2p && c->np >= (long long)g.nx * g.ny * g.nz;
+  float2* pair[3] = {nullptr, nullptr, nullptr};
+  const bool pairs = !g2p && c->np >= (long long)g.nx * g.ny * g.nz && g2p_pairs(c, fd, pair);
+  if (g2p && !c->g2p_quad[2])
+    for (auto& q : c->g2p_pair) dfree(q);  // (the quads hold pairs too)
   for (int ax = 0; ax < 3; ++ax) {
-    if ((g2p || pairs) && !c->g2p_quad[ax]) HIP_TRY(c, dalloc(c, &c->g2p_quad[ax], fd[ax]->nblocks * kBlockVol));
-    a.field[ax] = g2p || pairs ? static_cast<const void*>(c->g2p_quad[ax]) : c->f[F_U + ax];
+    if (g2p && !c->g2p_quad[ax]) HIP_TRY(c, dalloc(c, &c->g2p_quad[ax], fd[ax]->nblocks * kBlockVol));
+    a.field[ax] = g2p ? static_cast<const void*>(c->g2p_quad[ax]) : (pairs ? static_cast<const void*>(pair[ax]) : c->f[F_U + ax]);
   }
   // the G2P reduces the max speed of the velocities it writes (the next CFL scan's value)
   if (g2p) HIP_TRY(c, fill_u32(c->stream, reinterpret_cast<uint32_t*>(c->vmax_dev), 0u, 1));
@@ -241,8 +260,7 @@ int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double d
         hipLaunchKernelGGL(k_pack_quad, gp, dim3(256), 0, c->stream, *fd[ax], c->f[F_U + ax], c->f[F_SU + ax],
                            c->g2p_quad[ax]);
       else if (pairs)
-        hipLaunchKernelGGL(k_pack_pair, gp, dim3(256), 0, c->stream, *fd[ax], c->f[F_U + ax],
-                           reinterpret_cast<float2*>(c->g2p_quad[ax]));
+        hipLaunchKernelGGL(k_pack_pair, gp, dim3(256), 0, c->stream, *fd[ax], c->f[F_U + ax], pair[ax]);
     }
     if (g2p)
       hipLaunchKernelGGL(k_g2p_advect<float4>, dim3(grid), dim3(256), 0, c->stream, a);

@@ -178,6 +178,8 @@ struct Ctx {
   int32_t* esc_dev = nullptr;       // 8 clamp counters
   float* vmax_dev = nullptr;        // max particle speed (as float bits via atomicMax)
   float4* g2p_quad[3] = {nullptr, nullptr, nullptr};  // per face (vel, saved) of it and of its +x neighbour (G2P)
+  float2* g2p_pair[3] = {nullptr, nullptr, nullptr};  // vel alone (advection of a context without the quads)
+  bool g2p_no_pairs = false;                          // no memory for them
   bool vmax_valid = false;          // vmax_dev holds the max speed of the current velocities
 
   // scan scratch

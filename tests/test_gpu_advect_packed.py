@@ -5,6 +5,7 @@ wall and past it (clamped), on ragged grids.
 """
 import numpy as np
 import pytest
+import torch
 
 import pfflip_amd as G
 
@@ -38,3 +39,26 @@ def test_pairs_equal_plain_gathers(dims, order):
         out.append([q[:few] for q in ctx.download()[:3]])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+def test_pairs_take_their_own_size():
+    """advection alone holds 8 bytes a face, not the G2P's 16; a G2P after it the quads alone,
+    and advection then goes on in them"""
+    n = 128
+    ctx = G.Context(n, n, n, 1.0 / n)
+    r = np.random.default_rng(3)
+    p = r.uniform(0.05, 0.95, (n ** 3, 3)).astype(np.float32)
+    ctx.upload(*(np.ascontiguousarray(p[:, a]) for a in range(3)))
+    ctx.set_field(G.FIELD_U, r.normal(size=(n, n, n + 1)).astype(np.float32))
+    first = torch.cuda.mem_get_info()[0]
+    ctx.advect(0.1 / n, 2)
+    pairs = first - torch.cuda.mem_get_info()[0]
+    moved = ctx.download()[0]
+    faces = 3 * n * n * (n + 4)
+    assert pairs < 10 * faces
+    ctx.upload(*(np.ascontiguousarray(p[:, a]) for a in range(3)))
+    ctx.g2p(0.95, 0.9)
+    assert first - torch.cuda.mem_get_info()[0] < 18 * faces
+    ctx.advect(0.1 / n, 2)
+    assert first - torch.cuda.mem_get_info()[0] < 18 * faces
+    assert np.array_equal(moved, ctx.download()[0])
