@@ -7,11 +7,14 @@
 namespace {
 
 // partial sums of a layer's weight gradient (three workgroups each), and of the head's
-constexpr int kLpcWgradParts = 256, kLpcHeadParts = 1024;
+int lpc_wgrad_parts(long long nt) { return (int)std::min<long long>(256, nt * 8); }
+int lpc_head_parts(long long nt) { return (int)std::min<long long>(1024, nt * kTileVol / 16); }
 
 // c: the context of the call, or null
 int lpc_grow(pf_lpc* L, pf_ctx* c, long long nt, bool train) {
+  // (a capacity stands only once all its arrays do)
   if (nt > L->cap) {
+    L->cap = 0;
     dfree(L->X); dfree(L->h1); dfree(L->h2); dfree(L->o); dfree(L->tmax);
     HIP_TRY(L, dalloc(c, &L->X, nt * kHaloVol * 4));
     HIP_TRY(L, dalloc(c, &L->h1, nt * kTileVol * 16));
@@ -21,6 +24,7 @@ int lpc_grow(pf_lpc* L, pf_ctx* c, long long nt, bool train) {
     L->cap = nt;
   }
   if (train && nt > L->cap_train) {
+    L->cap_train = 0;
     dfree(L->h3); dfree(L->d3); dfree(L->d2); dfree(L->d1); dfree(L->go);
     HIP_TRY(L, dalloc(c, &L->h3, nt * kTileVol * 16));
     HIP_TRY(L, dalloc(c, &L->d3, nt * kTileVol * 16));
@@ -29,8 +33,9 @@ int lpc_grow(pf_lpc* L, pf_ctx* c, long long nt, bool train) {
     HIP_TRY(L, dalloc(c, &L->go, nt * kTileVol));
     L->cap_train = nt;
   }
-  const long long need = (long long)kLpcWgradParts * kOffWH + (long long)kLpcHeadParts * kNWH;
-  if (need > L->part_cap) {
+  const long long need = (long long)lpc_wgrad_parts(nt) * kOffWH + (long long)lpc_head_parts(nt) * kNWH;
+  if (train && need > L->part_cap) {
+    L->part_cap = 0;
     dfree(L->part);
     HIP_TRY(L, dalloc(c, &L->part, need));
     L->part_cap = need;
@@ -64,11 +69,11 @@ int lpc_forward(pf_lpc* L, hipStream_t s, long long nt, bool store_h3, const int
   return PF_OK;
 }
 
-// partials of the layer at offset OFF of the weights, to L->part from kLpcWgradParts * OFF
+// np partials of the layer at offset OFF of the weights, to L->part from np * OFF
 template <int CIN, int COUT, bool PADDED, int OFF>
 int lpc_wgrad(pf_lpc* L, hipStream_t s, const __bf16* in, const __bf16* g, long long nt, int np) {
   hipLaunchKernelGGL((k_lpc_wgrad<CIN, COUT, PADDED>), dim3(3 * np), dim3(192), 0, s, in, g, nt,
-                     L->part + (long long)kLpcWgradParts * OFF);
+                     L->part + (long long)np * OFF);
   HIP_TRY(L, hipGetLastError());
   return PF_OK;
 }
@@ -76,10 +81,9 @@ int lpc_wgrad(pf_lpc* L, hipStream_t s, const __bf16* in, const __bf16* g, long 
 // L->grad = d(sum o * go)/dw, from the activations of the last lpc_forward(store_h3)
 int lpc_backward(pf_lpc* L, hipStream_t s, long long nt) {
   const long long ncells = nt * kTileVol;
-  const int hg = (int)std::min<long long>(kLpcHeadParts, (ncells + 15) / 16);
-  const int np = (int)std::min<long long>(kLpcWgradParts, nt * 8);
+  const int hg = lpc_head_parts(nt), np = lpc_wgrad_parts(nt);
   hipLaunchKernelGGL(k_lpc_head_bwd, dim3(hg), dim3(256), 0, s, L->h3, L->go, L->bf.wh, ncells, L->d3,
-                     L->part + (long long)kLpcWgradParts * kOffWH);
+                     L->part + (long long)np * kOffWH);
   const dim3 grid((unsigned)(nt * 16));
   ConvArgs a{};
   a.ntiles = nt;
@@ -95,7 +99,7 @@ int lpc_backward(pf_lpc* L, hipStream_t s, long long nt) {
   LpcParts p;
   const int off[5] = {kOffW1, kOffW2, kOffW3, kOffWH, kNW};
   for (int l = 0; l < 4; ++l) {
-    p.part[l] = L->part + (long long)kLpcWgradParts * off[l];
+    p.part[l] = L->part + (long long)np * off[l];
     p.nparts[l] = l < 3 ? np : hg;
     p.off[l] = off[l];
   }

@@ -10,6 +10,7 @@ workgroups take two).
 """
 import numpy as np
 import pytest
+import torch
 
 import lpc_oracle as LO
 import pfflip_amd as G
@@ -39,3 +40,13 @@ def test_integer_gradients_are_exact(nt):
         np.abs(ref[o:o + n]).max() > 0 for o, n in zip(np.cumsum([0, *LO.SIZES[:3]]), LO.SIZES))
     assert np.array_equal(net.forward_tiles(X), out.astype(np.float32))
     assert np.array_equal(net.grad_tiles(X, gO), ref.astype(np.float32))
+
+
+def test_one_tile_takes_one_tile_of_memory():
+    """activations and gradients of a tile take about 1.2 MB, its 8 partials a layer 2 MB"""
+    _, X, gO = _case(1, 3)
+    G.LearnedPreconditioner(seed=1).grad_tiles(X, gO)  # (what the kernels' first launch takes)
+    net = G.LearnedPreconditioner(seed=1)
+    free = torch.cuda.mem_get_info()[0]
+    net.grad_tiles(X, gO)
+    assert free - torch.cuda.mem_get_info()[0] < 24 << 20
