@@ -341,7 +341,9 @@ __global__ void __launch_bounds__(192) k_lpc_wgrad(const __bf16* __restrict__ in
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int tap = CIN >= 16 ? dx : q, ci = CIN >= 16 ? mt * 16 + 4 * q + i : i;
-          if (tap < 3) dst[(tap * CIN + ci) * COUT + nb * 16 + m] = (double)sum[mt][dx][nb][i] + (double)low[mt][dx][nb][i];
+          // (past FP32's range the two-sum's rest is NaN: the sum stands alone)
+          const double hi = sum[mt][dx][nb][i], rest = isfinite(hi) ? low[mt][dx][nb][i] : 0.f;
+          if (tap < 3) dst[(tap * CIN + ci) * COUT + nb * 16 + m] = hi + rest;
         }
 }
 

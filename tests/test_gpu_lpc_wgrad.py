@@ -50,3 +50,21 @@ def test_one_tile_takes_one_tile_of_memory():
     free = torch.cuda.mem_get_info()[0]
     net.grad_tiles(X, gO)
     assert free - torch.cuda.mem_get_info()[0] < 24 << 20
+
+
+@pytest.mark.parametrize("e", [112, 117, 123])
+def test_gradients_past_the_range_of_float32_are_infinite(e):
+    """output gradients of 2^e: sums past FP32's range in the last sum alone (some stay below,
+    exact), in a workgroup's, in a chain; nothing is negative, so they come out as Inf and
+    not as NaN.  (The last layer's: further down 0 times Inf is NaN in the gradient itself.)"""
+    w, X, gO = _case(3, 5)
+    w, gO = np.abs(w), np.abs(gO)
+    net = G.LearnedPreconditioner(seed=1)
+    net.set_weights(w)
+    _, cache = LO.forward(X, w.astype(np.float64), bf16=True)
+    layer = slice(sum(LO.SIZES[:2]), sum(LO.SIZES[:3]))
+    ref = LO.backward(cache, gO, w.astype(np.float64), bf16=True)[layer]
+    assert ref.max() < 2 ** 24 and (ref >= 2 ** 16).any() and (ref < 2 ** 16).any()
+    with np.errstate(over="ignore"):
+        want = (ref * 2.0 ** e).astype(np.float32)
+    assert np.array_equal(net.grad_tiles(X, gO * np.float32(2.0 ** e))[layer], want)
