@@ -353,8 +353,8 @@ __global__ void __launch_bounds__(256) k_cg_iter(CgArgs a) {
       v[CG_QDQ] += qd * (double)L.inv.v[i] * qd;
       v[CG_RR] += rd * rd;
     }
+    if (PRE) break;  // (up to 512 workgroups a wave has one slot)
     t0 += step;
-    if (PRE && t0 < e) load();
   }
   cg_store_sums(a, v, sh);
 }

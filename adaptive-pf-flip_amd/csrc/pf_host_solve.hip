@@ -587,7 +587,7 @@ int cg_load(pf_ctx* c, CgState& g, VecArgs va, unsigned G, const double* r_src, 
   if (c->mr) {
     g.nsums = (int)cg_grid(va.nlist);
     hipLaunchKernelGGL(k_mr_load, dim3((unsigned)g.nsums), dim3(256), 0, c->stream, va, mr_row_op(c), r_src, c->x32,
-                       cg_r(c, g.par), first ? cg_p(c, g.par) : nullptr, first ? cg_q(c, g.par) : nullptr, nullptr, 1);
+                       cg_r(c, g.par), first ? cg_p(c, g.par) : nullptr, first ? cg_q(c, g.par) : nullptr, 1);
     LAUNCH_CHECK(c);
     return PF_OK;
   }
@@ -994,7 +994,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     auto load = [&](const double* src, float* p) {
       if (mr)
         hipLaunchKernelGGL(k_mr_load, dim3(GL), dim3(256), 0, c->stream, va, mop, src, c->x32, c->r32, p,
-                           static_cast<float*>(nullptr), static_cast<const float*>(nullptr), 0);
+                           static_cast<float*>(nullptr), 0);
       else
         hipLaunchKernelGGL(k_pcg_load, dim3(GL), dim3(256), 0, c->stream, va, src, c->x32, c->r32, c->z32, p,
                            c->invd32, learned ? 1 : 0);

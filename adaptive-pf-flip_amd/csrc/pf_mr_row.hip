@@ -351,21 +351,21 @@ __global__ void __launch_bounds__(256) k_mr_update(VecArgs a, const uint8_t* __r
   block_reduce_store<2>(v, mx, a.part, kMaxPartials);
 }
 
-// r = (float)r64, x = 0 (FIRST: p = q = 0 too); partial r.z with z = D^-1 r, or with the
-// given z (slot CG_RZ), and r.r (slot CG_RR); slots as k_cg_load's, or 0 and 1
+// r = (float)r64, x = 0 and, where given, p = 0 and q = 0; partial r.z with z = D^-1 r
+// (slot CG_RZ) and r.r (slot CG_RR) as k_cg_load, or in slots 0 and 1
 __global__ void __launch_bounds__(256) k_mr_load(VecArgs a, MrRowOp op, const double* __restrict__ r64,
                                                  float* __restrict__ x, float* __restrict__ r, float* __restrict__ p,
-                                                 float* __restrict__ q, const float* __restrict__ z, int cg) {
+                                                 float* __restrict__ q, int cg) {
   double rz = 0.0, rr = 0.0;
   FOR_MR_ROWS(a, op, R) {
     const Row4<double> rd = mr_own(r64, R);
-    const Row4<float> other = z ? mr_own(z, R) : mr_own(op.inv, R);
+    const Row4<float> inv = mr_own(op.inv, R);
     Row4<float> rf, zero = {{0.f, 0.f, 0.f, 0.f}};
     double s0 = 0.0, s1 = 0.0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       rf.v[i] = (float)rd.v[i];
-      s0 += (double)rf.v[i] * (double)(z ? other.v[i] : other.v[i] * rf.v[i]);
+      s0 += (double)rf.v[i] * (double)(inv.v[i] * rf.v[i]);
       s1 += (double)rf.v[i] * (double)rf.v[i];
     }
     mr_put(r, R, rf);

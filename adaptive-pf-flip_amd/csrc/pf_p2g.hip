@@ -643,7 +643,7 @@ __device__ inline void p2g_block(const P2GShared& a, const P2GField& fu, const P
 // ceil(3 n / 3072) rounds a third as long plus a tenth for ranking three times.
 constexpr uint32_t kP2GResident = 256 * 12;
 constexpr uint32_t kP2GSplitMost = 5 * kP2GResident;  // (past five rounds the last one matters little)
-__host__ __device__ inline bool p2g_split(uint32_t n) {
+inline bool p2g_split(uint32_t n) {
   const uint32_t whole = (n + kP2GResident - 1) / kP2GResident, third = (3 * n + kP2GResident - 1) / kP2GResident;
   return n <= kP2GSplitMost && 11 * third < 30 * whole;
 }
@@ -662,14 +662,12 @@ __global__ void __launch_bounds__(64) k_p2g_block(P2GShared a, P2GField fu, P2GF
   p2g_block<KT, F32, true>(a, fu, fv, fw, b, gridDim.y == 3 ? (int)blockIdx.y : -1);
 }
 
-// One launch per colour for larger grids, without the regions' memory.
+// One launch per colour, without the regions' memory: larger grids.
 template <int KT, bool F32>
 __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
   const uint32_t nblk = *a.count;
   if (blockIdx.x >= nblk) return;
-  const bool split = gridDim.y == 3 && p2g_split(nblk);
-  if (!split && blockIdx.y > 0) return;
-  p2g_block<KT, F32, false>(a, fu, fv, fw, a.list[blockIdx.x], split ? (int)blockIdx.y : -1);
+  p2g_block<KT, F32, false>(a, fu, fv, fw, a.list[blockIdx.x], -1);
 }
 
 // A wave per block of a face field: a node lies in the regions of at most two source
