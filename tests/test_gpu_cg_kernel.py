@@ -1,7 +1,7 @@
 """The Jacobi PCG iteration in one kernel (k_cg_iter) at the sizes where its layout can go
 wrong: one block, ragged ends, one list slot more or less than a workgroup's share, the
-change to the form that loads after the sums (more than 512 workgroups), and the
-iteration budget at a restart.
+change to the form that loads after the sums (more than 512 workgroups), several slots
+to a wave (more than 1024), and the iteration budget at a restart.
 
 Bars: the FP64 oracle's pressure where it is quick (1e-6, the bar of the other projection
 tests), and on larger open tanks the multigrid solve of the same system to a residual of
@@ -58,11 +58,24 @@ def test_matches_the_oracle(shape, kind):
         assert rel_err(ctx.field(f), g.dense(f)) < 1e-5
 
 
-# 18x18x18 blocks: 365 workgroups; 21^3: 579, past the change; 25 x 9 x 9 ragged
-@pytest.mark.parametrize("shape", [(72, 72, 72), (84, 83, 82), (101, 35, 34)])
-def test_matches_multigrid_on_larger_grids(shape):
+def _workgroups(ctx):
+    """of the iteration: sixteen listed blocks each, a multiple of 8, at most 1024"""
+    m = np.asarray(ctx.field(G.FIELD_MARKER)) == 1  # FLUID
+    m = np.pad(m.reshape(ctx.dims(G.FIELD_MARKER)[::-1]), [(0, -n % 4) for n in ctx.dims(G.FIELD_MARKER)[::-1]])
+    z, y, x = (n // 4 for n in m.shape)
+    listed = int(m.reshape(z, 4, y, 4, x, 4).any(axis=(1, 3, 5)).sum())
+    return min(-(-listed // 128) * 8, 1024)
+
+
+# up to 512 workgroups the row loads come before the sums, above after them; at the cap of
+# 1024 (17,576 blocks) some waves take two slots; ragged grids on each side
+@pytest.mark.parametrize("shape,groups", [((72, 72, 72), 224), ((84, 83, 82), 360), ((101, 35, 34), 88),
+                                          ((80, 133, 80), 504), ((82, 130, 81), 528), ((105, 171, 103), 1024)])
+def test_matches_multigrid_on_larger_grids(shape, groups):
     print(f"[cg] {shape}", flush=True)
     dx, ctx, _, _, gph = _context(shape, O.SCENE_BUBBLE)
+    ctx.mark_cells()
+    assert _workgroups(ctx) == groups
     faces = []
     for pre in (G.PRECOND_JACOBI, G.PRECOND_MULTIGRID):
         _grid_half(ctx, gph)
