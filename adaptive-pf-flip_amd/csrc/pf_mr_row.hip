@@ -136,10 +136,18 @@ template <typename T>
 __device__ inline Row4<T> mr_zrow(const T* __restrict__ a, const MrRow& R) {
   return mr_splat(mr_ld4(a + R.z), R.sz);
 }
-// a row's values back to its leaf cells' entries
+// a row's values back to its leaf cells' entries.  The two entries of a level-1 cell in a row
+// take the first one's value: the compiler may contract the arithmetic of a row's
+// entries differently, and values of one cell that differ by an ulp drift apart over a
+// solve (multigrid: 7e-7 of 4 in x64, a flux of 1.6e-5 left in the cells whose residual, formed
+// from all the entries, was 1e-12).  The cell's four lanes run the same instructions.
 template <typename T>
-__device__ inline void mr_put(T* __restrict__ a, const MrRow& R, const Row4<T>& v) {
+__device__ inline void mr_put(T* __restrict__ a, const MrRow& R, Row4<T> v) {
   if (!R.valid) return;
+  if (R.L == 1) {
+    v.v[1] = v.v[0];
+    v.v[3] = v.v[2];
+  }
   if (R.L < 2)
     mr_st4(a + R.own, v);
   else if (R.row == 0)

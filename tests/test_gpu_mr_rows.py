@@ -1,6 +1,7 @@
 """The multires operator by cell rows (pf_mr_row.hip) where its layout can go wrong: leaf
 cells clipped by a ragged domain, blocks of every level next to every other, a refined box
-at a corner, one refined block, no refinement at all.
+at a corner, one refined block, no refinement at all; many slots of blocks to a wave; and
+leaves that no row can hold.
 
 Bars: both fast solves (Jacobi PCG and multigrid), to a max residual of 1e-11, against the
 exact FP64 solution of the oracle's rows: those of the three-level tests, pressure within
@@ -131,3 +132,58 @@ def test_a_refused_solve_leaves_nothing_to_the_next():
         assert st.converged == 1
         out.append((st.iterations, ctx.field(G.FIELD_P)))
     assert out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dims,top,boxes,most", [
+    ((68, 72, 62), 54, ([16, 16, 16, 48, 40, 32], [24, 24, 16, 40, 40, 32]), 4096),
+    ((212, 232, 206), 214, ([48, 48, 48, 112, 96, 80], [64, 64, 48, 80, 80, 64]), 1 << 20)])
+def test_leaf_cells_balance(dims, top, boxes, most):
+    """What flows out of each leaf cell of three levels, summed from the faces, is zero to their
+    rounding (up to 96 faces, half an ulp each) and its volume times the residual, and the two fast solves
+    agree.  The second grid lists 135,000 blocks: waves take up to nine slots of four blocks
+    in the iterations and two in the cycle, the last ones ragged."""
+    dt, tol = 0.02, 1e-9
+    nx, ny, nz = dims
+    _, gph = _phase()
+    leaves = G.mr_layout_fine_box(*dims, level=2)
+    for b in boxes:
+        leaves = G.mr_layout_refine(*dims, leaves, b)
+    assert sorted(set(leaves[:, 0])) == [0, 1, 2]
+    level = np.zeros(dims[::-1], np.int8)
+    for L, bx, by, bz in leaves.tolist():
+        s = 4 << L
+        level[bz * s:(bz + 1) * s, by * s:(by + 1) * s, bx * s:(bx + 1) * s] = L
+    # a particle in every cell of 2^3 below the top, and in every fine cell of the finest box
+    f = boxes[1]
+    grids = [np.meshgrid(np.arange(1, nz - 1, 2), np.arange(1, top, 2), np.arange(1, nx - 1, 2), indexing="ij"),
+             np.meshgrid(*(np.arange(f[a], f[a + 3]) for a in (2, 1, 0)), indexing="ij")]
+    p = np.concatenate([np.stack([g[2].ravel(), g[1].ravel(), g[0].ravel()], 1) for g in grids]) + 0.5
+    r = np.random.default_rng(6)
+    v = r.normal(scale=0.3, size=p.shape)
+    t = (r.random(len(p)) < 0.2).astype(np.uint8)
+    ctx = G.MRContext(*dims, 1.0)
+    ctx.set_layout(leaves)
+    ctx.upload(*(np.ascontiguousarray(q, np.float32) for q in (*p.T, *v.T)), t)
+    got = []
+    for mode in (G.MR_SOLVE_FAST, G.MR_SOLVE_MULTIGRID):
+        _to_projection(ctx, gph, dt)
+        st = ctx.mr_project(gph, dt, G.mr_solve_cfg(20000, tol, 0.0, mode=mode))
+        assert st.converged == 1 and st.true_max_residual < tol and st.fallback_used == 0
+        faces = [np.asarray(ctx.field(f), np.float64).reshape(ctx.dims(f)[::-1]) for f in range(3)]
+        got.append((np.asarray(ctx.field(G.FIELD_P)), *faces))
+        fluid = np.asarray(ctx.field(G.FIELD_MARKER)).reshape(nz, ny, nx) == 1  # FLUID
+        listed = fluid[::4, ::4, ::4].sum()  # (a block's first cell is FLUID if one is)
+        assert listed > 131072 if most > 131072 else listed < most
+        out = sum(np.diff(a, axis=2 - f) for f, a in enumerate(faces))
+        ulp = 2.0 ** -24 * max(np.abs(a).max() for a in faces)
+        for L in range(3):
+            s = 1 << L
+            # (away from the walls, whose faces the rows leave out)
+            z, y, x = (slice(8, (n - 12) // 4 * 4) for n in dims[::-1])
+            a = out[z, y, x]
+            a = a.reshape(a.shape[0] // s, s, a.shape[1] // s, s, a.shape[2] // s, s).sum(axis=(1, 3, 5))
+            here = (level[z, y, x] == L)[::s, ::s, ::s] & fluid[z, y, x][::s, ::s, ::s]
+            assert here.sum() > 1000 and np.abs(a[here]).max() < 6 * 4 ** L * ulp + 8 ** L * tol, L
+    assert rel_err(got[0][0], got[1][0]) < 1e-6
+    for f in range(1, 4):
+        assert rel_err(got[0][f], got[1][f]) < 1e-5, f
