@@ -5,7 +5,7 @@
 // second.  Here a launch forms r, z, p and q = A p from the previous launch's, and the
 // sums p.q, r.z, z.q, q.D^-1 q and r.r in the same pass.  The next launch's alpha is
 // r.z / p.q as before, and the r.z after its update, which beta needs before r is formed,
-// comes from those sums exactly (r' = r - alpha q):
+// comes from those sums (r' = r - alpha q, but for the rounding of r' to FP32):
 //   r'.z' = r.z - 2 alpha z.q + alpha^2 q.D^-1 q
 // (in FP64; the next launch sums r'.z' itself, so nothing accumulates).  Recurring q
 // instead (Chronopoulos and Gear 1989, s = A r + beta s) drifts: a closed box at a
@@ -223,8 +223,6 @@ __device__ inline void cg_publish(const CgArgs& a, const SolveScalars& S) {
   __hip_atomic_store(a.word, 2 * a.seq + (S.done ? 1u : 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The list in slots of four blocks (one per 16 lanes of a wave), each XCD a contiguous
-// eighth.
 // The last launch's partial sums: every one that a thread adds is loaded before any is
 // waited for (a load of what other XCDs just wrote takes 1 to 2 us).
 __device__ inline void cg_fetch(const CgArgs& a, double (&w)[4][CG_SUMS]) {
@@ -284,10 +282,13 @@ struct CgLoads {
   float rxp, qxp, pxp, ixp, rxm, qxm, pxm, ixm;
 };
 
-// PRE: the first row's loads are issued before the sums are waited for, which hides
-// their latency (64^3: 7.8 -> 7.3 us with the sums as they were then) for 170 registers, two workgroups to a CU, instead
-// of 91: better while every workgroup is resident at once, so up to 512 of them (96^3,
-// 864 workgroups: 13.9 us without, 17.4 with; 128^3: 25.9 and 26.5).
+// The list goes in slots of four blocks (one per 16 lanes of a wave), each XCD a contiguous
+// eighth.
+// PRE: a wave's one row loads are issued before the sums are waited for, which hides their
+// latency for 170 registers, two workgroups to a CU, instead of 91.  No better once the
+// workgroups are not all resident, so up to 512 of them.  Without and with, per iteration of
+// whole solves: 64^3 (256 workgroups) 7.6 and 7.4 us, 72^3 (368) 9.3 and 9.5, 80^3 (504) 9.7
+// and 9.7, 84^3 (584) 11.1 and 11.8, 96^3 (864) 13.3 and 15.2.
 template <bool PRE>
 __global__ void __launch_bounds__(256) k_cg_iter(CgArgs a) {
   __shared__ double sh[4][CG_SUMS];

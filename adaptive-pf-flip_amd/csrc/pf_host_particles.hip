@@ -186,7 +186,8 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   for (int col = 0; col < 8; ++col) {
     a.list = c->color_list + (long long)col * c->color_cap;
     a.count = c->color_cnt + col;
-    const dim3 grid((unsigned)std::max<long long>(c->color_cap, 1));
+    // (the list's length is on the device: offer the split by axes where it may be short)
+    const dim3 grid((unsigned)std::max<long long>(c->color_cap, 1), c->color_cap <= 2 * kP2GSplitMost ? 3 : 1);
     const P2GShared sh = p2g_shared_args(a);
     const P2GField f0 = p2g_field_args(a, 0), f1 = p2g_field_args(a, 1), f2 = p2g_field_args(a, 2);
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(64), 0, c->stream, sh, f0, f1, f2); };

@@ -235,7 +235,9 @@ __device__ inline Row4<T> mr_apply(const MrRow& R, const Op& op, const Row4<T>& 
 // The list in slots of four blocks (one per 16 lanes), each XCD a contiguous eighth.  The
 // next slot's info bytes and the one after's list entries load while a slot is worked
 // on (list, info and values would be three waits in a row): an update 36.5 ->
-// 32.6 us on those blocks, a Jacobi iteration on 80 x 72 x 80 7.34 -> 7.23.
+// 32.6 us on those blocks.  The Jacobi iteration makes its walk before it waits for the sums,
+// so the first slot's list and info load meanwhile: 7.34 -> 7.23 us on 80 x 72 x 80, where
+// every wave has one slot.
 struct MrWalk {
   const uint32_t* list;
   const uint8_t* info;
@@ -516,8 +518,8 @@ __global__ void __launch_bounds__(256) k_mr_cycle(MrCycleArgs a) {
       uxm = a.x[R.xm];
     }
     if (MODE == MG_PSWEEP) {
-      // (a missing neighbour takes the block's own correction, times a zero coupling)
-      // (loads without a branch, in flight with the rest)
+      // (loads without a branch, in flight with the rest: a missing neighbour takes the
+      // block's own correction, times a zero coupling)
       auto corr = [&](int bx, int by, int bz) { return a.omega_c * a.xc[bm_index(a.dcc, bx, by, bz)]; };
       const int ny = R.ly == 3 ? min(R.by + 1, op.dc.nby - 1) : (R.ly == 0 ? max(R.by - 1, 0) : R.by);
       const int nz = R.lz == 3 ? min(R.bz + 1, op.dc.nbz - 1) : (R.lz == 0 ? max(R.bz - 1, 0) : R.bz);

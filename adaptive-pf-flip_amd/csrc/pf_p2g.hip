@@ -643,7 +643,7 @@ __device__ inline void p2g_block(const P2GShared& a, const P2GField& fu, const P
 // ceil(3 n / 3072) rounds a third as long plus a tenth for ranking three times.
 constexpr uint32_t kP2GResident = 256 * 12;
 constexpr uint32_t kP2GSplitMost = 5 * kP2GResident;  // (past five rounds the last one matters little)
-inline bool p2g_split(uint32_t n) {
+__host__ __device__ inline bool p2g_split(uint32_t n) {
   const uint32_t whole = (n + kP2GResident - 1) / kP2GResident, third = (3 * n + kP2GResident - 1) / kP2GResident;
   return n <= kP2GSplitMost && 11 * third < 30 * whole;
 }
@@ -654,7 +654,11 @@ inline bool p2g_split(uint32_t n) {
 // fields.  Bound by the vector ALU while the fullest cells of a wave last.  By colour ->
 // block + gather: 64^3 248 -> 98 + 13 us, 144 x 101 x 131 1075 -> 617 + 77, 128^3 x 0.6
 // 675 -> 391 + 58, 256^3 6670 -> 4757 + 595 (and a fill of six fields saved).
-constexpr long long kP2GRegionMost = 262144;  // 256^3 cells, 1.6 GB of regions
+// The line is one of memory, not of speed: the regions are 96 B a cell, kept by the context
+// (1.6 GB at the line, 256^3 cells).  Beyond it the whole splat call takes, by colour and with
+// regions, 8.1 and 6.6 ms at 272^3, 13.1 and 10.6 at 320^3, 23.4 and 20.7 at 400^3 (6.1 GB);
+// multires 7.1 and 7.1 at 384^3 effective, 14.8 and 14.6 at 512^3 (12.9 GB).
+constexpr long long kP2GRegionMost = 262144;
 template <int KT, bool F32>
 __global__ void __launch_bounds__(64) k_p2g_block(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
   const uint32_t b = blockIdx.x;
@@ -662,12 +666,15 @@ __global__ void __launch_bounds__(64) k_p2g_block(P2GShared a, P2GField fu, P2GF
   p2g_block<KT, F32, true>(a, fu, fv, fw, b, gridDim.y == 3 ? (int)blockIdx.y : -1);
 }
 
-// One launch per colour, without the regions' memory: larger grids.
+// One launch per colour, without the regions' memory: larger grids, and any grid whose
+// regions did not fit (the split is for those: a colour of a larger grid is long).
 template <int KT, bool F32>
 __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
   const uint32_t nblk = *a.count;
   if (blockIdx.x >= nblk) return;
-  p2g_block<KT, F32, false>(a, fu, fv, fw, a.list[blockIdx.x], -1);
+  const bool split = gridDim.y == 3 && p2g_split(nblk);
+  if (!split && blockIdx.y > 0) return;
+  p2g_block<KT, F32, false>(a, fu, fv, fw, a.list[blockIdx.x], split ? (int)blockIdx.y : -1);
 }
 
 // A wave per block of a face field: a node lies in the regions of at most two source
