@@ -436,15 +436,16 @@ def main():
             launches = nl // args.steps
             per_launch = (P2G_BYTES[0] * npart + P2G_BYTES[1] * fluid) / launches
             achieved = per_launch / (avg * 1e-3) / 1e9
-            tf = os.path.join(ROOT, "profiles", "p2g_color_rt256_traffic.md")
+            tf = os.path.join(ROOT, "profiles", "p2g_rt256_traffic.md")
             roofline = {"bound": "hbm", "kernel": "k_p2g_color<0, true>" if launches == 8 else "k_p2g_block<0, true> + k_p2g_gather", "achieved": round(achieved, 1),
                         "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                         "traffic": read_traffic(tf) if (os.path.exists(tf) and n == 256) else None,
                         "bytes_per_launch": int(per_launch), "avg_launch_ms": round(avg, 5),
                         "launches_timed": nl, "dominant_kernel_in_step_table": dominant,
                         "note": f"bytes = (25 B/particle + 24 B/fluid cell) / {launches} launches; the kernel is "
-                                "VALU-bound: valu_busy and waves_per_simd are the SQ counters of the committed "
-                                "256^3 counter summary"}
+                                "VALU-bound: valu_busy (the share of quad-cycles in which a SIMD issues a VALU "
+                                "instruction) and waves_per_simd are from the SQ counters of the committed 256^3 "
+                                "counter summary"}
             if os.path.exists(tf) and n == 256:
                 roofline["valu_busy"] = read_table_value(tf, "VALU busy")
                 roofline["waves_per_simd"] = read_table_value(tf, "resident waves per SIMD")
