@@ -668,6 +668,16 @@ int cg_run(pf_ctx* c, CgState& g, const VecArgs& va, int check, const Look& look
   }
 }
 
+// Workgroups of the pin scan: each ends in atomics on the same three words (about 12 ns
+// each), and walks its blocks one wait after another, so neither many nor few: 64 blocks
+// each, 512 to 2048 of them.  With 512, 1024 and 2048 the scan takes 17, 27 and 27 us at
+// 64^3, 39, 39 and 57 at 128^3, 118, 80 and 80 at 192^3, 278, 180 and 126 at 256^3, the
+// multires one 2.04, 1.30 and 0.86 ms at 512^3 effective.  (A look at the word before the atomic
+// is a read of what other XCDs change: 170 us instead of 126.)
+unsigned pin_grid(long long npb) {
+  return std::min<unsigned>(list_grid(npb), (unsigned)std::clamp<long long>(npb / 64, 512, 2048) & ~7u);
+}
+
 // single: the single-phase unit-density projection (ph unused, cdiv ignored);
 // c->mr: the multires finite-volume projection, stopping when
 // |rhs - A x|_inf < max(cfg->tol, mr_rel_tol * |rhs|_inf)
@@ -811,7 +821,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
       ma.pin_cell = c->mr_pin_dev;
     }
     HIP_TRY(c, fill_u32(c->stream, c->u32_dev + 5, 0u, 1));
-    hipLaunchKernelGGL(k_mr_pin, dim3(std::min(G, 512u)), dim3(256), 0, c->stream, ma);
+    hipLaunchKernelGGL(k_mr_pin, dim3(pin_grid(npb)), dim3(256), 0, c->stream, ma);
     LAUNCH_CHECK(c);
     if (refmode) {
       TIMED(c, PF_K_ASSEMBLE, hipLaunchKernelGGL(k_mr_assemble, dim3(G), dim3(256), 0, c->stream, ma));
@@ -827,7 +837,7 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     }
     LAUNCH_CHECK(c);
   } else {
-  hipLaunchKernelGGL(k_pin_detect, dim3(std::min(list_grid(npb), 512u)), dim3(256), 0, c->stream, pa);
+  hipLaunchKernelGGL(k_pin_detect, dim3(pin_grid(npb)), dim3(256), 0, c->stream, pa);
   LAUNCH_CHECK(c);
   AsmOut ao;
   ao.b64 = c->b64; ao.cd64 = c->cd64; ao.cx64 = c->cx64; ao.cy64 = c->cy64; ao.cz64 = c->cz64;

@@ -237,12 +237,9 @@ __global__ void __launch_bounds__(256) k_mr_pin(MrAsm a) {
   if (lane == 0) { s_air[w] = anyair; s_min[w] = mn; s_cnt[w] = cnt; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    // (the flag and the minimum settle early: look before the atomic)
-    if ((s_air[0] | s_air[1] | s_air[2] | s_air[3]) &&
-        !__hip_atomic_load(&a.pin[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-      atomicOr(&a.pin[0], 1u);
+    if (s_air[0] | s_air[1] | s_air[2] | s_air[3]) atomicOr(&a.pin[0], 1u);
     const uint32_t m4 = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
-    if (m4 < __hip_atomic_load(&a.pin[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&a.pin[1], m4);
+    if (m4 != 0xffffffffu) atomicMin(&a.pin[1], m4);
     const uint32_t c4 = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
     if (c4) atomicAdd(&a.pin[4], c4);
   }

@@ -294,9 +294,8 @@ __global__ void __launch_bounds__(256) k_pin_detect(ProjArgs a) {
     const uint32_t air = s_air[0] | s_air[1] | s_air[2] | s_air[3];
     const uint32_t mn = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
     const uint32_t cnt = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-    // (the flag and the minimum settle early: look before the atomic)
-    if (air && !__hip_atomic_load(&a.pin[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicOr(&a.pin[0], 1u);
-    if (mn < __hip_atomic_load(&a.pin[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&a.pin[1], mn);
+    if (air) atomicOr(&a.pin[0], 1u);
+    if (mn != 0xffffffffu) atomicMin(&a.pin[1], mn);
     if (cnt) atomicAdd(&a.pin[4], cnt);
   }
 }
