@@ -132,8 +132,8 @@ __device__ inline void block_flush_counters(int (&cnt)[8], float speed, int32_t*
 
 // grid-stride over particles (fixed grid), counters flushed once per workgroup.  The
 // grid's fields packed as Q: quads (the G2P), pairs of the velocity (advection alone), or
-// the plain velocity (advection of fewer particles than cells, where packing the grid
-// costs more than it saves: 14 ps a cell against 13 a particle).
+// the plain velocity (advection of few particles, where packing the grid costs more than it
+// saves).
 template <typename Q>
 __global__ void __launch_bounds__(256) k_g2p_advect(G2PArgs a) {
   constexpr bool QUAD = std::is_same<Q, float4>::value;

@@ -204,6 +204,16 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   return PF_OK;
 }
 
+// Whether an advection without G2P packs the grid's velocity into pairs first.  The packing
+// costs three launches (6 us) and 5.7 ps a cell and saves 9 ps a particle in second order, 13 in
+// third.  Plain gathers against pairs, in us (second order; third): 32^3 cells x 8 particles 34
+// and 39 (37.6; 42), 48^3 x 8 52 and 53 (63; 59), 64^3 x 2 42 and 46 (49; 50), 64^3 x 8 83 and 76
+// (105; 91), 96^3 x 1 53 and 61 (65; 66.5), 96^3 x 2 80 and 75 (101; 86), 128^3 x 1 86 and 86 (109;
+// 96), 128^3 x 4 250 and 188 (355; 248).
+bool advect_in_pairs(long long np, long long cells, int order) {
+  return np >= std::max(cells, order == 3 ? 600000 + cells / 5 * 2 : 700000 + cells / 3 * 2);
+}
+
 // Room for the velocity pairs of an advection without G2P: the G2P's quads where it has
 // allocated them, else arrays of their own (8 B a face).  False without the memory: the plain
 // gathers then, the same bits.
@@ -241,7 +251,7 @@ int run_g2p_advect(pf_ctx* c, bool g2p, bool adv, double aL, double aG, double d
   a.vmax_bits = reinterpret_cast<uint32_t*>(c->vmax_dev);
   const Dims* fd[3] = {&c->du, &c->dv, &c->dw};
   float2* pair[3] = {nullptr, nullptr, nullptr};
-  const bool pairs = !g2p && c->np >= (long long)g.nx * g.ny * g.nz && g2p_pairs(c, fd, pair);
+  const bool pairs = !g2p && advect_in_pairs(c->np, (long long)g.nx * g.ny * g.nz, order) && g2p_pairs(c, fd, pair);
   if (g2p && !c->g2p_quad[2])
     for (auto& q : c->g2p_pair) dfree(q);  // (the quads hold pairs too)
   for (int ax = 0; ax < 3; ++ax) {
