@@ -998,7 +998,13 @@ int run_project(pf_ctx* c, const pf_phase* ph, double dt, const pf_solve_cfg* cf
     // the buffer-addressed kernels take 32-bit byte offsets: arrays below 2 GiB
     const bool spmv_buffers = c->dc.nblocks * kBlockVol * 4 < (1LL << 31);
     CgState cg;
-    bool one_kernel = mr || spmv_buffers;         // the Jacobi iteration as k_cg_iter or k_mr_cg_iter
+    // The Jacobi iteration as k_cg_iter or k_mr_cg_iter.  k_cg_iter moves 52 B a cell where the
+    // separate kernels move 64, but between about 5 and 15 million cells those find part of
+    // theirs in the last-level cache.  Separate against one kernel, us an iteration: 160^3 53.8
+    // and 48.7, 176^3 67.5 and 69.3, 192^3 96 and 100, 208^3 122 and 130, 240^3 203 and 206, 256^3
+    // 250 and 245, 288^3 350 and 342.
+    const bool cached = npb > 80000 && npb < 240000;
+    bool one_kernel = mr || (spmv_buffers && !cached);
     const unsigned GL = mr ? cg_grid(npb) : G;    // workgroups of the load, one partial each
     // r32 from the FP64 residual, x32 = 0 (and p = 0)
     auto load = [&](const double* src, float* p) {

@@ -365,7 +365,7 @@ int pf_write_render_manifest(const char* path, const char* sim_kind, int32_t nx,
  * steps with steady_clock, apps/bench_large_scale3d_tp.cpp:559-563) */
 enum pf_kernel {
   PF_K_BIN_COUNT = 0, PF_K_BIN_SCATTER, PF_K_P2G, PF_K_FACE_OPS, PF_K_ASSEMBLE,
-  PF_K_PCG_SPMV,       /* the SpMV; on the sparse path with Jacobi the whole iteration */
+  PF_K_PCG_SPMV,       /* the SpMV; with Jacobi the whole iteration where it is one kernel */
   PF_K_PCG_UPDATE, PF_K_RESIDUAL64, PF_K_VELOCITY, PF_K_G2P_ADVECT,
   PF_K_LPC_APPLY,      /* one application of the learned preconditioner (5 kernels) */
   PF_K_INTERFACE,      /* interface fields and diagnostics (5 kernels) */

@@ -87,6 +87,24 @@ def test_matches_multigrid_on_larger_grids(shape, groups):
         assert np.abs(a - b).max() < bound
 
 
+def test_separate_kernels_match_multigrid():
+    """85,184 listed blocks: the range in which the iteration takes the separate kernels"""
+    n = 176
+    gph = G.Phase(10.0, 1.0, 1.0, 1.0)  # (from rest: a lower pressure leaves a lower bound)
+    gph.rho_tilde_0 = G.calibrate_rho_tilde0(gph, 1.0)
+    ctx = G.Context(n, n, n, 1.0 / n)
+    ctx.scene(G.SCENE_RT, 3)
+    faces = []
+    for pre in (G.PRECOND_JACOBI, G.PRECOND_MULTIGRID):
+        _grid_half(ctx, gph)
+        st = ctx.project(gph, 1e-3, G.default_solve_cfg(G.STOP_REL2, 1e-11, 20000, pre))
+        assert st.converged == 1 and st.true_rel_residual <= 1e-11 and st.fallback_used == 0
+        faces.append([ctx.field(f) for f in range(3)])
+    bound = 4 * (1e-3 * n) / gph.rho_g * 2.0 ** -24 * np.abs(ctx.field(G.FIELD_P)).max()
+    for a, b in zip(*faces):
+        assert np.abs(a).max() > 100 * bound and np.abs(a - b).max() < bound
+
+
 @pytest.mark.parametrize("budget", [1, 2, 60])
 def test_stops_at_the_iteration_budget(budget):
     _, ctx, _, _, gph = _context((32, 20, 32), O.SCENE_RT)
