@@ -125,7 +125,7 @@ int run_p2g_splat(pf_ctx* c, const pf_phase* ph, double Vp, bool single = false,
   const long long nb = c->dc.nblocks;
   if (nb <= kP2GRegionMost && c->np > 0 && !c->p2g_regions && !c->p2g_no_regions) {
     // (without the memory for them: by colours)
-    if (hipMalloc((void**)&c->p2g_regions, sizeof(float2) * 3 * 256 * (size_t)nb) != hipSuccess) {
+    if (hipMalloc((void**)&c->p2g_regions, (sizeof(float2) * 3 * 256 + 1) * (size_t)nb) != hipSuccess) {
       (void)hipGetLastError();
       c->p2g_regions = nullptr;
       c->p2g_no_regions = true;

@@ -73,6 +73,7 @@ struct P2GShared {
   float mp_l, mp_g;
   bool has_vol, pow2, fast32;
   float2* regions;  // the gathered form: [block][axis][256] (momentum, mass) node sums
+  uint8_t* held;    // ... and which blocks hold particles
 };
 
 struct P2GField {
@@ -101,6 +102,7 @@ inline P2GShared p2g_shared_args(const P2GArgs& a) {
   r.mp_l = a.mp_l; r.mp_g = a.mp_g;
   r.has_vol = a.has_vol; r.pow2 = a.pow2; r.fast32 = a.fast32;
   r.regions = a.regions;
+  r.held = reinterpret_cast<uint8_t*>(a.regions + 3 * 256 * a.dc.nblocks);
   return r;
 }
 
@@ -653,7 +655,9 @@ __host__ __device__ inline bool p2g_split(uint32_t n) {
 // partly idle at the end of each of the eight, wait for their atomics and need cleared
 // fields.  Bound by the vector ALU while the fullest cells of a wave last.  By colour ->
 // block + gather: 64^3 248 -> 98 + 13 us, 144 x 101 x 131 1075 -> 617 + 77, 128^3 x 0.6
-// 675 -> 391 + 58, 256^3 6670 -> 4757 + 595 (and a fill of six fields saved).
+// 675 -> 391 + 58, 256^3 6670 -> 4520 + 551 (and a fill of six fields saved).  A grid of that
+// size with next to nothing in it is the exception: 262,144 workgroups that return at
+// once take 200 us (20,000 particles spread over it, the whole call: 456 by colour, 516).
 // The line is one of memory, not of speed: the regions are 96 B a cell, kept by the context
 // (1.6 GB at the line, 256^3 cells).  Beyond it the whole splat call takes, by colour and with
 // regions, 8.1 and 6.6 ms at 272^3, 13.1 and 10.6 at 320^3, 23.4 and 20.7 at 400^3 (6.1 GB);
@@ -662,7 +666,9 @@ constexpr long long kP2GRegionMost = 262144;
 template <int KT, bool F32>
 __global__ void __launch_bounds__(64) k_p2g_block(P2GShared a, P2GField fu, P2GField fv, P2GField fw) {
   const uint32_t b = blockIdx.x;
-  if (a.start[(long long)b * kBlockVol] == a.start[((long long)b + 1) * kBlockVol]) return;
+  const bool held = a.start[(long long)b * kBlockVol] != a.start[((long long)b + 1) * kBlockVol];
+  if (threadIdx.x == 0 && blockIdx.y == 0) a.held[b] = held;
+  if (!held) return;
   p2g_block<KT, F32, true>(a, fu, fv, fw, b, gridDim.y == 3 ? (int)blockIdx.y : -1);
 }
 
@@ -680,7 +686,9 @@ __global__ void __launch_bounds__(64) k_p2g_color(P2GShared a, P2GField fu, P2GF
 // A wave per block of a face field: a node lies in the regions of at most two source
 // blocks per direction, of opposite parity, so of at most one block per colour; their
 // sums are added in colour order, as the launches by colour do.  Writes every node and
-// the block's activation, so the fields need no clearing.
+// the block's activation, so the fields need no clearing.  Which blocks hold particles it reads
+// from a byte a block: from two cell starts it took 345 us for a nearly empty 256^3 grid
+// with the block launch, 290 with the bytes.
 template <int AX>
 __device__ inline void p2g_gather_axis(const P2GShared& a, const P2GField& f, long long fb, int lane) {
   using A = Ax<AX>;
@@ -691,7 +699,7 @@ __device__ inline void p2g_gather_axis(const P2GShared& a, const P2GField& f, lo
     const int sx = Bx + lane % 3 - 1, sy = By + (lane / 3) % 3 - 1, sz = Bz + lane / 9 - 1;
     if (sx >= 0 && sy >= 0 && sz >= 0 && sx < a.dc.nbx && sy < a.dc.nby && sz < a.dc.nbz) {
       const long long b = sx + a.dc.nbx * (sy + (long long)a.dc.nby * sz);
-      occ = a.start[b * kBlockVol] != a.start[(b + 1) * kBlockVol];
+      occ = a.held[b];
     }
   }
   const uint32_t near = (uint32_t)__ballot(occ);  // the 27 blocks around that hold particles
